@@ -138,6 +138,12 @@ struct MatTile {
   int seg;                 // segment index (sets the march direction)
 };
 
+// A block of a tile that holds an interface: columns [x0, x1) (at most 56), rows
+// [j0, j1) (at most kMixRows).
+struct MixBlock {
+  int x0, x1, j0, j1;
+};
+
 struct MatPlane {
   bool active = false;
   int count = 0;
@@ -152,7 +158,8 @@ struct MatPlane {
   int built_fb = -1, built_seg = -1, built_edge = -1;
   // tables of the two-step pass (strips of the two-step window less 8 columns)
   MatTile *d_homog2 = nullptr, *d_mixed2 = nullptr;
-  int n_homog2 = 0, n_mixed2 = 0;
+  MixBlock *d_blocks2 = nullptr;  // the interface tiles as blocks, or none
+  int n_homog2 = 0, n_mixed2 = 0, n_blocks2 = 0;
   int built_pair_seg = -1, built_pair_fb = -1;
   // the interface tiles run on a second stream beside the single-material
   // ones (forked from and joined back into the grid's stream)

@@ -95,6 +95,19 @@ __global__ __launch_bounds__(FB, FB == 256 ? 2 : 3) void k_step2_mat_mixed(
                           cyt, sn);
 }
 
+// The interface tiles as blocks of rows that run side by side (block_pair_mixed),
+// where they are few.
+template <typename T>
+__global__ __launch_bounds__((kMixRows + 8) * 64) void k_step2_mat_block(
+    const T *__restrict__ src, T *__restrict__ dst, int nx, int ny, long pitch, long plane,
+    const MixBlock *__restrict__ blocks, const unsigned char *__restrict__ ids, long idp,
+    const SweepCoef<T> *__restrict__ cxt, const SweepCoef<T> *__restrict__ cyt) {
+  __shared__ Node<T> sn[(kMixRows + 8) * 64];
+  const MixBlock b = blocks[blockIdx.x];
+  block_pair_mixed<T>(src, dst, ids, idp, nx, ny, pitch, plane, b.x0, b.x1, b.j0, b.j1, cxt, cyt,
+                      sn);
+}
+
 // Energy density in FP64 (plane strain, isotropic):
 //   rho/2 |v|^2 + (sxx+syy)^2 / (8 (lambda+mu)) + ((sxx-syy)^2/2 + 2 sxy^2) / (4 mu)
 // summed over the grid; one FP64 partial per workgroup, summed on the host in
@@ -309,13 +322,15 @@ void mat_release(MatPlane *m) {
   m->aux = nullptr;
   m->ev_fork = m->ev_join = nullptr;
   for (void *p : {(void *)m->d_ids, m->d_cx, m->d_cy, (void *)m->d_homog, (void *)m->d_mixed,
-                  (void *)m->d_homog2, (void *)m->d_mixed2, (void *)m->d_etab})
+                  (void *)m->d_homog2, (void *)m->d_mixed2, (void *)m->d_blocks2,
+                  (void *)m->d_etab})
     dev_free(p);
   m->d_ids = nullptr;
   m->d_cx = m->d_cy = nullptr;
   m->d_homog = m->d_mixed = m->d_homog2 = m->d_mixed2 = nullptr;
+  m->d_blocks2 = nullptr;
   m->d_etab = nullptr;
-  m->n_homog = m->n_mixed = m->n_homog2 = m->n_mixed2 = 0;
+  m->n_homog = m->n_mixed = m->n_homog2 = m->n_mixed2 = m->n_blocks2 = 0;
   m->built_fb = m->built_seg = m->built_edge = m->built_pair_seg = m->built_pair_fb = -1;
 }
 
@@ -422,15 +437,49 @@ static void split_tiles(const MatPlane *m, int nx, int ny, int width, int ch, in
   }
 }
 
-static int upload_tiles(const std::vector<MatTile> &v, MatTile **d, int *n) {
+// Split the mixed tiles of the two-step pass (strips of `width` columns) into
+// bands of kMixRows rows: runs of bands whose read window holds one material
+// go back to the single-material tiles, the others become blocks of at most 56
+// columns.
+static void split_bands(const MatPlane *m, int nx, int ny, int width,
+                        const std::vector<MatTile> &mixed, std::vector<MatTile> *homog,
+                        std::vector<MixBlock> *blocks) {
+  const int parts = (width + 55) / 56, pw = (width + parts - 1) / parts;
+  for (const MatTile &t : mixed) {
+    const int x0 = t.strip * width, x1 = std::min(x0 + width, nx);
+    const int xa = std::max(x0 - 4, 0), xb = std::min(x1 + 3, nx - 1);
+    MatTile run{t.strip, t.j0, t.j0, -1, t.seg};
+    for (int a = t.j0; a < t.j1; a += kMixRows) {
+      const int b = std::min(a + kMixRows, t.j1);
+      const int ra = std::max(a - 4, 0), rb = std::min(b + 3, ny - 1);
+      const unsigned char first = m->ids[(long)ra * nx + xa];
+      bool one = true;
+      for (int j = ra; j <= rb && one; ++j) {
+        const unsigned char *r = m->ids.data() + (long)j * nx;
+        one = std::all_of(r + xa, r + xb + 1, [first](unsigned char id) { return id == first; });
+      }
+      const int mat = one ? (int)first : -1;
+      if (run.mat >= 0 && mat != run.mat) homog->push_back(run);
+      if (mat != run.mat) run.j0 = a;
+      run.j1 = b;
+      run.mat = mat;
+      for (int x = x0; x < x1 && !one; x += pw)
+        blocks->push_back({x, std::min(x + pw, x1), a, b});
+    }
+    if (run.mat >= 0) homog->push_back(run);
+  }
+}
+
+template <typename V>
+static int upload_tiles(const std::vector<V> &v, V **d, int *n) {
   dev_free(*d);
   *d = nullptr;
   *n = 0;
   if (v.empty()) return OK;
-  int rc = dev_alloc((void **)d, v.size() * sizeof(MatTile), "materials: tiles");
+  int rc = dev_alloc((void **)d, v.size() * sizeof(V), "materials: tiles");
   if (rc) return rc;
-  rc = mcheck(hipMemcpy(*d, v.data(), v.size() * sizeof(MatTile), hipMemcpyHostToDevice),
-                  "materials: tiles");
+  rc = mcheck(hipMemcpy(*d, v.data(), v.size() * sizeof(V), hipMemcpyHostToDevice),
+              "materials: tiles");
   if (rc) return rc;
   *n = (int)v.size();
   return OK;
@@ -452,8 +501,7 @@ static int mat_tiles(DevGrid *g, MatPlane *m, int edge) {
   return OK;
 }
 
-// The interface tiles are few and march slowly (both faces of every node),
-// so run after the single-material tiles they would leave the device mostly
+// Marched interface tiles are slow (both faces of every node), so run after the single-material tiles they would leave the device mostly
 // idle: 0.44 ms of a 6.5 ms two-step pass on 16384^2.  They are launched
 // first, on a second stream forked from the grid's stream, and joined back
 // before the next launch on it.  Both launches read the same input and write
@@ -483,6 +531,21 @@ static int pair_lanes(const DevGrid *g) {
   return fb == 64 || fb == 128 ? fb : 256;
 }
 
+// Whether the interface tiles run as `blocks` blocks rather than as `mixed`
+// marched tiles of `lanes` lanes and `rows` rows.  Measured (FP64 / FP32): a
+// round of blocks, one / two per CU, takes 11 / 7 us; a marched row 5 / 3 us while
+// its wavefronts fit in a round of three per SIMD, and the second stream that
+// hides the march behind the single-material tiles 15 us.  Two layers and an inclusion
+// on 4100 x 3000: 382 us a pass with blocks against 478 (FP64), 186 against 194
+// (FP32), on 1500 x 1000 76 against 114 and 31 against 65; a checkerboard of
+// interface tiles only, 3000 x 2000: 439 us marched against 546 in blocks.
+static bool blocks_pay(int elem, size_t mixed, int lanes, int rows, size_t blocks) {
+  const size_t waves = mixed * (lanes / 64), round = elem == 8 ? 256 : 512;
+  const double block_us = elem == 8 ? 11 : 7, row_us = elem == 8 ? 5 : 3;
+  return (double)((blocks + round - 1) / round) * block_us <
+         (double)((waves + 3071) / 3072) * (rows + 8) * row_us + 15;
+}
+
 // Tables of the two-step pass: strips of (window - 8) columns read 4 halo
 // columns and 4 halo rows on each side.
 static int mat_tiles2(DevGrid *g, MatPlane *m) {
@@ -490,8 +553,18 @@ static int mat_tiles2(DevGrid *g, MatPlane *m) {
   if (m->built_pair_seg == seg && m->built_pair_fb == fb) return OK;
   std::vector<MatTile> homog, mixed;
   split_tiles(m, g->nx, g->ny, fb - 8, 4, seg, 4, EDGE_CLAMP, &homog, &mixed);
+  std::vector<MatTile> homogb = homog;
+  std::vector<MixBlock> blocks;
+  split_bands(m, g->nx, g->ny, fb - 8, mixed, &homogb, &blocks);
+  if (blocks_pay(g->elem, mixed.size(), fb, std::min(seg, g->ny), blocks.size())) {
+    homog.swap(homogb);
+    mixed.clear();
+  } else {
+    blocks.clear();
+  }
   int rc = upload_tiles(homog, &m->d_homog2, &m->n_homog2);
   if (!rc) rc = upload_tiles(mixed, &m->d_mixed2, &m->n_mixed2);
+  if (!rc) rc = upload_tiles(blocks, &m->d_blocks2, &m->n_blocks2);
   if (rc) return rc;
   m->built_pair_seg = seg;
   m->built_pair_fb = fb;
@@ -511,6 +584,13 @@ static int launch_mat2(DevGrid *g, MatPlane *m) {
                        dst, g->nx, g->ny, g->pitch, g->plane, m->d_mixed2, m->d_ids, m->idp, cx,
                        cy);
   }
+  // blocks are few and short: on the grid's own stream, which costs less than
+  // forking a second one (250 x 300 FP64 26 us a pass against 40, 4100 x 3000
+  // 382 against 389)
+  if (m->n_blocks2)
+    hipLaunchKernelGGL((k_step2_mat_block<T>), dim3(m->n_blocks2), dim3((kMixRows + 8) * 64), 0,
+                       g->stream, src, dst, g->nx, g->ny, g->pitch, g->plane, m->d_blocks2,
+                       m->d_ids, m->idp, cx, cy);
   if (m->n_homog2 && FB == 64 && g->tiles.pair_split)
     hipLaunchKernelGGL((k_step2_mat_homog_split<T>), dim3(m->n_homog2), dim3(128), 0, g->stream,
                        src, dst, g->nx, g->ny, g->pitch, g->plane, m->d_homog2, cx, cy);

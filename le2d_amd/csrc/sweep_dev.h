@@ -1048,4 +1048,69 @@ __device__ __forceinline__ void march_pair_mixed(const T *__restrict__ src, T *_
   }
 }
 
+// The same two steps for a block of kMixRows output rows and up to 56 columns,
+// every row of it and its halo on a wavefront of its own: lane t of wavefront
+// v holds node (x0-4+t, j0-4+v).  What bounds a mixed tile is latency (each
+// row of the march waits for its ids, then for its nodes' constants, then for
+// two exchanges), and a pass waits for its mixed tiles: here the rows' waits
+// overlap, four sweeps one after another instead of (rows + 8) x 4.  It computes
+// 16 rows for 8, so the march stays where mixed tiles fill the device.  The
+// operations are march_pair_mixed's.  sn holds 16 x 64 nodes.
+constexpr int kMixRows = 8;
+
+template <typename T>
+__device__ __forceinline__ void block_pair_mixed(const T *__restrict__ src, T *__restrict__ dst,
+                                                 const unsigned char *__restrict__ ids, long idp,
+                                                 int nx, int ny, long pitch, long plane, int x0,
+                                                 int x1, int j0, int j1,
+                                                 const SweepCoef<T> *__restrict__ cxt,
+                                                 const SweepCoef<T> *__restrict__ cyt,
+                                                 Node<T> *sn) {
+  constexpr int ROWS = kMixRows + 8;
+  const int v = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int t = (int)(threadIdx.x & 63);
+  const int x = x0 - 4 + t, xc = min(max(x, 0), nx - 1);
+  const int j = j0 - 4 + v, jc = min(max(j, 0), ny - 1);
+  const int tlo = max(0, 4 - x0), thi = min(63, nx + 3 - x0);
+  Node<T> u = load_row_node(src + (long)jc * pitch, plane, (unsigned)xc * (unsigned)sizeof(T));
+  const int m = ids[(long)jc * idp + xc];
+#pragma unroll 1
+  for (int s = 0; s < 2; ++s) {
+    {
+      const SweepCoef<T> c = cxt[m];
+      sn[v * 64 + t] = u;
+      window_sync<64>();
+      W4<T> w[5];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        const Node<T> &n = sn[v * 64 + min(max(t - 2 + k, tlo), thi)];
+        w[k] = invariants(n.vx, n.sxx, n.vy, n.sxy, c);
+      }
+      window_sync<64>();
+      const W4<T> fl = faces(w[0], w[1], w[2], w[3], c);
+      const W4<T> fr = faces(w[1], w[2], w[3], w[4], c);
+      apply(u.vx, u.vy, u.sxx, u.syy, u.sxy, w[2], fl, fr, c);
+    }
+    sn[v * 64 + t] = u;
+    __syncthreads();
+    {
+      const SweepCoef<T> c = cyt[m];
+      W4<T> w[5];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        // row j-2+k clamped to the grid, then to the block (rows whose
+        // stencil leaves the block are not outputs' inputs)
+        const int r = min(max(min(max(j - 2 + k, 0), ny - 1) - (j0 - 4), 0), ROWS - 1);
+        w[k] = inv_y(sn[r * 64 + t], c);
+      }
+      if (s == 0) __syncthreads();  // the second step rewrites the rows
+      const W4<T> fl = faces(w[0], w[1], w[2], w[3], c);
+      const W4<T> fr = faces(w[1], w[2], w[3], w[4], c);
+      apply(u.vy, u.vx, u.syy, u.sxx, u.sxy, w[2], fl, fr, c);
+    }
+  }
+  if (v >= 4 && j < j1 && t >= 4 && t < 60 && x < x1)
+    store_row_node(dst + (long)j * pitch, plane, (unsigned)max(x, 0) * (unsigned)sizeof(T), u);
+}
+
 }  // namespace le2d
