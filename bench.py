@@ -205,7 +205,7 @@ def measured_counters(n, dtype, kernel):
 def roofline(n, es, ms_pair, ms_step, ms_x, ms_y, dtype_name, split=0):
     """Roofline of the launch that carries le_step_n: the two-step kernel
     (two node-updates per node per launch; k_step2_split when the tuner
-    chose 64-lane windows on two wavefronts) when it is on, else the
+    chose 64-column windows) when it is on, else the
     single-step kernel."""
     nodes = n * n
     pair_kernel = "k_step2_split" if split else "k_step2_xy"
@@ -776,7 +776,8 @@ def main():
                                                      args.warmup, args.profile_steps)
     el = els[0]
     value = n * n * args.steps / el / 1e9
-    roof = roofline(n, es, ms_pair, ms_step, ms_x, ms_y, args.dtype, t.get_step_pair_split())
+    roof = roofline(n, es, ms_pair, ms_step, ms_x, ms_y, args.dtype,
+                    t.get_step_pair_window() == 64)
     tiles = t.get_tiles() + (t.get_step_pairs(), t.get_step_pair_window(),
                              t.get_step_pair_split())
     other = None
@@ -792,7 +793,7 @@ def main():
         other = {"dtype": o_name, "value": round(n * n * args.steps / el2 / 1e9, 3),
                  "ms_per_step": round(el2 / args.steps * 1e3, 4),
                  "roofline": roofline(n, np.dtype(o_dt).itemsize, mp2, ms2, mx2, my2, o_name,
-                                      t2.get_step_pair_split()),
+                                      t2.get_step_pair_window() == 64),
                  "tiles": {"pair_seg": t2.get_step_pairs(),
                            "pair_lanes": t2.get_step_pair_window(),
                            "pair_split": t2.get_step_pair_split()},

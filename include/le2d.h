@@ -93,28 +93,25 @@ int le2d_get_tiles(le_task *task, int *x_rows, int *y_seg, int *y_block, int *xy
  * one step per pass.  le_step always takes one step. */
 int le2d_set_step_pairs(le_task *task, int seg);
 int le2d_get_step_pairs(le_task *task, int *seg);
-/* Lanes per two-step workgroup, 64, 128 or 256 (it writes that many columns
- * less eight).  The default is 64 lanes (one wavefront), or 256 for FP32 grids
- * of about 8192^2 and more. */
+/* Window of the two-step pass: 64, 128 or 256 columns, of which a workgroup
+ * writes all but eight (FP64: 256 runs as 128).  The default follows the
+ * grid: wide windows where it fills the device with them. */
 int le2d_set_step_pair_window(le_task *task, int lanes);
 int le2d_get_step_pair_window(le_task *task, int *lanes);
-/* With 64-lane windows: on = 1 runs the two stages of a pass on two
- * wavefronts of a 128-lane workgroup (each holds one stage's state, so more
- * are resident), 0 on one wavefront.  Bit-identical either way; the tuner
- * chooses between them with the window width. */
+/* Kept for callers: the setting is stored and reported, and every window now
+ * runs the two stages of a pass on two wavefronts. */
 int le2d_set_step_pair_split(le_task *task, int on);
 int le2d_get_step_pair_split(le_task *task, int *on);
-/* Time the two-step pass at segment heights 16 .. 160 (4 .. 160 on grids too
- * small to fill the device with 16-row segments) and windows of 64 (one or
- * two wavefronts, le2d_set_step_pair_split), 128 and 256 lanes on the task's
- * grid and keep the fastest.  The state does not
+/* Time the two-step pass at segment heights 16 .. 160 and those that fill
+ * whole rounds of workgroups (4 .. 160 on grids too small to fill the device
+ * with 16-row segments) and windows of 64, 128 and (FP32) 256 columns on the
+ * task's grid and keep the fastest.  The state does not
  * advance: each candidate reads the current state and writes the idle
  * buffer.  le_step_n does this once per
  * grid shape and process on its first call of 8 or more steps, unless the
  * caller has set a height (le2d_set_step_pairs), a material plane is set or
  * the environment has LE2D_TUNE=0.  A task with a material plane keeps the
- * default window and height; with 64-lane windows its first such call times
- * the one- and two-wavefront forms instead and keeps the faster. */
+ * default window and height. */
 int le2d_tune_step_pairs(le_task *task, int *seg);
 /* Run `passes` two-step passes, timing each launch with HIP events; mean ms
  * of one pass (two steps).  Needs seg > 0 and an ST_AOS task. */
@@ -224,8 +221,8 @@ int le2d_batch_wait(le2d_batch *b);
  * LE2D_BATCH_TILES, one workgroup per tile; LE2D_BATCH_PERSISTENT, resident
  * workgroups walk the tile table; LE2D_BATCH_PAIRS, one workgroup per tile
  * and two steps per launch (an odd step count ends with one single-step
- * launch); LE2D_BATCH_PAIRS_SPLIT, the same with 64-lane windows whose two
- * stages run on two wavefronts.  All forms give the same results. */
+ * launch); LE2D_BATCH_PAIRS_SPLIT, the same with windows of 64 columns.  All forms
+ * give the same results. */
 #define LE2D_BATCH_TILES 0
 #define LE2D_BATCH_PERSISTENT 1
 #define LE2D_BATCH_PAIRS 2
@@ -283,11 +280,10 @@ int le2d_server_set_shape(le2d_server *srv, int fb, int seg, int max_chunk);
  * picks the height for its live set, shorter when few requests are live);
  * 0: one step per launch.  Results do not change. */
 int le2d_server_set_pairs(le2d_server *srv, int pair_seg);
-/* Lanes per two-step workgroup, 64, 128 or 256; 0 (the default): 256 for
- * FP32 requests and 64 for FP64.  Results do not change. */
+/* Window of the two-step launches, 64, 128 or 256 columns; 0 (the default): by
+ * the live set.  Results do not change. */
 int le2d_server_set_pair_window(le2d_server *srv, int lanes);
-/* With 64-lane two-step windows, on = 1 runs each pass's two stages on two
- * wavefronts (default 0).  Results do not change. */
+/* Kept for callers (see le2d_set_step_pair_split); nothing depends on it. */
 int le2d_server_set_pair_split(le2d_server *srv, int on);
 /* Admission.  max_queue: requests that may wait (0, the default: no limit);
  * at the limit le2d_server_submit returns -LE2D_ERR_BUSY and the caller

@@ -317,7 +317,7 @@ class Task:
         self._check(self.lib.le2d_set_step_pairs(self.ref, seg), "set_step_pairs")
 
     def set_step_pair_window(self, lanes):
-        """Lanes per two-step workgroup: 64, 128 or 256 (writes lanes - 8 columns)."""
+        """Window of the two-step pass: 64, 128 or 256 columns (FP64: 256 runs as 128)."""
         self._check(self.lib.le2d_set_step_pair_window(self.ref, lanes), "set_step_pair_window")
 
     def get_step_pair_window(self):
@@ -327,7 +327,7 @@ class Task:
         return v.value
 
     def set_step_pair_split(self, on):
-        """64-lane windows: the two stages on two wavefronts (1) or one (0)."""
+        """Stored and reported; every window runs its stages on two wavefronts."""
         self._check(self.lib.le2d_set_step_pair_split(self.ref, int(on)), "set_step_pair_split")
 
     def get_step_pair_split(self):
@@ -337,7 +337,7 @@ class Task:
         return v.value
 
     def tune_step_pairs(self):
-        """Time the two-step pass at several segment heights and both window
+        """Time the two-step pass at several segment heights and window
         widths and keep the fastest (the state does not advance); returns the
         height (get_step_pair_window gives the width)."""
         v = ctypes.c_int()
@@ -541,12 +541,12 @@ class Server:
         self._check(self.lib.le2d_server_set_pairs(self.h, pair_seg), "set_pairs")
 
     def set_pair_window(self, lanes=0):
-        """Lanes per two-step workgroup: 64, 128 or 256 (0: 256 for FP32
-        requests, 64 for FP64)."""
+        """Window of the two-step launches: 64, 128 or 256 columns (0: by the
+        live set)."""
         self._check(self.lib.le2d_server_set_pair_window(self.h, lanes), "set_pair_window")
 
     def set_pair_split(self, on=1):
-        """64-lane two-step windows: the two stages on two wavefronts."""
+        """Kept for callers; nothing depends on it."""
         self._check(self.lib.le2d_server_set_pair_split(self.h, int(on)), "set_pair_split")
 
     def set_admission(self, max_queue=0, window=64, max_pass=16):

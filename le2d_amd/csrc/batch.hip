@@ -47,9 +47,8 @@ struct Shape {
   int fb, seg;
   int form;  // FORM_TILES: one workgroup per tile; FORM_PERSISTENT: resident
              // workgroups walk the table; FORM_PAIRS: one workgroup per tile of
-             // the two-step table, two steps per launch (fb 64, 128 or 256);
-             // FORM_PAIRS_SPLIT: the same with 64-lane windows whose two
-             // stages run on two wavefronts (march_pair_split)
+             // the two-step table, two steps per launch, in windows of 64, 128
+             // or 256 columns; FORM_PAIRS_SPLIT: the same in windows of 64
 };
 
 std::mutex g_tune_mu;
@@ -176,7 +175,8 @@ struct BatchImpl {
   int build_tiles(Shape s) {
     if (s.form == FORM_PAIRS && s.fb != 64 && s.fb != 128) s.fb = 256;
     if (s.form == FORM_PAIRS_SPLIT) s.fb = 64;
-    int rc = upload_table(two_step(s.form) ? s.fb - 8 : s.fb - 4, s.seg, &d_tiles, &ntiles);
+    int rc = upload_table(two_step(s.form) ? pair_cols(elem, s.fb) - 8 : s.fb - 4, s.seg, &d_tiles,
+                          &ntiles);
     if (rc) return rc;
     if (two_step(s.form)) {
       rc = upload_table(s.fb - 4, s.seg, &d_tiles1, &ntiles1);
@@ -206,12 +206,9 @@ struct BatchImpl {
     if (shape.form == FORM_PERSISTENT)
       hipLaunchKernelGGL((k_step_batch<T, FB>), dim3(blocks), dim3(FB), 0, stream, d, d_tiles,
                          ntiles, par);
-    else if (shape.form == FORM_PAIRS_SPLIT)
-      hipLaunchKernelGGL((k_step_batch_pairs_split<T>), dim3(ntiles), dim3(128), 0, stream, d,
-                         d_tiles, par);
-    else if (shape.form == FORM_PAIRS)
-      hipLaunchKernelGGL((k_step_batch_pairs<T, FB>), dim3(ntiles), dim3(FB), 0, stream, d,
-                         d_tiles, par);
+    else if (two_step(shape.form))
+      hipLaunchKernelGGL(batch_pair_kernel<T>(pair_cols(elem, FB)), dim3(ntiles), dim3(128), 0,
+                         stream, d, d_tiles, par);
     else
       hipLaunchKernelGGL((k_step_batch_tiles<T, FB>), dim3(ntiles), dim3(FB), 0, stream, d,
                          d_tiles, par);
@@ -366,27 +363,12 @@ int le2d_batch_commit(le2d_batch *b) {
   rc = B.elem == 8 ? B.upload_desc<double>() : B.upload_desc<float>();
   if (rc) return rc;
   // default shape until autotuned: the cached winner for this batch, else
-  // the two-step form in one-wave windows (the autotuner's choice in FP64,
-  // and within a few percent of it in FP32 on mixed batches) with the
-  // segment height that maximises (fill of the last round of resident
-  // workgroups) x (share of rows that are output rather than halo) over all
-  // instances
-  le2d::Shape s{64, 64, le2d::FORM_PAIRS};
-  {
-    long resident = le2d::pair_resident(B.elem, 64);
-    if (resident <= 0) resident = 2048;
-    double best_score = -1;
-    for (int seg : {8, 16, 32, 64, 128}) {
-      long blocks = 0;
-      for (const auto &in : B.inst) blocks += (long)((in.nx + 55) / 56) * ((in.ny + seg - 1) / seg);
-      const long rounds = (blocks + resident - 1) / resident;
-      const double score = (double)blocks / (double)(rounds * resident) * seg / (seg + 8);
-      if (score > best_score + 1e-9) {
-        best_score = score;
-        s.seg = seg;
-      }
-    }
-  }
+  // the two-step form in the window and segment height that the model of the
+  // single-grid pass gives for all instances together
+  std::vector<le2d::GridSize> sizes;
+  for (const auto &in : B.inst) sizes.push_back({in.nx, in.ny});
+  const le2d::PairShape p = le2d::pick_pair_shape(B.elem, sizes.data(), sizes.size(), 0, 160);
+  le2d::Shape s{p.window, p.seg, le2d::FORM_PAIRS};
   {
     std::lock_guard<std::mutex> lk(le2d::g_tune_mu);
     auto it = le2d::g_tune.find({B.elem, (int)B.inst.size(), B.total_nodes() >> 20});
@@ -537,8 +519,8 @@ int le2d_batch_autotune(le2d_batch *b, int trials, int *best_fb, int *best_seg, 
     for (int fb : fbs)
       for (int seg : segs) cand.push_back({fb, seg, form});
   for (int fb : fbs)
-    for (int seg : segs) cand.push_back({fb, seg, le2d::FORM_PAIRS});
-  for (int seg : segs) cand.push_back({64, seg, le2d::FORM_PAIRS_SPLIT});
+    for (int seg : segs)
+      if (le2d::pair_cols(B.elem, fb) == fb) cand.push_back({fb, seg, le2d::FORM_PAIRS});
   le2d::Shape best{B.shape};
   double best_t = 1e30;
   for (const le2d::Shape &c : cand) {

@@ -5,7 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
-#include "sweep_dev.h"
+#include "pair_dev.h"
 
 namespace le2d {
 
@@ -63,33 +63,41 @@ __global__ __launch_bounds__(FB, 3) void k_step_batch_tiles(const InstDesc<T> *_
 }
 
 // One workgroup per tile of the two-step table (strips of FB-8 columns): each
-// launch advances every instance by two steps (march_pair).
+// launch advances every instance by two steps (pair_tile), FB/64 columns per
+// lane ...
 template <typename T, int FB>
-__global__ __launch_bounds__(FB, 2) void k_step_batch_pairs(const InstDesc<T> *__restrict__ inst,
+__global__ __launch_bounds__(128, (pair_waves<T, FB / 64>())) void k_step_batch_pairs(const InstDesc<T> *__restrict__ inst,
                                                           const TileJob *__restrict__ tiles,
                                                           int step_parity) {
-  __shared__ W4<T> sw[pair_lds<FB>()];
-  __shared__ W4<T> sf[pair_lds<FB>()];
+  __shared__ PairLds<T, FB / 64> lds;
   const TileJob tj = tiles[xcd_tile(blockIdx.x, gridDim.x)];
   const InstDesc<T> &d = inst[tj.inst];
   const int p = d.par ^ step_parity;
-  march_pair<T, FB>(d.buf[p], d.buf[p ^ 1], d.nx, d.ny, d.pitch, d.plane, tj.strip, tj.j0, tj.j1,
-                    d.cx, d.cy, sw, sf);
+  pair_tile<T, FB / 64>(d.buf[p], d.buf[p ^ 1], d.nx, d.ny, d.pitch, d.plane, tj.strip, tj.j0,
+                        tj.j1, d.cx, d.cy, lds);
 }
 
-// The same with 64-lane windows whose two stages run on two wavefronts of
-// a 128-lane workgroup (march_pair_split).
+// ... or one.
 template <typename T>
-__global__ __launch_bounds__(128, 3) void k_step_batch_pairs_split(
+__global__ __launch_bounds__(128, (pair_waves<T, 1>())) void k_step_batch_pairs_split(
     const InstDesc<T> *__restrict__ inst, const TileJob *__restrict__ tiles, int step_parity) {
-  __shared__ W4<T> sw[128];
-  __shared__ W4<T> sf[128];
-  __shared__ T ring[2 * kSplitRows * 5 * 64];
+  __shared__ PairLds<T, 1> lds;
   const TileJob tj = tiles[xcd_tile(blockIdx.x, gridDim.x)];
   const InstDesc<T> &d = inst[tj.inst];
   const int p = d.par ^ step_parity;
-  march_pair_split<T, sizeof(T) == 4>(d.buf[p], d.buf[p ^ 1], d.nx, d.ny, d.pitch, d.plane,
-                                      tj.strip, tj.j0, tj.j1, d.cx, d.cy, sw, sf, ring);
+  pair_tile<T, 1>(d.buf[p], d.buf[p ^ 1], d.nx, d.ny, d.pitch, d.plane, tj.strip, tj.j0, tj.j1,
+                  d.cx, d.cy, lds);
+}
+
+// The batched two-step kernel of a window of `cols` columns (pair_cols).
+template <typename T>
+using BatchPairKernel = void (*)(const InstDesc<T> *, const TileJob *, int);
+template <typename T>
+inline BatchPairKernel<T> batch_pair_kernel(int cols) {
+  if (cols == 64) return k_step_batch_pairs_split<T>;
+  if constexpr (sizeof(T) == 4)
+    if (cols == 256) return k_step_batch_pairs<T, 256>;
+  return k_step_batch_pairs<T, 128>;
 }
 
 // Disk initial condition with the host le_set_ball's arithmetic: the node

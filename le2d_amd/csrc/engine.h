@@ -47,8 +47,9 @@ struct Tiles {
   int xy_seg;   // rows per segment of the fused x+y step
   int xy_block; // lanes per fused-step workgroup (64, 128, 256); writes xy_block-4 columns
   int pair_seg; // rows per segment of the two-step pass (0: one step per pass)
-  int pair_block; // lanes per two-step workgroup (64, 128 or 256); writes pair_block-8 columns
-  int pair_split = 0; // 64-lane two-step windows: the two stages on two wavefronts
+  int pair_block; // window of the two-step pass: 64, 128 or 256 columns (pair_cols)
+  int pair_split = 0; // a caller's setting that is kept and reported; every window runs its
+                      // two stages on two wavefronts
 };
 
 struct DevGrid {
@@ -119,14 +120,30 @@ int step2_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy);
 int copy_probe(size_t bytes, int iters, double *ms);
 
 Tiles default_tiles(int elem, int nx, int ny);
-// Workgroups of the two-step kernel (element size elem, fb lanes) resident on
-// the current device at once (occupancy API x compute units); 0 if unknown.
-long pair_resident(int elem, int fb);
+// Columns that a two-step window setting of 64, 128 or 256 runs in (of which
+// 8 are halo): FP64 at most 128, as two columns per lane fill the registers.
+inline int pair_cols(int elem, int window) {
+  const int most = elem == 8 ? 128 : 256;
+  return window < most ? window : most;
+}
+// Workgroups of the two-step kernel of a window setting that make one round
+// on the current device: the resident ones (occupancy API x compute units), at
+// most the four per CU that saturate it; 0 if unknown.
+long pair_resident(int elem, int window);
 // The same for the single-step kernel (clamped edges).
 long step_resident(int elem, int fb);
-// Segment height of the two-step pass for an nx x ny grid in windows of fb
-// lanes, from the occupancy model in default_tiles.
-int pair_seg_for(int elem, int nx, int ny, int fb);
+// Window setting and segment height (at most `cap` rows) of one two-step launch
+// over n grids, from the model in engine.hip; only: that window (0: any).
+struct GridSize {
+  int nx, ny;
+};
+struct PairShape {
+  int window, seg;
+};
+PairShape pick_pair_shape(int elem, const GridSize *g, size_t n, int only, int cap);
+// Segment heights at which an nx x ny grid's workgroups fill 1 .. 8 rounds of
+// the resident ones.
+std::vector<int> pair_round_segs(int elem, int nx, int ny, int window);
 // One grid row (five padded field rows) fits the 31-bit range of a buffer
 // resource, which the row loads and stores address through.
 bool row_fits(int elem, int nx);
@@ -160,6 +177,7 @@ struct MatPlane {
   MatTile *d_homog2 = nullptr, *d_mixed2 = nullptr;
   MixBlock *d_blocks2 = nullptr;  // the interface tiles as blocks, or none
   int n_homog2 = 0, n_mixed2 = 0, n_blocks2 = 0;
+  int full_homog2 = 0;  // the first of d_homog2: tiles of a whole segment
   int built_pair_seg = -1, built_pair_fb = -1;
   // the interface tiles run on a second stream beside the single-material
   // ones (forked from and joined back into the grid's stream)

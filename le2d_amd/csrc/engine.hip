@@ -312,14 +312,10 @@ Tiles default_tiles(int elem, int nx, int ny) {
   if (seg < 32) seg = 32;
   if (seg > ny) seg = ny;
   t.y_seg = (int)seg;
-  // two-step pass (le_step_n, paired le_step calls), measured on MI355X:
-  // FP64 takes one-wave windows (64 lanes, 56 columns, no barriers between
-  // waves; 8192^2 at 80-row segments 90 Gnode-updates/s against 85 with 128
-  // or 256 lanes).  FP32, issue- rather than latency-bound, keeps the 3% halo
-  // of 256-lane windows on grids 4096 or more columns wide (8192^2 229
-  // against 210; 2048^2 137 against 153 with 64 lanes).
-  t.pair_block = elem == 8 || nx < 4096 ? 64 : 256;
-  t.pair_seg = pair_seg_for(elem, nx, ny, t.pair_block);
+  const GridSize size{nx, ny};
+  const PairShape p = pick_pair_shape(elem, &size, 1, 0, 192);
+  t.pair_block = p.window;
+  t.pair_seg = p.seg;
   return t;
 }
 
@@ -329,7 +325,7 @@ Tiles default_tiles(int elem, int nx, int ny) {
 static int best_segment(long strips, int ny, long resident, int halo, int cap) {
   int best = 2;
   double best_score = -1;
-  for (int s : {2, 4, 6, 8, 12, 16, 24, 32, 48, 64, 80}) {
+  for (int s : {2, 4, 6, 8, 12, 16}) {
     if (s > cap || (s > ny && s != 2)) break;
     const long blocks = strips * ((ny + s - 1) / s);
     const long rounds = (blocks + resident - 1) / resident;
@@ -344,24 +340,68 @@ static int best_segment(long strips, int ny, long resident, int halo, int cap) {
   return best;
 }
 
-// Segment height of the two-step pass: the candidate height that maximises
-// (fill of the last round of resident workgroups) x (share of a segment's
-// rows that are output rather than the 8 re-read halo rows).  The grid's
-// workgroups run in rounds of `resident`; a last round that is mostly empty
-// leaves the device idle.  Taller segments than 80 rows (64-lane windows)
-// or 64 (wider) measured slower than the model says and are not taken.
-// Measured optima it reproduces (Gnode-updates/s): FP64 64 lanes, 80 rows
-// on 8192^2 (90.2; 86.4 at 160), 8192 x 1024 (75.2; 66.7 at 32) and 4096^2
-// (79.7), 48 on 2048^2 (61.0); FP32 256 lanes, 64 rows on 8192^2 (229.4;
-// 223.5 at 128) and 16384^2 (231.1; 223.2 at 160).  On grids whose
-// workgroups all fit in one round the pass lasts one workgroup's march, so
-// short segments win: FP64 12 rows on 1024^2 (43.2; 36.6 at 16), 4 on 512^2
-// (18.2; 13.4 at 16), 2 on 256^2 (7.3; 3.5 at 16).
-int pair_seg_for(int elem, int nx, int ny, int fb) {
-  long resident = pair_resident(elem, fb);
-  if (resident <= 0) resident = 2048;
-  const long strips = (nx + fb - 9) / (fb - 8);
-  return best_segment(strips, ny, resident, 8, fb == 64 ? 80 : 64);
+static long pair_slots(int elem, int window) {
+  const long r = pair_resident(elem, window);
+  return r > 0 ? r : 1024;
+}
+
+std::vector<int> pair_round_segs(int elem, int nx, int ny, int window) {
+  const int width = pair_cols(elem, window) - 8;
+  const long strips = (nx + width - 1) / width, slots = pair_slots(elem, window);
+  std::vector<int> segs;
+  for (long k = 1; k <= 8; ++k) {
+    const long n = k * slots / strips;
+    const int s = n > 0 ? (int)std::max<long>(2, (ny + n - 1) / n) : 0;
+    if (s && s <= 192 && (segs.empty() || segs.back() != s)) segs.push_back(s);
+  }
+  return segs;
+}
+
+// Cost of a shape: rounds of workgroups x rows each marches (its segment and
+// the 8 re-read halo rows) x columns of its window, per unit of the window's
+// rate.  A round is the workgroups that saturate the device, four per CU (two
+// wavefronts per SIMD: FP64 1024^2 in 64-column windows 40 us at 20 rows with
+// 1.9 wavefronts per SIMD, 44 at 16 with 2.4); a last round that is mostly
+// empty costs as much as a full one (FP64 2048^2 in 128-column windows 109 us at
+// 37 rows, one full round, 132 at 32 and 138 at 54), and a grid that does not
+// fill a round takes the shortest segments that stay in it (FP64 512^2 19 us at
+// 6 rows, 20.5 at 8).  Wider windows recompute fewer halo columns but need a
+// larger grid (FP64 2048^2 109 us at 128 columns against 120 at 64, 8192^2 1.55
+// ms against 1.64, but 1024^2 46 us against 40; FP32 8192^2 0.59 ms at 256
+// against 0.64 at 128 and 0.67 at 64, but 2048^2 51 us against 45 at 64).  The rates
+// are what wide windows gain beyond their smaller halo.
+PairShape pick_pair_shape(int elem, const GridSize *g, size_t n, int only, int cap) {
+  // one grid: every height; several: enough of them to meet a round closely
+  static const int few[] = {2,  3,  4,  5,  6,  7,  8,  10, 12,  14,  16,  18,  20, 24,
+                            28, 32, 37, 42, 48, 56, 64, 72, 80,  96,  112, 128, 144, 160};
+  PairShape best{only ? only : 64, 2};
+  double best_cost = 1e300;
+  for (int w : {64, 128, 256}) {
+    const int cols = pair_cols(elem, w), width = cols - 8;
+    if (only ? w != only : cols != w) continue;
+    const double rate = cols == 64 ? 1.0 : cols == 128 ? (elem == 8 ? 1.08 : 1.0) : 1.05;
+    const long slots = pair_slots(elem, w);
+    const int count = n == 1 ? 191 : (int)(sizeof few / sizeof *few);
+    for (int k = 0; k < count; ++k) {
+      const int s = n == 1 ? k + 2 : few[k];
+      if (s > cap && k) break;
+      long blocks = 0;
+      int tall = 0;
+      for (size_t i = 0; i < n; ++i) {
+        blocks += (long)((g[i].nx + width - 1) / width) * ((g[i].ny + s - 1) / s);
+        tall = std::max(tall, g[i].ny);
+      }
+      const long rounds = (blocks + slots - 1) / slots;
+      const double cost = (double)rounds * (std::min(s, tall) + 8) * cols / rate;
+      if (cost < best_cost * (1 - 1e-9)) {
+        best_cost = cost;
+        best = {w, s};
+      }
+      if (s >= tall) break;
+    }
+  }
+  best.seg = std::max(1, std::min(best.seg, cap));
+  return best;
 }
 
 // One 16-byte vector per lane, one pass: the fastest copy shape measured on

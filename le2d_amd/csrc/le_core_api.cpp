@@ -43,7 +43,6 @@ struct TaskState {
   int mode = LE2D_SYNC_WAIT;
   hipStream_t stream = nullptr;
   bool pairs_fixed = false;  // segment height set by the caller or tuned
-  bool mat_split_tuned = false;  // material plane: one or two wavefronts chosen
   // A step accepted by le_step but not yet run, so that it and the next
   // le_step share one two-step pass; run before anything else touches the
   // device state (flush_pending), with the coefficients it was called with.
@@ -53,9 +52,10 @@ struct TaskState {
 
 std::mutex g_mu;
 std::unordered_map<const real *, TaskState *> g_tasks;
-// tuned two-step segment heights per (element size, nx, ny), for the process
+// tuned two-step segment heights and windows per (element size, nx, ny), for
+// the process
 std::mutex g_pair_mu;
-std::map<std::tuple<int, int, int>, std::tuple<int, int, int>> g_pair_seg;  // rows, lanes, split
+std::map<std::tuple<int, int, int>, std::pair<int, int>> g_pair_seg;
 
 int env_mode() {
   const char *s = getenv("LE2D_SYNC");
@@ -167,9 +167,8 @@ int tune_pairs(le_task *t, TaskState *s) {
     std::lock_guard<std::mutex> lk(g_pair_mu);
     auto it = g_pair_seg.find(key);
     if (it != g_pair_seg.end()) {
-      s->g.tiles.pair_seg = std::get<0>(it->second);
-      s->g.tiles.pair_block = std::get<1>(it->second);
-      s->g.tiles.pair_split = std::get<2>(it->second);
+      s->g.tiles.pair_seg = it->second.first;
+      s->g.tiles.pair_block = it->second.second;
       s->pairs_fixed = true;
       return LE2D_OK;
     }
@@ -180,10 +179,9 @@ int tune_pairs(le_task *t, TaskState *s) {
   for (auto &e : ev) (void)hipEventCreate(&e);
   int rc = LE2D_OK;
   // mean ms of one pass at (block, seg) after one untimed pass; < 0 on error
-  auto time_one = [&](int block, int split, int seg, int reps) -> float {
+  auto time_one = [&](int block, int seg, int reps) -> float {
     s->g.tiles.pair_seg = seg;
     s->g.tiles.pair_block = block;
-    s->g.tiles.pair_split = split;
     for (int k = 0; k <= reps && !rc; ++k) {
       if (k == 1) (void)hipEventRecord(ev[0], s->stream);
       rc = le2d::step2_xy<real>(&s->g, cx, cy);
@@ -200,89 +198,61 @@ int tune_pairs(le_task *t, TaskState *s) {
   };
   struct Cand {
     float ms;
-    int block, split, seg;
+    int block, seg;
   };
   // warm-up at the default shape, about 25 ms: after host-side work the
   // device clocks are still low and would make the first candidates look slow
   {
-    const int b0 = s->g.tiles.pair_block, p0 = s->g.tiles.pair_split, s0 = s->g.tiles.pair_seg;
-    const float est = time_one(b0, p0, s0, 1);
+    const int b0 = s->g.tiles.pair_block, s0 = s->g.tiles.pair_seg;
+    const float est = time_one(b0, s0, 1);
     if (est > 0) {
       const int reps = std::max(1, std::min(64, (int)(25.0f / est)));
-      (void)time_one(b0, p0, s0, reps);
+      (void)time_one(b0, s0, reps);
     }
   }
   std::vector<Cand> res;
-  // windows: 256, 128 and 64 lanes, and 64-lane windows with the two stages
-  // on two wavefronts (k_step2_split)
-  const int blocks[4][2] = {{256, 0}, {128, 0}, {64, 0}, {64, 1}};
-  for (const auto &bs : blocks) {
-    const int block = bs[0], split = bs[1];
+  for (int block : {256, 128, 64}) {
+    if (le2d::pair_cols((int)sizeof(real), block) != block) continue;
     // segments under 16 rows only for grids that 16-row segments leave short
     // of one round of resident workgroups (there a pass lasts one
     // workgroup's march)
     const long strips = (s->g.nx + block - 9) / (block - 8);
     const long resident = le2d::pair_resident((int)sizeof(real), block);
-    const bool small = strips * ((s->g.ny + 15) / 16) < (resident > 0 ? resident : 2048);
+    const bool small = strips * ((s->g.ny + 15) / 16) < (resident > 0 ? resident : 1024);
+    std::vector<int> segs;
     for (int seg : cand) {
       if (seg < 16 && !small) continue;
       if (seg > s->g.ny && seg != cand[0]) break;  // taller segments are all one
-      const float ms = time_one(block, split, seg, 4);
+      segs.push_back(seg);
+    }
+    if (!small)  // and the heights that fill whole rounds
+      for (int seg : le2d::pair_round_segs((int)sizeof(real), s->g.nx, s->g.ny, block))
+        if (seg >= 16 && seg <= s->g.ny && !std::count(segs.begin(), segs.end(), seg))
+          segs.push_back(seg);
+    for (int seg : segs) {
+      const float ms = time_one(block, seg, 4);
       if (ms < 0) break;
-      res.push_back({ms, block, split, seg});
+      res.push_back({ms, block, seg});
     }
   }
-  Cand best{1e30f, 256, 0, 64};
+  Cand best{1e30f, 128, 64};
   if (!rc && !res.empty()) {
     std::sort(res.begin(), res.end(), [](const Cand &a, const Cand &b) { return a.ms < b.ms; });
     if (res.size() > 3) res.resize(3);
     for (const Cand &c : res) {
-      const float ms = time_one(c.block, c.split, c.seg, 12);
+      const float ms = time_one(c.block, c.seg, 12);
       if (ms < 0) break;
-      if (ms < best.ms) best = {ms, c.block, c.split, c.seg};
+      if (ms < best.ms) best = {ms, c.block, c.seg};
     }
   }
   for (auto &e : ev) (void)hipEventDestroy(e);
   s->g.tiles.pair_seg = best.seg;
   s->g.tiles.pair_block = best.block;
-  s->g.tiles.pair_split = best.split;
   s->pairs_fixed = true;
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(g_pair_mu);
-  g_pair_seg[key] = std::make_tuple(best.seg, best.block, best.split);
+  g_pair_seg[key] = {best.seg, best.block};
   return LE2D_OK;
-}
-
-// Material planes keep their default window and segment height (other
-// shapes would rebuild the tile tables on the host), but with 64-lane windows
-// the two forms of the pass share the tables: time each over three passes,
-// out of place (each pass reads the current state and writes the idle
-// buffer; the swap is undone), and keep the faster.
-int tune_mat_split(TaskState *s) {
-  hipEvent_t ev[2];
-  for (auto &e : ev) (void)hipEventCreate(&e);
-  int rc = LE2D_OK, pick = 0;
-  float best = 1e30f;
-  for (int split : {0, 1}) {
-    s->g.tiles.pair_split = split;
-    for (int k = 0; k <= 3 && !rc; ++k) {
-      if (k == 1) (void)hipEventRecord(ev[0], s->stream);
-      rc = le2d::step2_xy_mat<real>(&s->g, &s->mat);
-      if (!rc) s->g.cur ^= 1;  // the state has not moved
-    }
-    (void)hipEventRecord(ev[1], s->stream);
-    if (rc || hipEventSynchronize(ev[1]) != hipSuccess) break;
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, ev[0], ev[1]);
-    if (ms < best) {
-      best = ms;
-      pick = split;
-    }
-  }
-  for (auto &e : ev) (void)hipEventDestroy(e);
-  s->g.tiles.pair_split = pick;
-  s->mat_split_tuned = true;
-  return rc;
 }
 
 bool tuning_enabled() {
@@ -338,12 +308,6 @@ int run(le_task *t, int what, int edge, int steps, bool defer = false) {
   if (what == (DO_X | DO_Y) && edge == le2d::EDGE_CLAMP && s->g.tiles.pair_seg > 0 &&
       !s->pairs_fixed && !s->mat.active && steps >= 8 && tuning_enabled()) {
     rc = tune_pairs(t, s);
-    if (rc) return rc;
-  }
-  if (what == (DO_X | DO_Y) && edge == le2d::EDGE_CLAMP && s->g.tiles.pair_seg > 0 &&
-      s->g.tiles.pair_block == 64 && !s->pairs_fixed && s->mat.active && !s->mat_split_tuned &&
-      steps >= 8 && tuning_enabled()) {
-    rc = tune_mat_split(s);
     if (rc) return rc;
   }
   if (what == (DO_X | DO_Y) && edge == le2d::EDGE_CLAMP && s->g.tiles.pair_seg > 0) {
@@ -826,12 +790,22 @@ int le2d_set_material_plane(le_task *task, int count, const double *c1_c2_rho,
   TaskState *s = find(task);
   int rc = ensure_device(task, s);
   if (rc) return rc;
+  if (!s->pairs_fixed) {
+    // With a plane the default two-step window is 64 columns below 2^26 nodes:
+    // wider ones put more nodes into tiles that hold an interface than they save in
+    // halo columns (4100 x 3000 FP64 402 us a pass against 425 at 128, FP32
+    // 147 against 168 at 256).
+    const le2d::GridSize g{s->g.nx, s->g.ny};
+    const int only = count > 0 && (long)g.nx * g.ny < (1L << 26) ? 64 : 0;
+    const le2d::PairShape p = le2d::pick_pair_shape((int)sizeof(real), &g, 1, only, 192);
+    s->g.tiles.pair_block = p.window;
+    s->g.tiles.pair_seg = p.seg;
+  }
   if (count == 0) {
     le2d::mat_release(&s->mat);
     s->mat.active = false;
     return LE2D_OK;
   }
-  s->mat_split_tuned = false;
   return le2d::mat_set(&s->g, &s->mat, count, c1_c2_rho, ids, (double)task->dt,
                        (double)task->h.x, (double)task->h.y);
 }

@@ -12,7 +12,7 @@
 #include <mutex>
 #include <vector>
 
-#include "sweep_dev.h"
+#include "pair_dev.h"
 
 namespace le2d {
 
@@ -46,46 +46,51 @@ __global__ __launch_bounds__(FB) void k_step_mat_mixed(const T *__restrict__ src
                                 cxt, cyt, sn);
 }
 
-// Two-step pass: single-material tiles run march_pair with their material's
-// constants, the others the node-local two-step march; both in windows of FB
-// lanes (strips of FB-8 columns), the grid's two-step window width.
+// Order of the two-step pass's single-material tiles: the `full` ones of a whole
+// segment in XCD-aware order, then the shorter ones left of tiles that hold an
+// interface.  A full tile that starts last would add a whole march to the pass
+// (4100 x 3000 FP64 in 128-column windows 442 us a pass in one XCD-aware order,
+// 385 in this one).
+__device__ __forceinline__ int homog_tile(int k, int full) {
+  return k < full ? xcd_tile(k, full) : k;
+}
+
+// Two-step pass: single-material tiles run pair_tile with their material's
+// constants, the others the node-local two-step march; both in strips of FB-8
+// columns, the grid's two-step window.
 template <typename T, int FB>
-__global__ __launch_bounds__(FB, 2) void k_step2_mat_homog(const T *__restrict__ src,
+__global__ __launch_bounds__(128, (pair_waves<T, FB / 64>())) void k_step2_mat_homog(const T *__restrict__ src,
                                                          T *__restrict__ dst, int nx, int ny,
                                                          long pitch, long plane,
                                                          const MatTile *__restrict__ tiles,
+                                                         int full,
                                                          const SweepCoef<T> *__restrict__ cxt,
                                                          const SweepCoef<T> *__restrict__ cyt) {
-  __shared__ W4<T> sw[pair_lds<FB>()];
-  __shared__ W4<T> sf[pair_lds<FB>()];
-  const MatTile tj = tiles[xcd_tile(blockIdx.x, gridDim.x)];
+  __shared__ PairLds<T, FB / 64> lds;
+  const MatTile tj = tiles[homog_tile(blockIdx.x, full)];
   const SweepCoef<T> cx = cxt[tj.mat], cy = cyt[tj.mat];
-  march_pair<T, FB>(src, dst, nx, ny, pitch, plane, tj.strip, tj.j0, tj.j1, cx, cy, sw, sf);
+  pair_tile<T, FB / 64>(src, dst, nx, ny, pitch, plane, tj.strip, tj.j0, tj.j1, cx, cy, lds);
 }
 
-// The same for 64-lane windows with the two stages on two wavefronts
-// (march_pair_split).
+// The same in windows of 64 columns.
 template <typename T>
-__global__ __launch_bounds__(128, 3) void k_step2_mat_homog_split(
+__global__ __launch_bounds__(128, (pair_waves<T, 1>())) void k_step2_mat_homog_split(
     const T *__restrict__ src, T *__restrict__ dst, int nx, int ny, long pitch, long plane,
-    const MatTile *__restrict__ tiles, const SweepCoef<T> *__restrict__ cxt,
+    const MatTile *__restrict__ tiles, int full, const SweepCoef<T> *__restrict__ cxt,
     const SweepCoef<T> *__restrict__ cyt) {
-  __shared__ W4<T> sw[128];
-  __shared__ W4<T> sf[128];
-  __shared__ T ring[2 * kSplitRows * 5 * 64];
-  const MatTile tj = tiles[xcd_tile(blockIdx.x, gridDim.x)];
+  __shared__ PairLds<T, 1> lds;
+  const MatTile tj = tiles[homog_tile(blockIdx.x, full)];
   const SweepCoef<T> cx = cxt[tj.mat], cy = cyt[tj.mat];
-  march_pair_split<T, sizeof(T) == 4>(src, dst, nx, ny, pitch, plane, tj.strip, tj.j0, tj.j1, cx,
-                                      cy, sw, sf, ring);
+  pair_tile<T, 1>(src, dst, nx, ny, pitch, plane, tj.strip, tj.j0, tj.j1, cx, cy, lds);
 }
 
 // Interface tiles of the two-step pass, launched beside the single-material
-// kernel.  At 64 lanes that is the two-wavefront form, three waves of at most
-// 168 VGPRs per SIMD: held to the same bound, a wave of this kernel starts as
-// soon as one neighbouring wave ends (128 lanes keep the bound too, without
-// spilling).  At 256 lanes two waves per SIMD keep it free of spills.
+// kernel.  In windows of 64 columns that runs three waves of at most 168 VGPRs
+// per SIMD: held to the same bound, a wave of this kernel starts as soon as
+// one neighbouring wave ends (128 lanes keep the bound too, without
+// spilling).
 template <typename T, int FB>
-__global__ __launch_bounds__(FB, FB == 256 ? 2 : 3) void k_step2_mat_mixed(
+__global__ __launch_bounds__(FB, 3) void k_step2_mat_mixed(
     const T *__restrict__ src, T *__restrict__ dst, int nx, int ny, long pitch, long plane,
     const MatTile *__restrict__ tiles, const unsigned char *__restrict__ ids, long idp,
     const SweepCoef<T> *__restrict__ cxt, const SweepCoef<T> *__restrict__ cyt) {
@@ -526,11 +531,6 @@ static int join_aux(DevGrid *g, MatPlane *m) {
   return OK;
 }
 
-static int pair_lanes(const DevGrid *g) {
-  const int fb = g->tiles.pair_block;
-  return fb == 64 || fb == 128 ? fb : 256;
-}
-
 // Whether the interface tiles run as `blocks` blocks rather than as `mixed`
 // marched tiles of `lanes` lanes and `rows` rows.  Measured (FP64 / FP32): a
 // round of blocks, one / two per CU, takes 11 / 7 us; a marched row 5 / 3 us while
@@ -549,10 +549,11 @@ static bool blocks_pay(int elem, size_t mixed, int lanes, int rows, size_t block
 // Tables of the two-step pass: strips of (window - 8) columns read 4 halo
 // columns and 4 halo rows on each side.
 static int mat_tiles2(DevGrid *g, MatPlane *m) {
-  const int seg = g->tiles.pair_seg, fb = pair_lanes(g);
+  const int seg = g->tiles.pair_seg, fb = pair_cols(g->elem, g->tiles.pair_block);
   if (m->built_pair_seg == seg && m->built_pair_fb == fb) return OK;
   std::vector<MatTile> homog, mixed;
   split_tiles(m, g->nx, g->ny, fb - 8, 4, seg, 4, EDGE_CLAMP, &homog, &mixed);
+  m->full_homog2 = (int)homog.size();
   std::vector<MatTile> homogb = homog;
   std::vector<MixBlock> blocks;
   split_bands(m, g->nx, g->ny, fb - 8, mixed, &homogb, &blocks);
@@ -591,12 +592,15 @@ static int launch_mat2(DevGrid *g, MatPlane *m) {
     hipLaunchKernelGGL((k_step2_mat_block<T>), dim3(m->n_blocks2), dim3((kMixRows + 8) * 64), 0,
                        g->stream, src, dst, g->nx, g->ny, g->pitch, g->plane, m->d_blocks2,
                        m->d_ids, m->idp, cx, cy);
-  if (m->n_homog2 && FB == 64 && g->tiles.pair_split)
-    hipLaunchKernelGGL((k_step2_mat_homog_split<T>), dim3(m->n_homog2), dim3(128), 0, g->stream,
-                       src, dst, g->nx, g->ny, g->pitch, g->plane, m->d_homog2, cx, cy);
-  else if (m->n_homog2)
-    hipLaunchKernelGGL((k_step2_mat_homog<T, FB>), dim3(m->n_homog2), dim3(FB), 0, g->stream, src,
-                       dst, g->nx, g->ny, g->pitch, g->plane, m->d_homog2, cx, cy);
+  if (m->n_homog2) {
+    const dim3 grid(m->n_homog2);
+    if constexpr (FB == 64)
+      hipLaunchKernelGGL((k_step2_mat_homog_split<T>), grid, dim3(128), 0, g->stream, src, dst,
+                         g->nx, g->ny, g->pitch, g->plane, m->d_homog2, m->full_homog2, cx, cy);
+    else
+      hipLaunchKernelGGL((k_step2_mat_homog<T, FB>), grid, dim3(128), 0, g->stream, src, dst,
+                         g->nx, g->ny, g->pitch, g->plane, m->d_homog2, m->full_homog2, cx, cy);
+  }
   return m->n_mixed2 ? join_aux(g, m) : OK;
 }
 
@@ -650,10 +654,13 @@ int step2_xy_mat(DevGrid *g, MatPlane *m) {
   if (g->tiles.pair_seg < 1) return set_error(ERR_ARG, "step2_xy_mat: no pair segment height");
   int rc = mat_tiles2(g, m);
   if (rc) return rc;
-  const int fb = pair_lanes(g);
-  rc = fb == 64    ? launch_mat2<T, 64>(g, m)
-       : fb == 128 ? launch_mat2<T, 128>(g, m)
-                   : launch_mat2<T, 256>(g, m);
+  const int cols = pair_cols(g->elem, g->tiles.pair_block);
+  if constexpr (sizeof(T) == 4)
+    rc = cols == 64    ? launch_mat2<T, 64>(g, m)
+         : cols == 128 ? launch_mat2<T, 128>(g, m)
+                       : launch_mat2<T, 256>(g, m);
+  else
+    rc = cols == 64 ? launch_mat2<T, 64>(g, m) : launch_mat2<T, 128>(g, m);
   if (rc) return rc;
   rc = mcheck(hipGetLastError(), "step2_xy_mat launch");
   if (rc) return rc;

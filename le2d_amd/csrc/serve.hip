@@ -119,20 +119,17 @@ struct Server {
   int window = 64, max_pass = 16;
   int fb = 256, seg = 16;
   int pair_seg = 64;  // two-step launches: largest segment height; 0: one step per launch
-  // lanes per two-step workgroup (64, 128 or 256); 0: 256 for FP32 requests,
-  // which are issue-bound, 64 (one wavefront, no barriers between waves)
-  // for FP64, which are latency-bound
+  // window of the two-step pass (64, 128 or 256 columns); 0: by the live set
   int pair_fb = 0;
-  // 64-lane two-step windows with the two stages on two wavefronts
-  int pair_split = 0;
+  int pair_split = 0;  // kept for callers; the windows' launches do not depend on it
   // The settings above are written by API calls (under mu); the engine
   // thread launches with this copy, taken under mu whenever it rebuilds the
   // tables, so a setting that changes mid-chunk never meets tables built
   // for another.
   struct Launch {
-    int fb = 256, seg = 16, pair_seg = 64, pair_fb = 0, pair_split = 0;
+    int fb = 256, seg = 16, pair_seg = 64, pair_fb = 0;
   } act;
-  int pair_lanes(int si) const { return act.pair_fb ? act.pair_fb : (si == 1 ? 64 : 256); }
+  int pair_window[2] = {64, 64};  // columns of the current tables' two-step windows
   char *arena_dev = nullptr;
   Arena arena;
   std::mutex mu;
@@ -244,39 +241,27 @@ struct Server {
     return OK;
   }
 
-  // Two-step segment height for the live set of one precision: the height,
-  // at most pair_seg rows, that maximises (fill of the last round of
-  // resident workgroups) x (share of rows that are output rather than halo)
-  // over all live requests.  Many live requests keep tall segments; the few
-  // of a light load or of the tail of a burst take short ones, as a small
-  // grid does.
-  int live_pair_seg(int si, const std::vector<Req *> &set) const {
-    const int lanes = pair_lanes(si);
-    long resident = pair_resident(si == 1 ? 8 : 4, lanes);
-    if (resident <= 0) resident = 2048;
-    int best = std::min(act.pair_seg, 2);
-    double best_score = -1;
-    for (int s : {2, 4, 6, 8, 12, 16, 24, 32, 48, 64, 80, 96, 128}) {
-      if (s > act.pair_seg) break;
-      long blocks = 0;
-      for (const Req *r : set)
-        blocks += (long)((r->spec.nx + lanes - 9) / (lanes - 8)) * ((r->spec.ny + s - 1) / s);
-      if (blocks <= 0) break;
-      const long rounds = (blocks + resident - 1) / resident;
-      const double score = (double)blocks / (double)(rounds * resident) * s / (s + 8);
-      if (score > best_score + 1e-9) {
-        best_score = score;
-        best = s;
-      }
-    }
-    return best;
+  // Window and segment height (at most pair_seg rows) of the two-step launches
+  // for the live set of one precision, from the model of the single-grid
+  // pass over all live requests.  Many live requests keep wide windows and
+  // tall segments; the few of a light load or of the tail of a burst take
+  // narrow and short ones, as a small grid does.
+  PairShape live_pair_shape(int si, const std::vector<Req *> &set) const {
+    std::vector<GridSize> g;
+    for (const Req *r : set) g.push_back({r->spec.nx, r->spec.ny});
+    return pick_pair_shape(si == 1 ? 8 : 4, g.data(), g.size(), act.pair_fb, act.pair_seg);
   }
 
   template <typename T>
   int build_tables(int si, const std::vector<Req *> &set) {
     std::vector<InstDesc<T>> desc(set.size());
     std::vector<TileJob> tiles, tiles2;
-    const int seg2 = act.pair_seg > 0 ? live_pair_seg(si, set) : 0;
+    int seg2 = 0;
+    if (act.pair_seg > 0) {
+      const PairShape p = live_pair_shape(si, set);
+      seg2 = p.seg;
+      pair_window[si] = pair_cols((int)sizeof(T), p.window);
+    }
     pre1[si].assign(1, 0);
     pre2[si].assign(1, 0);
     for (size_t i = 0; i < set.size(); ++i) {
@@ -296,9 +281,9 @@ struct Server {
       for (int j0 = 0; j0 < q.ny; j0 += sg)
         for (int s = 0; s < strips; ++s)
           tiles.push_back({(int)i, s, j0, std::min(j0 + sg, q.ny), j0 / sg});
-      if (act.pair_seg > 0) {  // strips of lanes - 8 output columns (k_step_batch_pairs)
-        const int lanes = pair_lanes(si);
-        const int strips2 = (q.nx + lanes - 9) / (lanes - 8);
+      if (act.pair_seg > 0) {  // strips of the window less 8 columns
+        const int width = pair_window[si] - 8;
+        const int strips2 = (q.nx + width - 1) / width;
         const int sg2 = std::max(1, std::min(seg2, q.ny));
         for (int j0 = 0; j0 < q.ny; j0 += sg2)
           for (int s = 0; s < strips2; ++s)
@@ -354,19 +339,8 @@ struct Server {
     if (count <= 0) return;
     const dim3 grid((unsigned)count);
     const InstDesc<T> *d = static_cast<const InstDesc<T> *>(d_inst[si]);
-    const int lanes = pair_lanes(si);
-    if (lanes == 64 && act.pair_split)
-      hipLaunchKernelGGL((k_step_batch_pairs_split<T>), grid, dim3(128), 0, stream[si], d,
-                         d_tiles2[si], step_parity);
-    else if (lanes == 64)
-      hipLaunchKernelGGL((k_step_batch_pairs<T, 64>), grid, dim3(64), 0, stream[si], d,
-                         d_tiles2[si], step_parity);
-    else if (lanes == 128)
-      hipLaunchKernelGGL((k_step_batch_pairs<T, 128>), grid, dim3(128), 0, stream[si], d,
-                         d_tiles2[si], step_parity);
-    else
-      hipLaunchKernelGGL((k_step_batch_pairs<T, 256>), grid, dim3(256), 0, stream[si], d,
-                         d_tiles2[si], step_parity);
+    hipLaunchKernelGGL(batch_pair_kernel<T>(pair_window[si]), grid, dim3(128), 0, stream[si], d,
+                       d_tiles2[si], step_parity);
   }
 
   // Requests of the current tables of precision si with at least k steps
@@ -457,7 +431,7 @@ struct Server {
           set[r.spec.real_size == 8 ? 1 : 0].push_back(&r);
         }
         if (dirty) {
-          act = {fb, seg, pair_seg, pair_fb, pair_split};
+          act = {fb, seg, pair_seg, pair_fb};
           rebuild = true;
           dirty = false;
         }

@@ -4,7 +4,7 @@
 #include <mutex>
 #include <tuple>
 
-#include "sweep_dev.h"
+#include "pair_dev.h"
 
 namespace le2d {
 
@@ -116,37 +116,31 @@ __global__ __launch_bounds__(FB, 3) void k_step_xy(const T *__restrict__ src, T 
   march_tile_alt<T, EDGE, FB>(src, dst, nx, ny, pitch, plane, strip, j0, j1, segi, cx, cy, sw, sf);
 }
 
-// Two fused steps over one grid (march_pair in sweep_dev.h).  Occupancy 2:
-// the two stages hold twice the march state of k_step_xy.
+// Two steps over one grid (pair_tile in pair_dev.h) in windows of FB columns,
+// FB/64 per lane ...
 template <typename T, int FB>
-__global__ __launch_bounds__(FB, 2) void k_step2_xy(const T *__restrict__ src, T *__restrict__ dst,
-                                                 int nx, int ny, long pitch, long plane, int seg,
-                                                 int nstrips, SweepCoef<T> cx, SweepCoef<T> cy) {
-  __shared__ W4<T> sw[pair_lds<FB>()];
-  __shared__ W4<T> sf[pair_lds<FB>()];
+__global__ __launch_bounds__(128, (pair_waves<T, FB / 64>())) void k_step2_xy(const T *__restrict__ src, T *__restrict__ dst,
+                                                  int nx, int ny, long pitch, long plane, int seg,
+                                                  int nstrips, SweepCoef<T> cx, SweepCoef<T> cy) {
+  __shared__ PairLds<T, FB / 64> lds;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int strip = tile % nstrips, segi = tile / nstrips;
   const int j0 = segi * seg;
   const int j1 = min(j0 + seg, ny);
-  march_pair<T, FB>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, sw, sf);
+  pair_tile<T, FB / 64>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds);
 }
 
-// Two fused steps, the stages on two wavefronts (march_pair_split): 128
-// lanes per workgroup, each wavefront one 64-lane window of one stage; three
-// workgroups' waves per SIMD (four spill in FP64).  HOLD: FP32 keeps each
-// slot's y-invariants in registers.
+// ... and in windows of 64 columns, one per lane.
 template <typename T, bool HOLD>
-__global__ __launch_bounds__(128, 3) void k_step2_split(
+__global__ __launch_bounds__(128, (pair_waves<T, 1>())) void k_step2_split(
     const T *__restrict__ src, T *__restrict__ dst, int nx, int ny, long pitch, long plane,
     int seg, int nstrips, SweepCoef<T> cx, SweepCoef<T> cy) {
-  __shared__ W4<T> sw[128];
-  __shared__ W4<T> sf[128];
-  __shared__ T ring[2 * kSplitRows * 5 * 64];
+  __shared__ PairLds<T, 1> lds;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int strip = tile % nstrips, segi = tile / nstrips;
   const int j0 = segi * seg;
   const int j1 = min(j0 + seg, ny);
-  march_pair_split<T, HOLD>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, sw, sf, ring);
+  pair_tile<T, 1>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -186,23 +180,16 @@ int step_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy, int edge
   return OK;
 }
 
-template <typename T, int FB>
-static int launch_step2_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy, int seg) {
-  const int nstrips = (g->nx + FB - 9) / (FB - 8);
-  const long nsegs = (g->ny + seg - 1) / seg;
-  const long nblocks = nsegs * nstrips;
-  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "step2_xy: grid too large");
-  const T *src = static_cast<const T *>(g->buf[g->cur]);
-  T *dst = static_cast<T *>(g->buf[g->cur ^ 1]);
-  if (FB == 64 && g->tiles.pair_split)
-    hipLaunchKernelGGL((k_step2_split<T, sizeof(T) == 4>),
-                       dim3((unsigned)nblocks), dim3(128), 0,
-                       g->stream, src, dst, g->nx, g->ny, g->pitch, g->plane, seg, nstrips, cx,
-                       cy);
-  else
-    hipLaunchKernelGGL((k_step2_xy<T, FB>), dim3((unsigned)nblocks), dim3(FB), 0, g->stream, src,
-                       dst, g->nx, g->ny, g->pitch, g->plane, seg, nstrips, cx, cy);
-  return OK;
+// The two-step kernel of a window of `cols` columns (pair_cols).
+template <typename T>
+using PairKernel = void (*)(const T *, T *, int, int, long, long, int, int, SweepCoef<T>,
+                            SweepCoef<T>);
+template <typename T>
+static PairKernel<T> pair_kernel(int cols) {
+  if (cols == 64) return k_step2_split<T, sizeof(T) == 4>;
+  if constexpr (sizeof(T) == 4)
+    if (cols == 256) return k_step2_xy<T, 256>;
+  return k_step2_xy<T, 128>;
 }
 
 template <typename T>
@@ -210,57 +197,56 @@ int step2_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy) {
   if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "step2_xy: element size mismatch");
   const int seg = g->tiles.pair_seg;
   if (seg < 1) return set_error(ERR_ARG, "step2_xy: no pair segment height");
-  const int fb = g->tiles.pair_block;
-  const int rc = fb == 64    ? launch_step2_xy<T, 64>(g, cx, cy, seg)
-                 : fb == 128 ? launch_step2_xy<T, 128>(g, cx, cy, seg)
-                             : launch_step2_xy<T, 256>(g, cx, cy, seg);
-  if (rc) return rc;
+  const int cols = pair_cols(g->elem, g->tiles.pair_block);
+  const int nstrips = (g->nx + cols - 9) / (cols - 8);
+  const long nsegs = (g->ny + seg - 1) / seg;
+  const long nblocks = nsegs * nstrips;
+  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "step2_xy: grid too large");
+  hipLaunchKernelGGL(pair_kernel<T>(cols), dim3((unsigned)nblocks), dim3(128), 0, g->stream,
+                     static_cast<const T *>(g->buf[g->cur]), static_cast<T *>(g->buf[g->cur ^ 1]),
+                     g->nx, g->ny, g->pitch, g->plane, seg, nstrips, cx, cy);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(ERR_DEVICE, "step2_xy launch: %s", hipGetErrorString(e));
   g->cur ^= 1;
   return OK;
 }
 
-template <typename T, int FB, bool PAIR>
-static int occupancy_of() {
+template <typename K>
+static int occupancy_of(K kernel, int lanes) {
   int n = 0;
-  hipError_t e;
-  if constexpr (PAIR)
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_step2_xy<T, FB>, FB, 0);
-  else
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_step_xy<T, EDGE_CLAMP, FB>, FB, 0);
-  return e == hipSuccess ? n : 0;
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, lanes, 0) == hipSuccess ? n : 0;
+}
+
+template <typename T>
+static int occupancy(bool pair, int cols) {
+  if (pair) return min(4, occupancy_of(pair_kernel<T>(cols), 128));
+  return cols == 64    ? occupancy_of(k_step_xy<T, EDGE_CLAMP, 64>, 64)
+         : cols == 128 ? occupancy_of(k_step_xy<T, EDGE_CLAMP, 128>, 128)
+                       : occupancy_of(k_step_xy<T, EDGE_CLAMP, 256>, 256);
 }
 
 // Workgroups per CU x CUs of the current device, cached per device.
-template <bool PAIR>
-static long resident_of(int elem, int fb) {
+static long resident_of(bool pair, int elem, int cols) {
   static std::mutex mu;
-  static std::map<std::tuple<int, int, int>, long> cache;
+  static std::map<std::tuple<int, bool, int, int>, long> cache;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return 0;
   std::lock_guard<std::mutex> lk(mu);
-  const auto key = std::make_tuple(dev, elem, fb);
+  const auto key = std::make_tuple(dev, pair, elem, cols);
   auto it = cache.find(key);
   if (it != cache.end()) return it->second;
-  int per = 0;
-  if (elem == 8)
-    per = fb == 64    ? occupancy_of<double, 64, PAIR>()
-          : fb == 128 ? occupancy_of<double, 128, PAIR>()
-                      : occupancy_of<double, 256, PAIR>();
-  else
-    per = fb == 64    ? occupancy_of<float, 64, PAIR>()
-          : fb == 128 ? occupancy_of<float, 128, PAIR>()
-                      : occupancy_of<float, 256, PAIR>();
+  const int per = elem == 8 ? occupancy<double>(pair, cols) : occupancy<float>(pair, cols);
   const long r = (long)per * cus;
   cache[key] = r;
   return r;
 }
 
-long pair_resident(int elem, int fb) { return resident_of<true>(elem, fb); }
-long step_resident(int elem, int fb) { return resident_of<false>(elem, fb); }
+long pair_resident(int elem, int window) {
+  return resident_of(true, elem, pair_cols(elem, window));
+}
+long step_resident(int elem, int fb) { return resident_of(false, elem, fb); }
 
 template int step2_xy<double>(DevGrid *, const SweepCoef<double> &, const SweepCoef<double> &);
 template int step2_xy<float>(DevGrid *, const SweepCoef<float> &, const SweepCoef<float> &);

@@ -159,17 +159,25 @@ __device__ __forceinline__ W4<T> invariants(T vn, T sn, T vt, T sxy, const Sweep
   return w;
 }
 
-// Faces of the four invariants between positions p and p+1, given the
-// invariants at p-1, p, p+1, p+2.
+// Faces of the four invariants between positions p and p+1: the upwind and
+// the two adjoining values of each (+c1 and +c2: upwind is the left side; -c1
+// and -c2: the right side).
+template <typename T>
+__device__ __forceinline__ W4<T> faces4(T am, T bm, T cm, T dm, const W4<T> &w0, const W4<T> &w1,
+                                        const SweepCoef<T> &c) {
+  W4<T> f;
+  f.a = face_flux(am, w0.a, w1.a, c.hk1);
+  f.b = face_flux(bm, w1.b, w0.b, c.hk1);
+  f.c = face_flux(cm, w0.c, w1.c, c.hk2);
+  f.d = face_flux(dm, w1.d, w0.d, c.hk2);
+  return f;
+}
+
+// The same, given the invariants at p-1, p, p+1, p+2.
 template <typename T>
 __device__ __forceinline__ W4<T> faces(const W4<T> &wm, const W4<T> &w0, const W4<T> &w1,
                                        const W4<T> &w2, const SweepCoef<T> &c) {
-  W4<T> f;
-  f.a = face_flux(wm.a, w0.a, w1.a, c.hk1);  // +c1: upwind is the left side
-  f.b = face_flux(w2.b, w1.b, w0.b, c.hk1);  // -c1: upwind is the right side
-  f.c = face_flux(wm.c, w0.c, w1.c, c.hk2);
-  f.d = face_flux(w2.d, w1.d, w0.d, c.hk2);
-  return f;
+  return faces4(wm.a, w2.b, wm.c, w2.d, w0, w1, c);
 }
 
 // Back-transform of the increments (simple/le_core.c:221-249).  vn/sn are
@@ -475,413 +483,6 @@ __device__ __forceinline__ void march_tile_alt(const T *__restrict__ src, T *__r
 }
 
 // ---------------------------------------------------------------------------
-// Two full steps per pass.
-//
-// A workgroup of FB lanes holds columns x0-4 .. x0+FB-5 and writes the FB-8
-// columns x0 .. x0+FB-9 of rows [j0, j1) at time n+2.  Stage 1 is the fused
-// step of time n (x-sweep of each raw row, register y-march) and emits the
-// time-(n+1) rows j0-2 .. j1+1; stage 2 x-sweeps each of them as it appears
-// and runs a second y-march that emits the time-(n+2) rows.  Raw rows
-// j0-4 .. j1+5 are read once (clamped at the grid edges, as the reference
-// clamps), so a pass moves 5 reads + 5 writes per node for two steps.
-//
-// Edges.  Each x-sweep reads its neighbour lanes through indices clamped
-// into the lanes that hold grid columns, so both stages see the reference's
-// column clamp whatever lanes outside the grid hold.  Stage-2 positions above
-// row 0 or below row ny-1 take that edge row's stage-2 value (the reference's
-// row clamp of the time-(n+1) state).  The operands and operations of every
-// update are those of two single steps, so the result is bit-identical.
-// sw and sf hold pair_lds<FB>() entries each (see there).
-
-// Lane t+1's value on lane t (lane 63 receives 0): a wavefront shift of the
-// data-parallel primitives (DPP wave_shl:1), no LDS round trip.
-__device__ __forceinline__ int lane_next(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true);
-}
-__device__ __forceinline__ float lane_next(float v) {
-  return __builtin_bit_cast(float, lane_next(__builtin_bit_cast(int, v)));
-}
-__device__ __forceinline__ double lane_next(double v) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)lane_next((int)(unsigned)b);
-  const unsigned hi = (unsigned)lane_next((int)(unsigned)(b >> 32));
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-template <typename T>
-__device__ __forceinline__ W4<T> lane_next(const W4<T> &v) {
-  W4<T> r;
-  r.a = lane_next(v.a);
-  r.b = lane_next(v.b);
-  r.c = lane_next(v.c);
-  r.d = lane_next(v.d);
-  return r;
-}
-// Lane t-1's value on lane t (lane 0 receives 0): DPP wave_shr:1.
-__device__ __forceinline__ float lane_prev(float v) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
-}
-
-// FP32 one-wavefront x-sweep faces with shared slopes.  The limiter's
-// numerator (u0 - um) + eps of a face is, operand for operand, the
-// denominator du + eps of the face upwind of it: the face on the left for
-// the invariants moving to +x (a, c), the face on the right for those moving
-// to -x (b, d).  Lane t forms its face's du and du + eps once from lanes nb.y
-// and nb.z (du = w1 - w0 for a, c and w0 - w1 for b, d), and takes the
-// numerators from lanes t-1 and t+1 by lane shifts: two subtractions per
-// face and invariant instead of four, the same operations on the same
-// operands.  Lanes 0 and 63 receive shifted zeros; no output reads their
-// faces.
-__device__ __forceinline__ W4<float> faces_shared(const W4<float> &w0, const W4<float> &w1,
-                                                  const SweepCoef<float> &c) {
-  const float eps = 1e-6f;
-  const float da = w1.a - w0.a, db = w0.b - w1.b, dc = w1.c - w0.c, dd = w0.d - w1.d;
-  const float sa = da + eps, sb = db + eps, sc = dc + eps, sd = dd + eps;
-  W4<float> f;
-  f.a = __builtin_fmaf(limiter(slope_ratio(lane_prev(sa), sa)) * c.hk1, da, w0.a);
-  f.b = __builtin_fmaf(limiter(slope_ratio(lane_next(sb), sb)) * c.hk1, db, w1.b);
-  f.c = __builtin_fmaf(limiter(slope_ratio(lane_prev(sc), sc)) * c.hk2, dc, w0.c);
-  f.d = __builtin_fmaf(limiter(slope_ratio(lane_next(sd), sd)) * c.hk2, dd, w1.d);
-  return f;
-}
-
-// x-sweep of one window row with clamped neighbour lanes: the face between
-// lanes t-1 and t reads lanes nb = (t-2, t-1, t, t+1), each clamped into the
-// lanes holding grid columns.  Meaningful on lanes 2..FB-3.
-// FP32: every lane forms a face and applies (lanes outside 2..FB-3 produce
-// values no output reads; their LDS indices stay in the window), so the
-// x-sweep has no divergent branch (1.9% faster two-step pass).  FP64 keeps
-// the branches: without them the one-wave pass spills.
-template <typename T, int FB>
-__device__ __forceinline__ Node<T> window_xsweep_cl(Node<T> u, W4<T> *sw, W4<T> *sf, int t,
-                                                    const int4 &nb, const SweepCoef<T> &c) {
-  const W4<T> w = invariants(u.vx, u.sxx, u.vy, u.sxy, c);
-  sw[t] = w;
-  window_sync<FB>();
-  if constexpr (FB == 64) {
-    // One-wavefront window: lane t+1's face reaches lane t by a lane shift
-    // (one LDS round trip fewer; FP64 8192^2 two-step pass 1.5% faster,
-    // 2048^2 3-6%).  FP64 forms faces on lanes 2..FB-2 only (branch-free it
-    // spills); the others shift zeros that no apply reads.
-    if constexpr (sizeof(T) == 4) {
-      const W4<T> f = faces_shared(sw[nb.y], sw[nb.z], c);
-      apply(u.vx, u.vy, u.sxx, u.syy, u.sxy, w, f, lane_next(f), c);
-    } else {
-      W4<T> f = {T(0), T(0), T(0), T(0)};
-      if (t >= 2 && t <= FB - 2) f = faces(sw[nb.x], sw[nb.y], sw[nb.z], sw[nb.w], c);
-      const W4<T> fr = lane_next(f);
-      if (t >= 2 && t <= FB - 3) apply(u.vx, u.vy, u.sxx, u.syy, u.sxy, w, f, fr, c);
-    }
-    // the next x-sweep of this window rewrites sw only after every lane read it
-    window_sync<FB>();
-  } else if constexpr (sizeof(T) == 4) {
-    sf[t] = faces(sw[nb.x], sw[nb.y], sw[nb.z], sw[nb.w], c);
-    window_sync<FB>();
-    apply(u.vx, u.vy, u.sxx, u.syy, u.sxy, w, sf[t], sf[min(t + 1, FB - 1)], c);
-  } else {
-    if (t >= 2 && t <= FB - 2) sf[t] = faces(sw[nb.x], sw[nb.y], sw[nb.z], sw[nb.w], c);
-    window_sync<FB>();
-    if (t >= 2 && t <= FB - 3) apply(u.vx, u.vy, u.sxx, u.syy, u.sxy, w, sf[t], sf[t + 1], c);
-  }
-  return u;
-}
-
-// LDS entries (W4) of each of march_pair's two arrays: a one-wavefront window
-// gives the stage-2 x-sweeps their own half (no barrier orders the two
-// exchanges of a step, so separate arrays let them overlap); wider windows,
-// whose barriers serialise the exchanges anyway, share one (measured 2.8%
-// faster for 256 lanes in FP64).
-template <int FB>
-constexpr int pair_lds() { return FB <= 64 ? 2 * FB : FB; }
-
-template <typename T, int FB>
-__device__ __forceinline__ void march_pair(const T *__restrict__ src, T *__restrict__ dst, int nx,
-                                           int ny, long pitch, long plane, int strip, int j0,
-                                           int j1, const SweepCoef<T> &cx,
-                                           const SweepCoef<T> &cy, W4<T> *sw, W4<T> *sf) {
-  const int t = threadIdx.x;
-  const int x0 = strip * (FB - 8);
-  const int x = x0 - 4 + t;
-  const unsigned boff = (unsigned)min(max(x, 0), nx - 1) * (unsigned)sizeof(T);
-  const unsigned woff = (unsigned)max(x, 0) * (unsigned)sizeof(T);
-  const bool writer = t >= 4 && t <= FB - 5 && x < nx;
-  // lanes of grid column 0 and nx-1 (clamped into the window)
-  const int tlo = max(0, 4 - x0), thi = min(FB - 1, nx + 3 - x0);
-  const int4 nb = make_int4(min(max(t - 2, tlo), thi), min(max(t - 1, tlo), thi),
-                            min(max(t, tlo), thi), min(max(t + 1, tlo), thi));
-  constexpr int PAIR_LDS2 = pair_lds<FB>() / FB - 1;  // 1: stage 2 has its own half
-#define ROW(p) load_row_node(src + (long)ypos<EDGE_CLAMP>((p), ny) * pitch, plane, boff)
-#define XS(n) window_xsweep_cl<T, FB>((n), sw, sf, t, nb, cx)
-#define XS2(n) window_xsweep_cl<T, FB>((n), sw + PAIR_LDS2 * FB, sf + PAIR_LDS2 * FB, t, nb, cx)
-  // Stage 1: slots A/B/C hold the x-swept time-n rows q, q+1, q+2, F0/F1 the
-  // faces, wb the invariants of row q-1, N0/N1 the raw rows in flight (as in
-  // march_tile).  Stage 2: slots A2/B2/C2 hold the x-swept time-(n+1) rows
-  // r, r+1, r+2 (r = q-2), G0/G1 its faces, vb the invariants of row r-1.
-  // HOLD (FP32, which has the registers): the y-invariants of every slot are
-  // kept (WA.., VA..) instead of re-formed each step.
-  constexpr bool HOLD = sizeof(T) == 4;
-  Node<T> A, B, C, N0, N1, A2, B2, C2, Xm2, Xm1;
-  W4<T> F0, F1, wb, G0, G1, vb, WA, WB, WC, VA, VB, VC;
-  int q = j0 - 2;
-  {
-    const W4<T> w2 = inv_y(XS(ROW(q - 2)), cy);
-    wb = inv_y(XS(ROW(q - 1)), cy);
-    A = XS(ROW(q));
-    B = XS(ROW(q + 1));
-    C = XS(ROW(q + 2));
-    N0 = ROW(q + 3);
-    WA = inv_y(A, cy);
-    WB = inv_y(B, cy);
-    if constexpr (HOLD) WC = inv_y(C, cy);
-    F0 = faces(w2, wb, WA, WB, cy);  // face q-1 | q
-  }
-  // Stage-1 step: time-(n+1) row q (in P0), its x-sweep into X, then the next
-  // raw row x-swept into P0.
-#define S1(P0, P1, P2, W0, W1, W2, FI, FO, NC, NN, X)                        \
-  {                                                                           \
-    NN = ROW(q + 4);                                                          \
-    const W4<T> w0 = HOLD ? W0 : inv_y(P0, cy);                               \
-    FO = faces(wb, w0, HOLD ? W1 : inv_y(P1, cy), HOLD ? W2 : inv_y(P2, cy), cy); \
-    apply(P0.vy, P0.vx, P0.syy, P0.sxx, P0.sxy, w0, FI, FO, cy);              \
-    wb.a = w0.a;                                                              \
-    wb.c = w0.c;                                                              \
-    X = XS2(P0);                                                              \
-    P0 = XS(NC);                                                              \
-    if constexpr (HOLD) W0 = inv_y(P0, cy);                                   \
-    ++q;                                                                      \
-  }
-  S1(A, B, C, WA, WB, WC, F0, F1, N0, N1, Xm2)  // q = j0-2
-  S1(B, C, A, WB, WC, WA, F1, F0, N1, N0, Xm1)  // q = j0-1
-  S1(C, A, B, WC, WA, WB, F0, F1, N0, N1, A2)   // q = j0
-  S1(A, B, C, WA, WB, WC, F1, F0, N1, N0, B2)   // q = j0+1
-  if (j0 + 1 >= ny) B2 = A2;                    // row clamp of the time-(n+1) state
-  if (j0 - 1 < 0) Xm1 = A2;
-  if (j0 - 2 < 0) Xm2 = Xm1;
-  vb = inv_y(Xm1, cy);
-  VA = inv_y(A2, cy);
-  VB = inv_y(B2, cy);
-  G0 = faces(inv_y(Xm2, cy), vb, VA, VB, cy);  // face j0-1 | j0
-  int r = j0;
-  // One stage-1 step (row q = r+2 of time n+1 into Q2, clamped past the last
-  // row), then one stage-2 step writing row r of time n+2.
-#define S2(P0, P1, P2, W0, W1, W2, FI, FO, NC, NN, Q0, Q1, Q2, V0, V1, V2, GI, GO) \
-  {                                                                           \
-    NN = ROW(q + 4);                                                          \
-    const W4<T> w0 = HOLD ? W0 : inv_y(P0, cy);                               \
-    FO = faces(wb, w0, HOLD ? W1 : inv_y(P1, cy), HOLD ? W2 : inv_y(P2, cy), cy); \
-    apply(P0.vy, P0.vx, P0.syy, P0.sxx, P0.sxy, w0, FI, FO, cy);              \
-    wb.a = w0.a;                                                              \
-    wb.c = w0.c;                                                              \
-    {                                                                         \
-      const Node<T> xn = XS2(P0);                                             \
-      if (q >= ny) {                                                          \
-        Q2 = Q1;                                                              \
-        if constexpr (HOLD) V2 = V1;                                          \
-      } else {                                                                \
-        Q2 = xn;                                                              \
-        if constexpr (HOLD) V2 = inv_y(Q2, cy);                               \
-      }                                                                       \
-    }                                                                         \
-    P0 = XS(NC);                                                              \
-    if constexpr (HOLD) W0 = inv_y(P0, cy);                                   \
-    ++q;                                                                      \
-    const W4<T> v0 = HOLD ? V0 : inv_y(Q0, cy);                               \
-    GO = faces(vb, v0, HOLD ? V1 : inv_y(Q1, cy), HOLD ? V2 : inv_y(Q2, cy), cy); \
-    apply(Q0.vy, Q0.vx, Q0.syy, Q0.sxx, Q0.sxy, v0, GI, GO, cy);              \
-    if (writer) store_row_node(dst + (long)r * pitch, plane, woff, Q0);      \
-    if (++r >= j1) break;                                                     \
-    vb.a = v0.a;                                                              \
-    vb.c = v0.c;                                                              \
-  }
-  // stage 1 continues at phase 4 of its six-step slot cycle, stage 2 at 0
-  for (;;) {
-    S2(B, C, A, WB, WC, WA, F0, F1, N0, N1, A2, B2, C2, VA, VB, VC, G0, G1)
-    S2(C, A, B, WC, WA, WB, F1, F0, N1, N0, B2, C2, A2, VB, VC, VA, G1, G0)
-    S2(A, B, C, WA, WB, WC, F0, F1, N0, N1, C2, A2, B2, VC, VA, VB, G0, G1)
-    S2(B, C, A, WB, WC, WA, F1, F0, N1, N0, A2, B2, C2, VA, VB, VC, G1, G0)
-    S2(C, A, B, WC, WA, WB, F0, F1, N0, N1, B2, C2, A2, VB, VC, VA, G0, G1)
-    S2(A, B, C, WA, WB, WC, F1, F0, N1, N0, C2, A2, B2, VC, VA, VB, G1, G0)
-  }
-#undef S2
-#undef S1
-#undef XS2
-#undef XS
-#undef ROW
-}
-
-// ---------------------------------------------------------------------------
-// Two full steps per pass with the two stages on two wavefronts.
-//
-// The window, segment, edge rules and operations of march_pair with a
-// 64-lane window, but stage 1 (x-sweep of the raw rows, y-march to time
-// n+1) runs on wavefront 0 and stage 2 (x-sweep of the time-(n+1) rows,
-// y-march to time n+2) on wavefront 1 of a 128-lane workgroup.  Each time-
-// (n+1) row passes from the first to the second through an LDS ring of 2*RB
-// slots, one workgroup barrier per RB rows: wavefront 0 writes row k into slot
-// k % (2*RB) and arrives at barrier k / RB after the last row of that group
-// (or the last row of all); wavefront 1 passes barrier b before it reads rows
-// b*RB .. b*RB+RB-1, and passes barrier b+1 only after reading them, while
-// wavefront 0 fills the other half of the ring; so a slot is rewritten only
-// after its row was read.  Both wavefronts pass exactly ceil((j1 - j0 + 4) /
-// RB) barriers (stage-1 rows j0-2 .. j1+1).  Each wavefront holds one stage's
-// march state, about
-// half of march_pair's registers, so more of them are resident per SIMD; each
-// x-sweep's LDS exchange stays within its wavefront (wavefront-scope
-// ordering) in its own half of sw / sf.  The result is march_pair's, bit for
-// bit.  sw and sf hold 128 entries each, ring 2*RB x 5 x 64 values.
-__device__ __forceinline__ void split_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
-template <typename T>
-__device__ __forceinline__ void ring_put(T *slot, int t, const Node<T> &u) {
-  slot[t] = u.vx;
-  slot[64 + t] = u.vy;
-  slot[128 + t] = u.sxx;
-  slot[192 + t] = u.sxy;
-  slot[256 + t] = u.syy;
-}
-
-template <typename T>
-__device__ __forceinline__ Node<T> ring_get(const T *slot, int t) {
-  Node<T> u;
-  u.vx = slot[t];
-  u.vy = slot[64 + t];
-  u.sxx = slot[128 + t];
-  u.sxy = slot[192 + t];
-  u.syy = slot[256 + t];
-  return u;
-}
-
-// Rows per barrier of the ring (RB): 2 and 3 measured no faster than 1.
-constexpr int kSplitRows = 1;
-
-template <typename T, bool HOLD, int RB = kSplitRows>
-__device__ __forceinline__ void march_pair_split(const T *__restrict__ src, T *__restrict__ dst,
-                                                 int nx, int ny, long pitch, long plane,
-                                                 int strip, int j0, int j1,
-                                                 const SweepCoef<T> &cx, const SweepCoef<T> &cy,
-                                                 W4<T> *sw, W4<T> *sf, T *ring) {
-  constexpr int FB = 64;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int t = (int)(threadIdx.x & 63);
-  const int x0 = strip * (FB - 8);
-  const int x = x0 - 4 + t;
-  const int tlo = max(0, 4 - x0), thi = min(FB - 1, nx + 3 - x0);
-  const int4 nb = make_int4(min(max(t - 2, tlo), thi), min(max(t - 1, tlo), thi),
-                            min(max(t, tlo), thi), min(max(t + 1, tlo), thi));
-  const int rows = j1 - j0 + 4;  // stage-1 rows j0-2 .. j1+1
-  constexpr int RS = 2 * RB;     // ring slots
-  sw += FB * wave;
-  sf += FB * wave;
-#define XS(n) window_xsweep_cl<T, FB>((n), sw, sf, t, nb, cx)
-  if (wave == 0) {
-    // Stage 1 (as march_pair's): slots A/B/C hold the x-swept time-n rows
-    // q, q+1, q+2, F0/F1 the faces, wb the invariants of row q-1, N0/N1 the
-    // raw rows in flight; HOLD keeps each slot's y-invariants (WA..).
-    const unsigned boff = (unsigned)min(max(x, 0), nx - 1) * (unsigned)sizeof(T);
-#define ROW(p) load_row_node(src + (long)ypos<EDGE_CLAMP>((p), ny) * pitch, plane, boff)
-    Node<T> A, B, C, N0, N1;
-    W4<T> F0, F1, wb, WA, WB, WC;
-    int q = j0 - 2, k = 0;
-    {
-      const W4<T> w2 = inv_y(XS(ROW(q - 2)), cy);
-      wb = inv_y(XS(ROW(q - 1)), cy);
-      A = XS(ROW(q));
-      B = XS(ROW(q + 1));
-      C = XS(ROW(q + 2));
-      N0 = ROW(q + 3);
-      WA = inv_y(A, cy);
-      WB = inv_y(B, cy);
-      if constexpr (HOLD) WC = inv_y(C, cy);
-      F0 = faces(w2, wb, WA, WB, cy);  // face q-1 | q
-    }
-#define P1(P0, P1, P2, W0, W1, W2, FI, FO, NC, NN)                           \
-  {                                                                           \
-    NN = ROW(q + 4);                                                          \
-    const W4<T> w0 = HOLD ? W0 : inv_y(P0, cy);                               \
-    FO = faces(wb, w0, HOLD ? W1 : inv_y(P1, cy), HOLD ? W2 : inv_y(P2, cy), cy); \
-    apply(P0.vy, P0.vx, P0.syy, P0.sxx, P0.sxy, w0, FI, FO, cy);              \
-    wb.a = w0.a;                                                              \
-    wb.c = w0.c;                                                              \
-    ring_put(ring + (k % RS) * 5 * FB, t, P0);                                \
-    if (k % RB == RB - 1 || k == rows - 1) split_sync();                      \
-    if (++k >= rows) break;                                                   \
-    P0 = XS(NC);                                                              \
-    if constexpr (HOLD) W0 = inv_y(P0, cy);                                   \
-    ++q;                                                                      \
-  }
-    for (;;) {
-      P1(A, B, C, WA, WB, WC, F0, F1, N0, N1)
-      P1(B, C, A, WB, WC, WA, F1, F0, N1, N0)
-      P1(C, A, B, WC, WA, WB, F0, F1, N0, N1)
-      P1(A, B, C, WA, WB, WC, F1, F0, N1, N0)
-      P1(B, C, A, WB, WC, WA, F0, F1, N0, N1)
-      P1(C, A, B, WC, WA, WB, F1, F0, N1, N0)
-    }
-#undef P1
-#undef ROW
-  } else {
-    // Stage 2: slots A2/B2/C2 hold the x-swept time-(n+1) rows r, r+1, r+2,
-    // G0/G1 the faces, vb the invariants of row r-1.  Positions above row 0
-    // or below row ny-1 take that edge row's value (march_pair's clamps).
-    const unsigned woff = (unsigned)max(x, 0) * (unsigned)sizeof(T);
-    const bool writer = t >= 4 && t <= FB - 5 && x < nx;
-    Node<T> A2, B2, C2, Xm2, Xm1;
-    W4<T> G0, G1, vb, VA, VB, VC;
-    int k = 0;
-    // barrier before each group of RB rows, then row k from its slot
-#define GET() (k % RB == 0 ? split_sync() : (void)0, XS(ring_get(ring + ((k++) % RS) * 5 * FB, t)))
-    Xm2 = GET();  // row j0-2
-    Xm1 = GET();  // row j0-1
-    A2 = GET();   // row j0
-    B2 = GET();   // row j0+1
-    if (j0 + 1 >= ny) B2 = A2;
-    if (j0 - 1 < 0) Xm1 = A2;
-    if (j0 - 2 < 0) Xm2 = Xm1;
-    vb = inv_y(Xm1, cy);
-    VA = inv_y(A2, cy);
-    VB = inv_y(B2, cy);
-    G0 = faces(inv_y(Xm2, cy), vb, VA, VB, cy);  // face j0-1 | j0
-    int r = j0, q = j0 + 2;
-#define P2(Q0, Q1, Q2, V0, V1, V2, GI, GO)                                    \
-  {                                                                           \
-    {                                                                         \
-      const Node<T> xn = GET();                                               \
-      if (q >= ny) {                                                          \
-        Q2 = Q1;                                                              \
-        if constexpr (HOLD) V2 = V1;                                          \
-      } else {                                                                \
-        Q2 = xn;                                                              \
-        if constexpr (HOLD) V2 = inv_y(Q2, cy);                               \
-      }                                                                       \
-    }                                                                         \
-    ++q;                                                                      \
-    const W4<T> v0 = HOLD ? V0 : inv_y(Q0, cy);                               \
-    GO = faces(vb, v0, HOLD ? V1 : inv_y(Q1, cy), HOLD ? V2 : inv_y(Q2, cy), cy); \
-    apply(Q0.vy, Q0.vx, Q0.syy, Q0.sxx, Q0.sxy, v0, GI, GO, cy);              \
-    if (writer) store_row_node(dst + (long)r * pitch, plane, woff, Q0);      \
-    if (++r >= j1) break;                                                     \
-    vb.a = v0.a;                                                              \
-    vb.c = v0.c;                                                              \
-  }
-    for (;;) {
-      P2(A2, B2, C2, VA, VB, VC, G0, G1)
-      P2(B2, C2, A2, VB, VC, VA, G1, G0)
-      P2(C2, A2, B2, VC, VA, VB, G0, G1)
-      P2(A2, B2, C2, VA, VB, VC, G1, G0)
-      P2(B2, C2, A2, VB, VC, VA, G0, G1)
-      P2(C2, A2, B2, VC, VA, VB, G1, G0)
-    }
-#undef P2
-#undef GET
-  }
-#undef XS
-}
-
-// ---------------------------------------------------------------------------
 // Heterogeneous media: node-local march for tiles that straddle a material
 // interface.
 //
@@ -956,7 +557,7 @@ __device__ __forceinline__ void march_tile_mixed(const T *__restrict__ src, T *_
 
 // Two full steps of the node-local scheme over a tile that straddles a
 // material interface: the strip geometry, edge rules and stage order of
-// march_pair, with every node's update in its own material (as
+// pair_tile (pair_dev.h), with every node's update in its own material (as
 // march_tile_mixed).  Rows are held in shift registers: few tiles take this
 // path.  sn has FB entries.
 template <typename T, int FB>
