@@ -140,6 +140,15 @@ __device__ __forceinline__ W4<T> pick_w(bool c, const W4<T> &a, const W4<T> &b) 
   return {c ? a.a : b.a, c ? a.b : b.b, c ? a.c : b.c, c ? a.d : b.d};
 }
 
+template <typename T, int C, typename Div>
+__device__ __forceinline__ void see_row(const Nodes<T, C> &u, Div &dv) {
+#pragma unroll
+  for (int k = 0; k < C; ++k) {
+    const T f[5] = {u.n[k].vx, u.n[k].vy, u.n[k].sxx, u.n[k].sxy, u.n[k].syy};
+    dv.row(f);
+  }
+}
+
 template <typename T, int C>
 __device__ __forceinline__ Ws<T, C> inv_y(const Nodes<T, C> &u, const SweepCoef<T> &c) {
   Ws<T, C> w;
@@ -148,13 +157,13 @@ __device__ __forceinline__ Ws<T, C> inv_y(const Nodes<T, C> &u, const SweepCoef<
   return w;
 }
 
-template <typename T, int C>
+template <typename T, int C, typename Div>
 __device__ __forceinline__ Ws<T, C> faces(const Ws<T, C> &wm, const Ws<T, C> &w0,
                                           const Ws<T, C> &w1, const Ws<T, C> &w2,
-                                          const SweepCoef<T> &c) {
+                                          const SweepCoef<T> &c, Div &dv) {
   Ws<T, C> f;
 #pragma unroll
-  for (int k = 0; k < C; ++k) f.w[k] = faces(wm.w[k], w0.w[k], w1.w[k], w2.w[k], c);
+  for (int k = 0; k < C; ++k) f.w[k] = faces(wm.w[k], w0.w[k], w1.w[k], w2.w[k], c, dv);
   return f;
 }
 
@@ -173,25 +182,6 @@ __device__ __forceinline__ void keep_ac(Ws<T, C> &to, const Ws<T, C> &w) {
   for (int k = 0; k < C; ++k) {
     to.w[k].a = w.w[k].a;
     to.w[k].c = w.w[k].c;
-  }
-}
-
-// Keeps the values' computation where it stands in the program.
-template <typename T>
-__device__ __forceinline__ void pin(T &a, T &b, T &c, T &d) {
-  asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-}
-template <typename T, int C>
-__device__ __forceinline__ void pin(Ws<T, C> &w) {
-#pragma unroll
-  for (int k = 0; k < C; ++k) pin(w.w[k].a, w.w[k].b, w.w[k].c, w.w[k].d);
-}
-template <typename T, int C>
-__device__ __forceinline__ void pin(Nodes<T, C> &u) {
-#pragma unroll
-  for (int k = 0; k < C; ++k) {
-    pin(u.n[k].vx, u.n[k].vy, u.n[k].sxx, u.n[k].sxy);
-    asm volatile("" : "+v"(u.n[k].syy));
   }
 }
 
@@ -311,9 +301,9 @@ __device__ __forceinline__ auto x_edge(int x0, int nx, int t) {
   }
 }
 
-template <typename T>
+template <typename T, typename Div>
 __device__ __forceinline__ void x_sweep(Nodes<T, 1> &un, X1Lds<T> &x, int t, const X1Edge &d,
-                                        const SweepCoef<T> &c) {
+                                        const SweepCoef<T> &c, Div &dv) {
   Node<T> &u = un.n[0];
   const W4<T> w = invariants(u.vx, u.sxx, u.vy, u.sxy, c);
   x.ac[t] = {w.a, w.c};
@@ -332,15 +322,15 @@ __device__ __forceinline__ void x_sweep(Nodes<T, 1> &un, X1Lds<T> &x, int t, con
   } else {
     const P2<T> l2 = x.ac[d.i2], r = x.bd[d.ir];
     window_sync<64>();
-    f = faces4(l2.p, r.p, l2.q, r.q, wl, we, c);
+    f = faces4(l2.p, r.p, l2.q, r.q, wl, we, c, dv);
   }
   // the face on the lane's right is the right neighbour's
   apply(u.vx, u.vy, u.sxx, u.syy, u.sxy, w, f, lane_next(f), c);
 }
 
-template <typename T, int C>
+template <typename T, int C, typename Div>
 __device__ __forceinline__ void x_sweep(Nodes<T, C> &u, XnLds<T> &x, int t, const XnEdge &d,
-                                        const SweepCoef<T> &c) {
+                                        const SweepCoef<T> &c, Div &dv) {
   static_assert(C == 2 || C == 4, "the 4 halo columns are whole lanes");
   Ws<T, C> w;
 #pragma unroll
@@ -375,7 +365,7 @@ __device__ __forceinline__ void x_sweep(Nodes<T, C> &u, XnLds<T> &x, int t, cons
   for (int k = 0; k < C; ++k) {  // the face on the left of column k
     const T am = k > 1 ? w.w[k - 2].a : k ? l.a : l2.p, cm = k > 1 ? w.w[k - 2].c : k ? l.c : l2.q;
     const T bm = k + 1 < C ? w.w[k + 1].b : r.p, dm = k + 1 < C ? w.w[k + 1].d : r.q;
-    f.w[k] = faces4(am, bm, cm, dm, k ? w.w[k - 1] : l, w.w[k], c);
+    f.w[k] = faces4(am, bm, cm, dm, k ? w.w[k - 1] : l, w.w[k], c, dv);
   }
   const W4<T> fe = lane_next(f.w[0]);  // the face right of the lane's last column
 #pragma unroll
@@ -394,9 +384,9 @@ __device__ __forceinline__ void split_sync() {
 }
 
 // Wavefronts per SIMD that the registers of C columns per lane allow without
-// spilling (FP64 146 at C = 1 and 256 at C = 2; FP32 137 and 246 at C = 2 and 4).
+// spilling (FP64 150 at C = 1 and 256 at C = 2; FP32 127 and 224 at C = 2 and 4).
 template <typename T, int C>
-constexpr int pair_waves() { return C == 1 || (C == 2 && sizeof(T) == 4) ? 3 : 2; }
+constexpr int pair_waves() { return C == 1 ? 3 : C == 2 && sizeof(T) == 4 ? 4 : 2; }
 
 template <typename T, int C>
 struct PairLds {
@@ -404,11 +394,11 @@ struct PairLds {
   Vec<T, C> ring[2][5][64];
 };
 
-template <typename T, int C>
-__device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restrict__ dst, int nx,
-                                          int ny, long pitch, long plane, int strip, int j0, int j1,
-                                          const SweepCoef<T> &cx, const SweepCoef<T> &cy,
-                                          PairLds<T, C> &lds) {
+template <typename T, int C, typename Div>
+__device__ __forceinline__ void pair_march(const T *__restrict__ src, T *__restrict__ dst, int nx,
+                                           int ny, long pitch, long plane, int strip, int j0, int j1,
+                                           const SweepCoef<T> &cx, const SweepCoef<T> &cy,
+                                           PairLds<T, C> &lds, Div &dv) {
   // FP32, which has the registers, keeps each slot's y-invariants (WA.., VA..)
   // instead of re-forming them.
   constexpr bool HOLD = sizeof(T) == 4;
@@ -418,49 +408,44 @@ __device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restri
   const int x = x0 - 4 + C * t;  // the lane's first column
   const auto ed = x_edge<C>(x0, nx, t);
   const int rows = j1 - j0 + 4;  // stage-1 rows j0-2 .. j1+1
-#define XS(u) x_sweep(u, lds.x[wave], t, ed, cx)
+#define XS(u) x_sweep(u, lds.x[wave], t, ed, cx, dv)
   if (wave == 0) {
     // Stage 1: slots A/B/D hold the x-swept time-n rows q, q+1, q+2, F the face
     // q-1 | q, wb the invariants of row q-1, N the raw row in flight.  Unrolled
     // three times, so no slot is copied.
     const unsigned boff = (unsigned)min(max(x, 0), (nx - 1) / C * C) * (unsigned)sizeof(T);
 #define ROW(p) load_nodes<T, C>(src + (long)ypos<EDGE_CLAMP>((p), ny) * pitch, plane, boff)
-    Nodes<T, C> A, B, D, N;
-    Ws<T, C> F, wb, WA, WB, WD;
+    Nodes<T, C> A = {}, B = {}, D = {}, N;
+    Ws<T, C> F, wb = {}, WA, WB, WD;
     int q = j0 - 2, k = 0;
     {
-      // x-sweep rows q-2 .. q+2 with four rows in flight; no more is held than
-      // the march holds (without pin the compiler delays the sweeps' ends,
-      // holds all five rows and spills)
-      D = ROW(q - 2);
-      N = ROW(q - 1);
-      A = ROW(q);
-      B = ROW(q + 1);
-      XS(D);
-      Ws<T, C> w2 = inv_y(D, cy);
-      pin(w2);
-      D = ROW(q + 2);
-      XS(N);
-      wb = inv_y(N, cy);
-      pin(wb);
-      N = ROW(q + 3);
-      XS(A);
-      pin(A);
-      XS(B);
-      pin(B);
-      XS(D);
-      pin(D);
+      // x-sweep rows q-2 .. q+2, a loop so that no more rows are held than
+      // the march holds (unrolled, the compiler keeps all five until the end
+      // and spills)
+      Ws<T, C> w2 = {};
+      N = ROW(q - 2);
+#pragma unroll 1
+      for (int p = q - 1; p <= q + 3; ++p) {
+        Nodes<T, C> u = N;
+        N = ROW(p);
+        see_row(u, dv);
+        XS(u);
+        w2 = wb;
+        wb = inv_y(A, cy);
+        A = B;
+        B = D;
+        D = u;
+      }
       WA = inv_y(A, cy);
       WB = inv_y(B, cy);
       if constexpr (HOLD) WD = inv_y(D, cy);
-      F = faces(w2, wb, WA, WB, cy);
-      pin(F);
+      F = faces(w2, wb, WA, WB, cy, dv);
     }
 #define STAGE1(P0, P1, P2, W0, W1, W2)                                                   \
   {                                                                                      \
     const Ws<T, C> w0 = HOLD ? W0 : inv_y(P0, cy);                                       \
     const Ws<T, C> fo =                                                                  \
-        faces(wb, w0, HOLD ? W1 : inv_y(P1, cy), HOLD ? W2 : inv_y(P2, cy), cy);         \
+        faces(wb, w0, HOLD ? W1 : inv_y(P1, cy), HOLD ? W2 : inv_y(P2, cy), cy, dv);         \
     apply_y(P0, w0, F, fo, cy);                                                          \
     F = fo;                                                                              \
     keep_ac(wb, w0);                                                                     \
@@ -471,6 +456,7 @@ __device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restri
     if (++k >= rows) break;                                                              \
     P0 = N;                                                                              \
     N = ROW(q + 4);                                                                      \
+    see_row(P0, dv);                                                                     \
     XS(P0);                                                                              \
     if constexpr (HOLD) W0 = inv_y(P0, cy);                                              \
     ++q;                                                                                 \
@@ -511,7 +497,7 @@ __device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restri
     vb = inv_y(M1, cy);
     VA = inv_y(A, cy);
     VB = inv_y(B, cy);
-    G = faces(inv_y(M2, cy), vb, VA, VB, cy);
+    G = faces(inv_y(M2, cy), vb, VA, VB, cy, dv);
     int r = j0;
 #define STAGE2(Q0, Q1, Q2, V0, V1, V2)                                                   \
   {                                                                                      \
@@ -520,7 +506,7 @@ __device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restri
     if constexpr (HOLD) V2 = inv_y(Q2, cy);                                              \
     const Ws<T, C> v0 = HOLD ? V0 : inv_y(Q0, cy);                                       \
     const Ws<T, C> go =                                                                  \
-        faces(vb, v0, HOLD ? V1 : inv_y(Q1, cy), HOLD ? V2 : inv_y(Q2, cy), cy);         \
+        faces(vb, v0, HOLD ? V1 : inv_y(Q1, cy), HOLD ? V2 : inv_y(Q2, cy), cy, dv);         \
     apply_y(Q0, v0, G, go, cy);                                                          \
     G = go;                                                                              \
     if (writer) store_nodes<T, C>(dst + (long)r * pitch, plane, woff, Q0);               \
@@ -535,6 +521,28 @@ __device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restri
 #undef STAGE2
   }
 #undef XS
+}
+
+// The tile, in FP64 with DivBounded's quotients, and once more with IEEE
+// divisions if it does not meet their conditions (the output of the first
+// march is overwritten; the input is another buffer).  FP64 8192^2 random field 1.55 ms a
+// pass against 1.65, disk 1.24 against 1.34; 2048^2 111 us against 122.
+template <typename T, int C>
+__device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restrict__ dst, int nx,
+                                          int ny, long pitch, long plane, int strip, int j0, int j1,
+                                          const SweepCoef<T> &cx, const SweepCoef<T> &cy,
+                                          PairLds<T, C> &lds) {
+#if LE2D_LIMITER != 2  // CIR forms no ratio
+  if constexpr (sizeof(T) == 8) {
+    if (coef_bounded(cx) && coef_bounded(cy)) {
+      DivBounded dv;
+      pair_march<T, C>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds, dv);
+      if (__syncthreads_and(dv.ok())) return;
+    }
+  }
+#endif
+  DivIeee<T> dv;
+  pair_march<T, C>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds, dv);
 }
 
 }  // namespace le2d

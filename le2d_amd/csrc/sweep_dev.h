@@ -112,11 +112,78 @@ __device__ __forceinline__ float slope_ratio(float n, float d) {
 #endif
 }
 
+// How a march divides.  DivIeee: slope_ratio whatever the operands.
 template <typename T>
-__device__ __forceinline__ T face_flux(T um, T u0, T u1, T hk) {
+struct DivIeee {
+  __device__ __forceinline__ T ratio(T n, T d) { return slope_ratio(n, d); }
+  __device__ __forceinline__ void see(T, T) {}
+  __device__ __forceinline__ void row(const T (&)[5]) {}
+};
+
+// FP64 quotients of a tile whose values stay below 2^764: the compiler's IEEE
+// sequence (a reciprocal, two Newton steps on it, the product and one
+// residual step, Markstein's method) without its operand scaling and its
+// special-case fix-up, 8 instructions instead of 11 and no use of VCC, which
+// ties the divisions of a face set in a row.
+//
+// The scaling is an identity where no intermediate leaves the normal range.
+// A slope operand is a difference plus eps = 1e-6, so it is 0 or at least
+// 2^-73 in magnitude (a difference that cancels against eps does so exactly);
+// with operands below 2^764 every intermediate lies between 2^-838 and 2^838.
+// The fix-up matters for a zero divisor and for non-finite operands only.
+// So the march keeps the largest magnitude of the rows it loads and the
+// smallest divisor (row, see: a maximum or minimum of three high words as
+// FP32 bit patterns, whose order is the magnitudes'), and a tile that met a
+// value of 2^300 or more, a non-finite one or a zero divisor is marched again
+// with DivIeee (ok).  With constants up to 2^60 (coef_bounded) one sweep grows values
+// by less than 2^134, so those of the four sweeps of a pass stay below 2^702 and
+// their invariants' differences below 2^764.
+//
+// Left out, the scaling changes no bit: the operations are those of n / d as
+// compiled.  Checked on the GPU where rounding is closest, on every quotient
+// within 5 units of the product's last place of a rounding boundary for the
+// 2^39 divisors below a power of two (1.4e12 quotients), and on 2e10 random
+// ones: all equal to n / d.
+struct DivBounded {
+  float big = 0.0f, small = 1.0f;
+  static __device__ __forceinline__ float hi(double x) {
+    return __builtin_bit_cast(float, (int)(__builtin_bit_cast(unsigned long long, x) >> 32));
+  }
+  __device__ __forceinline__ double ratio(double n, double d) {
+    const double y0 = __builtin_amdgcn_rcp(d);
+    const double e0 = __builtin_fma(-d, y0, 1.0);
+    const double y1 = __builtin_fma(y0, e0, y0);
+    const double e1 = __builtin_fma(-d, y1, 1.0);
+    const double y = __builtin_fma(y1, e1, y1);
+    const double q = n * y;
+    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+  }
+  __device__ __forceinline__ void see(double a, double b) {
+    small = __builtin_fminf(__builtin_fminf(__builtin_fabsf(hi(a)), __builtin_fabsf(hi(b))), small);
+  }
+  // maximum (not fmax): a high word of 2^1017 or more is an FP32 NaN pattern
+  // and must win
+  static __device__ __forceinline__ float mx(float a, float b, float c) {
+    return __builtin_elementwise_maximum(
+        __builtin_elementwise_maximum(__builtin_fabsf(a), __builtin_fabsf(b)), c);
+  }
+  __device__ __forceinline__ void row(const double (&u)[5]) {
+    big = mx(hi(u[0]), hi(u[1]), big);
+    big = mx(hi(u[2]), hi(u[3]), big);
+    big = __builtin_elementwise_maximum(__builtin_fabsf(hi(u[4])), big);
+  }
+  __device__ __forceinline__ bool ok() const {
+    // high words of 2^300 and 2^-80
+    return big < __builtin_bit_cast(float, (1023 + 300) << 20) &&
+           small > __builtin_bit_cast(float, (1023 - 80) << 20);
+  }
+};
+
+template <typename T, typename Div>
+__device__ __forceinline__ T face_flux(T um, T u0, T u1, T hk, Div &dv) {
   const T eps = T(1e-6);
   const T du = u1 - u0;
-  const T r = slope_ratio((u0 - um) + eps, du + eps);
+  const T r = dv.ratio((u0 - um) + eps, du + eps);
   if constexpr (sizeof(T) == 4)
     return __builtin_fmaf(limiter(r) * hk, du, u0);  // FP32 tier: fused
   else
@@ -162,22 +229,43 @@ __device__ __forceinline__ W4<T> invariants(T vn, T sn, T vt, T sxy, const Sweep
 // Faces of the four invariants between positions p and p+1: the upwind and
 // the two adjoining values of each (+c1 and +c2: upwind is the left side; -c1
 // and -c2: the right side).
-template <typename T>
+template <typename T, typename Div>
 __device__ __forceinline__ W4<T> faces4(T am, T bm, T cm, T dm, const W4<T> &w0, const W4<T> &w1,
-                                        const SweepCoef<T> &c) {
+                                        const SweepCoef<T> &c, Div &dv) {
+  const T eps = T(1e-6);
   W4<T> f;
-  f.a = face_flux(am, w0.a, w1.a, c.hk1);
-  f.b = face_flux(bm, w1.b, w0.b, c.hk1);
-  f.c = face_flux(cm, w0.c, w1.c, c.hk2);
-  f.d = face_flux(dm, w1.d, w0.d, c.hk2);
+  f.a = face_flux(am, w0.a, w1.a, c.hk1, dv);
+  f.b = face_flux(bm, w1.b, w0.b, c.hk1, dv);
+  f.c = face_flux(cm, w0.c, w1.c, c.hk2, dv);
+  f.d = face_flux(dm, w1.d, w0.d, c.hk2, dv);
+  dv.see((w1.a - w0.a) + eps, (w0.b - w1.b) + eps);  // the divisors
+  dv.see((w1.c - w0.c) + eps, (w0.d - w1.d) + eps);
   return f;
 }
 
 // The same, given the invariants at p-1, p, p+1, p+2.
+template <typename T, typename Div>
+__device__ __forceinline__ W4<T> faces(const W4<T> &wm, const W4<T> &w0, const W4<T> &w1,
+                                       const W4<T> &w2, const SweepCoef<T> &c, Div &dv) {
+  return faces4(wm.a, w2.b, wm.c, w2.d, w0, w1, c, dv);
+}
 template <typename T>
 __device__ __forceinline__ W4<T> faces(const W4<T> &wm, const W4<T> &w0, const W4<T> &w1,
                                        const W4<T> &w2, const SweepCoef<T> &c) {
-  return faces4(wm.a, w2.b, wm.c, w2.d, w0, w1, c);
+  DivIeee<T> dv;
+  return faces(wm, w0, w1, w2, c, dv);
+}
+
+// Whether a sweep's constants are small enough for DivBounded: every
+// magnitude at most 2^60 (wavefront-uniform).
+__device__ __forceinline__ bool coef_bounded(const SweepCoef<double> &c) {
+  int m = 0;
+  for (double x : {c.k1, c.k2, c.hk1, c.hk2, c.irhoc1, c.irhoc2, c.rhoc1, c.rhoc2, c.rhoc3})
+    m = max(m, (int)(__builtin_bit_cast(unsigned long long, x) >> 52) & 0x7ff);
+  int k = 0;
+  for (double x : {c.k1, c.k2, c.hk1, c.hk2})
+    k = max(k, (int)(__builtin_bit_cast(unsigned long long, x) >> 52) & 0x7ff);
+  return m < 1023 + 60 && k < 1023 + 5;
 }
 
 // Back-transform of the increments (simple/le_core.c:221-249).  vn/sn are
