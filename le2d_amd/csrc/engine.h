@@ -48,6 +48,7 @@ struct Tiles {
   int xy_block; // lanes per fused-step workgroup (64, 128, 256); writes xy_block-4 columns
   int pair_seg; // rows per segment of the two-step pass (0: one step per pass)
   int pair_block; // window of the two-step pass: 64, 128 or 256 columns (pair_cols)
+  int block_rows = 0; // two-step pass in blocks that write this many rows (0: the march)
   int pair_split = 0; // a caller's setting that is kept and reported; every window runs its
                       // two stages on two wavefronts
 };
@@ -141,6 +142,11 @@ struct PairShape {
   int window, seg;
 };
 PairShape pick_pair_shape(int elem, const GridSize *g, size_t n, int only, int cap);
+// The block kernels of the two-step pass (block_dev.h): rows that kind k writes,
+// and the compute units of the current device (0 if unknown).
+constexpr int kBlockKinds = 6;
+int block_rows(int elem, int kind);
+int device_cus();
 // Segment heights at which an nx x ny grid's workgroups fill 1 .. 8 rounds of
 // the resident ones.
 std::vector<int> pair_round_segs(int elem, int nx, int ny, int window);

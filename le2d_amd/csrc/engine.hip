@@ -316,6 +316,13 @@ Tiles default_tiles(int elem, int nx, int ny) {
   const PairShape p = pick_pair_shape(elem, &size, 1, 0, 192);
   t.pair_block = p.window;
   t.pair_seg = p.seg;
+  // blocks where each has a compute unit to itself, of the fewest rows that give
+  // that (block_dev.h has both sides' times)
+  t.block_rows = 0;
+  for (int k = 0; k < kBlockKinds && !t.block_rows; ++k) {
+    const int rows = block_rows(elem, k);
+    if ((long)((nx + 55) / 56) * ((ny + rows - 1) / rows) <= device_cus()) t.block_rows = rows;
+  }
   return t;
 }
 

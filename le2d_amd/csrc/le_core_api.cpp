@@ -55,7 +55,7 @@ std::unordered_map<const real *, TaskState *> g_tasks;
 // tuned two-step segment heights and windows per (element size, nx, ny), for
 // the process
 std::mutex g_pair_mu;
-std::map<std::tuple<int, int, int>, std::pair<int, int>> g_pair_seg;
+std::map<std::tuple<int, int, int>, std::tuple<int, int, int>> g_pair_seg;  // rows, window, block
 
 int env_mode() {
   const char *s = getenv("LE2D_SYNC");
@@ -167,8 +167,9 @@ int tune_pairs(le_task *t, TaskState *s) {
     std::lock_guard<std::mutex> lk(g_pair_mu);
     auto it = g_pair_seg.find(key);
     if (it != g_pair_seg.end()) {
-      s->g.tiles.pair_seg = it->second.first;
-      s->g.tiles.pair_block = it->second.second;
+      s->g.tiles.pair_seg = std::get<0>(it->second);
+      s->g.tiles.pair_block = std::get<1>(it->second);
+      s->g.tiles.block_rows = std::get<2>(it->second);
       s->pairs_fixed = true;
       return LE2D_OK;
     }
@@ -178,10 +179,12 @@ int tune_pairs(le_task *t, TaskState *s) {
   hipEvent_t ev[2];
   for (auto &e : ev) (void)hipEventCreate(&e);
   int rc = LE2D_OK;
-  // mean ms of one pass at (block, seg) after one untimed pass; < 0 on error
-  auto time_one = [&](int block, int seg, int reps) -> float {
+  // mean ms of one pass at (block, seg), or in blocks of `rows` rows, after one
+  // untimed pass; < 0 on error
+  auto time_one = [&](int block, int seg, int rows, int reps) -> float {
     s->g.tiles.pair_seg = seg;
     s->g.tiles.pair_block = block;
+    s->g.tiles.block_rows = rows;
     for (int k = 0; k <= reps && !rc; ++k) {
       if (k == 1) (void)hipEventRecord(ev[0], s->stream);
       rc = le2d::step2_xy<real>(&s->g, cx, cy);
@@ -203,11 +206,11 @@ int tune_pairs(le_task *t, TaskState *s) {
   // warm-up at the default shape, about 25 ms: after host-side work the
   // device clocks are still low and would make the first candidates look slow
   {
-    const int b0 = s->g.tiles.pair_block, s0 = s->g.tiles.pair_seg;
-    const float est = time_one(b0, s0, 1);
+    const int b0 = s->g.tiles.pair_block, s0 = s->g.tiles.pair_seg, r0 = s->g.tiles.block_rows;
+    const float est = time_one(b0, s0, r0, 1);
     if (est > 0) {
       const int reps = std::max(1, std::min(64, (int)(25.0f / est)));
-      (void)time_one(b0, s0, reps);
+      (void)time_one(b0, s0, r0, reps);
     }
   }
   std::vector<Cand> res;
@@ -230,7 +233,7 @@ int tune_pairs(le_task *t, TaskState *s) {
         if (seg >= 16 && seg <= s->g.ny && !std::count(segs.begin(), segs.end(), seg))
           segs.push_back(seg);
     for (int seg : segs) {
-      const float ms = time_one(block, seg, 4);
+      const float ms = time_one(block, seg, 0, 4);
       if (ms < 0) break;
       res.push_back({ms, block, seg});
     }
@@ -240,18 +243,33 @@ int tune_pairs(le_task *t, TaskState *s) {
     std::sort(res.begin(), res.end(), [](const Cand &a, const Cand &b) { return a.ms < b.ms; });
     if (res.size() > 3) res.resize(3);
     for (const Cand &c : res) {
-      const float ms = time_one(c.block, c.seg, 12);
+      const float ms = time_one(c.block, c.seg, 0, 12);
       if (ms < 0) break;
       if (ms < best.ms) best = {ms, c.block, c.seg};
     }
   }
+  // blocks, up to two for each compute unit, against the fastest march
+  int rows = 0;
+  for (int k = 0; k < le2d::kBlockKinds && !rc && best.ms < 1e30f; ++k) {
+    const int r = le2d::block_rows((int)sizeof(real), k);
+    const long n = (long)((s->g.nx + 55) / 56) * ((s->g.ny + r - 1) / r);
+    if (n > 2 * le2d::device_cus()) continue;
+    const float ms = time_one(best.block, best.seg, r, 12);
+    if (ms < 0) break;
+    if (ms < best.ms) {
+      best.ms = ms;
+      rows = r;
+    }
+    if (2 * n < le2d::device_cus()) break;  // taller ones leave more of the device idle
+  }
   for (auto &e : ev) (void)hipEventDestroy(e);
   s->g.tiles.pair_seg = best.seg;
   s->g.tiles.pair_block = best.block;
+  s->g.tiles.block_rows = rows;
   s->pairs_fixed = true;
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(g_pair_mu);
-  g_pair_seg[key] = {best.seg, best.block};
+  g_pair_seg[key] = {best.seg, best.block, rows};
   return LE2D_OK;
 }
 
@@ -693,6 +711,7 @@ int le2d_set_step_pairs(le_task *task, int seg) {
   if (rc) return rc;
   if (seg < 0) return le2d::set_error(LE2D_ERR_ARG, "step pairs: segment %d", seg);
   s->g.tiles.pair_seg = seg;
+  s->g.tiles.block_rows = 0;  // a height is the march's
   s->pairs_fixed = true;
   return LE2D_OK;
 }
@@ -720,6 +739,7 @@ int le2d_set_step_pair_window(le_task *task, int lanes) {
   if (lanes != 64 && lanes != 128 && lanes != 256)
     return le2d::set_error(LE2D_ERR_ARG, "step pairs: window %d", lanes);
   s->g.tiles.pair_block = lanes;
+  s->g.tiles.block_rows = 0;  // a window is the march's
   s->pairs_fixed = true;
   return LE2D_OK;
 }

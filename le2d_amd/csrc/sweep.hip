@@ -4,7 +4,7 @@
 #include <mutex>
 #include <tuple>
 
-#include "pair_dev.h"
+#include "block_dev.h"
 
 namespace le2d {
 
@@ -143,6 +143,19 @@ __global__ __launch_bounds__(128, (pair_waves<T, 1>())) void k_step2_split(
   pair_tile<T, 1>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds);
 }
 
+// Two steps over one grid in blocks of R rows on each of WV wavefronts
+// (block_tile).
+template <typename T, int R, int WV>
+__global__ __launch_bounds__(64 * WV) void k_step2_block(const T *__restrict__ src,
+                                                       T *__restrict__ dst, int nx, int ny,
+                                                       long pitch, long plane, int nstrips,
+                                                       SweepCoef<T> cx, SweepCoef<T> cy) {
+  __shared__ BlockLds<T> lds[WV];
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  block_tile<T, R, WV>(src, dst, nx, ny, pitch, plane, tile % nstrips,
+                       tile / nstrips * (R * WV - 8), cx, cy, lds);
+}
+
 // ---------------------------------------------------------------------------
 // Launchers.
 
@@ -192,9 +205,63 @@ static PairKernel<T> pair_kernel(int cols) {
   return k_step2_xy<T, 128>;
 }
 
+// The block kernels by the rows they write, shortest first.
+template <typename T>
+struct BlockKernel {
+  int rows, wavefronts;
+  void (*kernel)(const T *, T *, int, int, long, long, int, SweepCoef<T>, SweepCoef<T>);
+};
+template <typename T, int R, int WV>
+constexpr BlockKernel<T> block_kernel() {
+  return {R * WV - 8, WV, k_step2_block<T, R, WV>};
+}
+static const BlockKernel<double> kBlocks8[] = {
+    block_kernel<double, 2, 6>(), block_kernel<double, 2, 8>(), block_kernel<double, 3, 8>(),
+    block_kernel<double, 4, 8>(), block_kernel<double, 5, 8>(), block_kernel<double, 6, 8>()};
+static const BlockKernel<float> kBlocks4[] = {
+    block_kernel<float, 2, 6>(), block_kernel<float, 2, 8>(),  block_kernel<float, 3, 8>(),
+    block_kernel<float, 4, 8>(), block_kernel<float, 4, 12>(), block_kernel<float, 6, 12>()};
+static_assert(sizeof kBlocks8 / sizeof *kBlocks8 == kBlockKinds &&
+              sizeof kBlocks4 / sizeof *kBlocks4 == kBlockKinds);
+template <typename T>
+static const BlockKernel<T> *block_kernels() {
+  if constexpr (sizeof(T) == 8) return kBlocks8;
+  else return kBlocks4;
+}
+
+int block_rows(int elem, int kind) {
+  return elem == 8 ? kBlocks8[kind].rows : kBlocks4[kind].rows;
+}
+
+int device_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 0;
+  return cus;
+}
+
+template <typename T>
+static int step2_block(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy) {
+  const int nstrips = (g->nx + 55) / 56;
+  const BlockKernel<T> *b = block_kernels<T>();
+  for (int k = 1; k < kBlockKinds; ++k)
+    if (block_kernels<T>()[k].rows == g->tiles.block_rows) b = block_kernels<T>() + k;
+  const long nblocks = (long)nstrips * ((g->ny + b->rows - 1) / b->rows);
+  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "step2_xy: grid too large");
+  hipLaunchKernelGGL(b->kernel, dim3((unsigned)nblocks), dim3(64 * b->wavefronts), 0, g->stream,
+                     static_cast<const T *>(g->buf[g->cur]), static_cast<T *>(g->buf[g->cur ^ 1]),
+                     g->nx, g->ny, g->pitch, g->plane, nstrips, cx, cy);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_error(ERR_DEVICE, "step2_xy launch: %s", hipGetErrorString(e));
+  g->cur ^= 1;
+  return OK;
+}
+
 template <typename T>
 int step2_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy) {
   if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "step2_xy: element size mismatch");
+  if (g->tiles.block_rows) return step2_block<T>(g, cx, cy);
   const int seg = g->tiles.pair_seg;
   if (seg < 1) return set_error(ERR_ARG, "step2_xy: no pair segment height");
   const int cols = pair_cols(g->elem, g->tiles.pair_block);
@@ -229,10 +296,9 @@ static int occupancy(bool pair, int cols) {
 static long resident_of(bool pair, int elem, int cols) {
   static std::mutex mu;
   static std::map<std::tuple<int, bool, int, int>, long> cache;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
+  int dev = 0;
+  const int cus = device_cus();
+  if (!cus || hipGetDevice(&dev) != hipSuccess) return 0;
   std::lock_guard<std::mutex> lk(mu);
   const auto key = std::make_tuple(dev, pair, elem, cols);
   auto it = cache.find(key);
