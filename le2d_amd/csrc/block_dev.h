@@ -1,6 +1,6 @@
-// block_dev.h -- two full steps per pass on blocks held in registers, for grids
-// that do not fill the device.
+// block_dev.h -- one or two full steps per pass on blocks held in registers.
 //
+// Two steps, for grids that do not fill the device.
 // What bounds a pass of pair_dev.h's march on a small grid is one workgroup's
 // march: every row waits for the row before it, two exchanges and a barrier, and
 // short segments, which put more of the device to work, recompute more halo
@@ -9,7 +9,7 @@
 // sweeps on all of it at once: all loads in flight together, the x-sweeps of a
 // wavefront's rows independent of each other, and two exchanges of boundary
 // rows between neighbouring wavefronts per y-sweep.  It writes the 56 columns
-// and R*WV-8 rows between the halos.  It does not overlap one block's loads with
+// and R*WV-8 rows between the halos (one step: 60 and R*WV-4).  It does not overlap one block's loads with
 // another's arithmetic, so it is taken where every block has a compute unit to
 // itself and the march stays elsewhere.
 //
@@ -18,8 +18,15 @@
 // of blocks) 37 against 34; FP32 250 x 300 4.5 against 6.5, 512^2 7.1 against 9.3, 1031
 // x 517 9.5 against 12.1, 900^2 13.4 against 16.1.
 //
-// The operands and operations of every update are those of two single steps,
-// so the result is bit-identical.
+// One step.  With half the halo the blocks pay on larger grids too: in FP32,
+// where two or more of them share a compute unit and one loads while another computes,
+// they beat the march at every size (1500 x 1001 11.7 us against 14.4, 8192 x 4096
+// 254 against 266, where the copy rate allows 214), in FP64 on small and on large
+// grids (512^2 8.0 us against 10.3, 3000^2 153 against 170, copy rate 115).  Wavefronts
+// come in fours, one per SIMD (3 x 6 rows 12.2 us at 512^2, 3 x 8 8.0).
+//
+// The operands and operations of every update are those of single steps, so the
+// result is bit-identical.
 #pragma once
 
 #include "pair_dev.h"
@@ -47,22 +54,24 @@ __device__ __forceinline__ void pin(Node<T> &n) {
   asm volatile("" : "+v"(n.vx), "+v"(n.vy), "+v"(n.sxx), "+v"(n.sxy), "+v"(n.syy));
 }
 
-template <typename T, int R, int WV, typename Div>
+template <typename T, int STEPS, int EDGE, int R, int WV, typename Div>
 __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__restrict__ dst, int nx,
                                             int ny, long pitch, long plane, int strip, int j0,
                                             const SweepCoef<T> &cx, const SweepCoef<T> &cy,
                                             BlockLds<T> (&lds)[WV], Div &dv) {
-  static_assert(R >= 2 && R * WV > 8, "a wavefront's boundary is two rows");
+  constexpr int H = 2 * STEPS;  // halo columns and rows
+  static_assert(R >= 2 && R * WV > 2 * H, "a wavefront's boundary is two rows");
+  static_assert(STEPS == 1 || EDGE == EDGE_CLAMP, "the ring edge is for one step");
   const int v = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int t = (int)(threadIdx.x & 63);
-  const int x0 = strip * 56, x = x0 - 4 + t;
-  const int jw = j0 - 4 + v * R;  // this wavefront's first row
+  const int x0 = strip * (64 - 2 * H), x = x0 - H + t;
+  const int jw = j0 - H + v * R;  // this wavefront's first row
   const unsigned boff = (unsigned)min(max(x, 0), nx - 1) * (unsigned)sizeof(T);
-  const X1Edge ed = x_edge<1>(x0, nx, t);
+  const X1Edge ed = x_edge<1, H>(x0, nx, t);
   Nodes<T, 1> u[R];
 #pragma unroll
   for (int r = 0; r < R; ++r)
-    u[r] = load_nodes<T, 1>(src + (long)min(max(jw + r, 0), ny - 1) * pitch, plane, boff);
+    u[r] = load_nodes<T, 1>(src + (long)min(ypos<EDGE>(jw + r, ny), ny - 1) * pitch, plane, boff);
 #pragma unroll
   for (int r = 0; r < R; ++r) see_row(u[r], dv);
 #pragma unroll 1
@@ -72,8 +81,9 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
       x_sweep(u[r], lds[v].x, t, ed, cx, dv);
       pin(u[r].n[0]);
     }
-    // rows outside the grid take the edge row's value
-    if (jw < 0 || jw + R > ny) {  // wavefront-uniform
+    // after a step rows outside the grid take the edge row's value (one step's are
+    // loaded so)
+    if (STEPS > 1 && (jw < 0 || jw + R > ny)) {  // wavefront-uniform
 #pragma unroll
       for (int r = R - 2; r >= 0; --r) u[r] = pick_nodes(jw + r < 0, u[r + 1], u[r]);
 #pragma unroll
@@ -94,19 +104,20 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
     const P2<T> above = lds[va].y.last[t], below2 = lds[vb].y.second[t];
     W4<T> e = lds[vb].y.first[t], e2 = {}, wm = {};
     __syncthreads();
-    e = pick_w(jw + R >= ny, w.w[R - 1], e);
-    e2.b = jw + R >= ny - 1 ? e.b : below2.p;
-    e2.d = jw + R >= ny - 1 ? e.d : below2.q;
-    wm.a = jw <= 0 ? w.w[0].a : above.p;
-    wm.c = jw <= 0 ? w.w[0].c : above.q;
+    e = pick_w(STEPS > 1 && jw + R >= ny, w.w[R - 1], e);
+    e2.b = STEPS > 1 && jw + R >= ny - 1 ? e.b : below2.p;
+    e2.d = STEPS > 1 && jw + R >= ny - 1 ? e.d : below2.q;
+    wm.a = STEPS > 1 && jw <= 0 ? w.w[0].a : above.p;
+    wm.c = STEPS > 1 && jw <= 0 ? w.w[0].c : above.q;
     // each wavefront forms the face below its last row, the wavefront below
     // takes it over
     const W4<T> fe = faces(w.w[R - 2], w.w[R - 1], e, e2, cy, dv);
     lds[v].face[t] = fe;
     __syncthreads();
     W4<T> fi = lds[va].face[t];
-    if (s == 0) __syncthreads();  // the next x-sweeps reuse the memory
-    if (jw == 0) fi = faces(w.w[0], w.w[0], w.w[0], w.w[1], cy, dv);  // the grid's first face
+    if (s + 1 < STEPS) __syncthreads();  // the next x-sweeps reuse the memory
+    if (STEPS > 1 && jw == 0)  // the grid's first face
+      fi = faces(w.w[0], w.w[0], w.w[0], w.w[1], cy, dv);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const W4<T> fo = r == R - 1 ? fe
@@ -117,19 +128,19 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
       pin(n);
       fi = fo;
     }
-    if (s) break;
+    if (s + 1 >= STEPS) break;
   }
   const unsigned woff = (unsigned)max(x, 0) * (unsigned)sizeof(T);
-  const bool writer = t >= 4 && t < 60 && x < nx;
+  const bool writer = t >= H && t < 64 - H && x < nx;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int i = v * R + r;  // row of the block
-    if (i >= 4 && i < R * WV - 4 && jw + r < ny && writer)
+    if (i >= H && i < R * WV - H && jw + r < ny && writer)
       store_nodes<T, 1>(dst + (long)(jw + r) * pitch, plane, woff, u[r]);
   }
 }
 
-template <typename T, int R, int WV>
+template <typename T, int STEPS, int EDGE, int R, int WV>
 __device__ __forceinline__ void block_tile(const T *__restrict__ src, T *__restrict__ dst, int nx,
                                            int ny, long pitch, long plane, int strip, int j0,
                                            const SweepCoef<T> &cx, const SweepCoef<T> &cy,
@@ -138,13 +149,13 @@ __device__ __forceinline__ void block_tile(const T *__restrict__ src, T *__restr
   if constexpr (sizeof(T) == 8) {  // as pair_tile
     if (coef_bounded(cx) && coef_bounded(cy)) {
       DivBounded dv;
-      block_march<T, R, WV>(src, dst, nx, ny, pitch, plane, strip, j0, cx, cy, lds, dv);
+      block_march<T, STEPS, EDGE, R, WV>(src, dst, nx, ny, pitch, plane, strip, j0, cx, cy, lds, dv);
       if (__syncthreads_and(dv.ok())) return;
     }
   }
 #endif
   DivIeee<T> dv;
-  block_march<T, R, WV>(src, dst, nx, ny, pitch, plane, strip, j0, cx, cy, lds, dv);
+  block_march<T, STEPS, EDGE, R, WV>(src, dst, nx, ny, pitch, plane, strip, j0, cx, cy, lds, dv);
 }
 
 }  // namespace le2d

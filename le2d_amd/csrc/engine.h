@@ -48,6 +48,7 @@ struct Tiles {
   int xy_block; // lanes per fused-step workgroup (64, 128, 256); writes xy_block-4 columns
   int pair_seg; // rows per segment of the two-step pass (0: one step per pass)
   int pair_block; // window of the two-step pass: 64, 128 or 256 columns (pair_cols)
+  int step_rows = 0;  // fused step in blocks that write this many rows (0: the march of xy_seg)
   int block_rows = 0; // two-step pass in blocks that write this many rows (0: the march)
   int pair_split = 0; // a caller's setting that is kept and reported; every window runs its
                       // two stages on two wavefronts
@@ -131,8 +132,6 @@ inline int pair_cols(int elem, int window) {
 // on the current device: the resident ones (occupancy API x compute units), at
 // most the four per CU that saturate it; 0 if unknown.
 long pair_resident(int elem, int window);
-// The same for the single-step kernel (clamped edges).
-long step_resident(int elem, int fb);
 // Window setting and segment height (at most `cap` rows) of one two-step launch
 // over n grids, from the model in engine.hip; only: that window (0: any).
 struct GridSize {
@@ -142,10 +141,12 @@ struct PairShape {
   int window, seg;
 };
 PairShape pick_pair_shape(int elem, const GridSize *g, size_t n, int only, int cap);
-// The block kernels of the two-step pass (block_dev.h): rows that kind k writes,
-// and the compute units of the current device (0 if unknown).
-constexpr int kBlockKinds = 6;
+// The block kernels of the two-step pass and of the single step (block_dev.h):
+// rows that kind k writes; and the compute units of the current device (0 if
+// unknown).
+constexpr int kBlockKinds = 6, kStepBlockKinds = 4;
 int block_rows(int elem, int kind);
+int step_block_rows(int elem, int kind);
 int device_cus();
 // Segment heights at which an nx x ny grid's workgroups fill 1 .. 8 rounds of
 // the resident ones.

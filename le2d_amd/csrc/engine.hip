@@ -270,7 +270,8 @@ int grid_download(DevGrid *g, void *host, int soa) {
   return check(hipStreamSynchronize(g->stream), "download sync");
 }
 
-static int best_segment(long strips, int ny, long resident, int halo, int cap);
+static int step_blocks(int elem, int nx, int ny);
+static int step_segment(int nx, int ny);
 
 Tiles default_tiles(int elem, int nx, int ny) {
   Tiles t;
@@ -278,29 +279,21 @@ Tiles default_tiles(int elem, int nx, int ny) {
   // FP64 0.895 ms against 1.026 at 4 rows, FP32 0.426 against 0.457
   t.x_rows = 1;
   t.pair_split = 0;
-  {
-    // fused step: 256-lane windows (252 output columns) and ~64 workgroups
-    // per CU in segments of at least 16 rows (measured best on 8192^2: 16-24
-    // rows; short segments keep the halo rows of neighbouring segments in L2).
-    // Grids under 4096 columns take one-wave windows (60 columns, no
-    // barriers between waves): 2048^2 FP64 50.5 against 45.9 Gnode-updates/s,
-    // FP32 144 against 137.
+  t.step_rows = step_blocks(elem, nx, ny);
+  if (t.step_rows == 0) {
+    t.xy_block = 64;
+    t.xy_seg = step_segment(nx, ny);
+  } else {
+    // the tiles of a material plane's single steps: 256-lane windows from 4096
+    // columns on, else one-wave windows, and ~64 workgroups per CU in segments of
+    // at least 16 rows (short segments keep the halo rows of neighbouring segments
+    // in L2), shorter where that leaves the device idle
     t.xy_block = nx >= 4096 ? 256 : 64;
     const long strips = (nx + t.xy_block - 5) / (t.xy_block - 4);
     const long want = (16384 + strips - 1) / strips;
-    long seg = (ny + want - 1) / want;
-    if (seg < 16) seg = 16;
-    if (seg > ny) seg = ny;
-    t.xy_seg = (int)seg;
-    // grids that 16-row segments leave short of one round of resident
-    // workgroups: a step lasts one workgroup's march (4 halo rows, then the
-    // segment), so the occupancy model of the two-step pass picks a shorter
-    // segment (512^2 FP64 16.5 Gnode-updates/s at 2-4 rows against 11.5 at
-    // 16; 1024^2 39.6 at 12 against 33.9)
-    long resident = step_resident(elem, t.xy_block);
-    if (resident <= 0) resident = 768;
-    if (strips * ((ny + 15) / 16) < resident)
-      t.xy_seg = best_segment(strips, ny, resident, 4, 16);
+    t.xy_seg = (int)std::min<long>(std::max<long>(16, (ny + want - 1) / want), ny);
+    if (t.xy_block == 64 && strips * ((ny + 15) / 16) < 12 * device_cus())
+      t.xy_seg = std::min(16, step_segment(nx, ny));
   }
   t.y_block = nx >= 8 * 256 ? 256 : (nx >= 8 * 128 ? 128 : 64);
   // about 512 workgroups (two per CU), each marching at least 32 rows:
@@ -326,21 +319,45 @@ Tiles default_tiles(int elem, int nx, int ny) {
   return t;
 }
 
-// The candidate segment height (2 .. cap rows) that maximises (fill of the
-// last round of `resident` workgroups) x (share of a segment's rows that are
-// output rather than the `halo` re-read rows).
-static int best_segment(long strips, int ny, long resident, int halo, int cap) {
+// Rows of the single step's blocks, 0 for the march.  The lowest blocks of which every
+// one has a compute unit to itself (us, march against block: FP64 96 x 80 6.0
+// against 4.1, 300 x 250 7.5 against 5.5, 512^2 10.3 against 8.0).  Past that FP32
+// stays with blocks of 20 rows (900^2 10.5 against 8.2, 1500 x 1001 14.4 against 11.7, 3000^2
+// 84 against 73) up to grids far outside the last-level cache, where 44 rows re-read
+// fewer halo rows (8192 x 4096 254 against 272 at 20; 3000^2 74.3 against 72.9).  FP64
+// blocks hold the registers of two wavefronts per SIMD and last long, so the march
+// comes first (900^2 18.4 against 20.4, 1500 x 1001 26.0 against 30.9) until blocks of 24
+// rows make several rounds (2048^2 77 both, 3000^2 170 against 153, 8192 x 4096
+// 577 against 565).
+static int step_blocks(int elem, int nx, int ny) {
+  const long strips = (nx + 59) / 60, cus = device_cus();
+  auto blocks = [&](int kind) {
+    const int rows = step_block_rows(elem, kind);
+    return strips * ((ny + rows - 1) / rows);
+  };
+  int kind = 0;
+  while (kind < kStepBlockKinds - 1 && blocks(kind) > cus) ++kind;
+  if (kind < kStepBlockKinds - 1) return step_block_rows(elem, kind);
+  if (blocks(kind) >= (elem == 8 ? 12 : 24) * cus) return step_block_rows(elem, kind);
+  return elem == 8 ? 0 : step_block_rows(elem, kind - 1);
+}
+
+// Segment height of the single step's march in 64-column windows.  A row costs a
+// wavefront about the same again for each wavefront that shares its SIMD, and as
+// much once more for its own latency, so a launch of w wavefronts per SIMD (at most
+// three at once) lasts (rows marched) x (1 + w): FP64 1500 x 1001 26.0 us at 13 rows
+// (w = 2), 28.7 at 16 (2), 29.1 at 11 (3), 30.7 at 8 (4); 512^2 10.3 at 6 (1), 11.7
+// at 4 (2).
+static int step_segment(int nx, int ny) {
+  const long strips = (nx + 59) / 60, simds = std::max(4, 4 * device_cus());
   int best = 2;
-  double best_score = -1;
-  for (int s : {2, 4, 6, 8, 12, 16}) {
-    if (s > cap || (s > ny && s != 2)) break;
-    const long blocks = strips * ((ny + s - 1) / s);
-    const long rounds = (blocks + resident - 1) / resident;
-    const double fill = (double)blocks / (double)(rounds * resident);
-    const double rows = std::min(s, ny);
-    const double score = fill * rows / (rows + halo);
-    if (score > best_score + 1e-9) {
-      best_score = score;
+  long best_cost = 0;
+  for (int s = 2; s <= std::max(2, std::min(ny, 64)); ++s) {
+    const long n = strips * ((ny + s - 1) / s), full = n / (3 * simds);
+    const long last = (n - full * 3 * simds + simds - 1) / simds;
+    const long cost = (s + 5) * (full * 4 + (last ? 1 + last : 0));
+    if (!best_cost || cost < best_cost) {
+      best_cost = cost;
       best = s;
     }
   }

@@ -663,6 +663,7 @@ int le2d_set_tiles(le_task *task, int x_rows, int y_seg, int y_block, int xy_seg
   if (y_block) s->g.tiles.y_block = y_block;
   if (xy_seg) s->g.tiles.xy_seg = xy_seg;
   if (xy_block) s->g.tiles.xy_block = xy_block;
+  if (xy_seg || xy_block) s->g.tiles.step_rows = 0;  // the march of that shape
   return LE2D_OK;
 }
 

@@ -289,15 +289,15 @@ struct XnEdge {
   int tl, th, e;
 };
 
-template <int C>
+template <int C, int HALO = 4>  // HALO: halo columns, 4 for two steps, 2 for one
 __device__ __forceinline__ auto x_edge(int x0, int nx, int t) {
-  const int last = nx + 3 - x0;  // window column of grid column nx-1
+  const int last = nx - 1 + HALO - x0;  // window column of grid column nx-1
   if constexpr (C == 1) {
-    const int lo = x0 == 0 ? 4 : 0, hi = min(63, last);
+    const int lo = x0 == 0 ? HALO : 0, hi = min(63, last);
     return X1Edge{x0 == 0 || last < 63, min(max(t - 2, lo), hi), min(max(t - 1, lo), hi),
                   min(max(t, lo), hi), min(max(t + 1, lo), hi)};
   } else {
-    return XnEdge{x0 == 0 || last < 64 * C, x0 == 0 ? 4 / C : -1, last / C, last % C};
+    return XnEdge{x0 == 0 || last < 64 * C, x0 == 0 ? HALO / C : -1, last / C, last % C};
   }
 }
 
@@ -394,14 +394,80 @@ struct PairLds {
   Vec<T, C> ring[2][5][64];
 };
 
+// FP32, which has the registers, keeps each slot's y-invariants (WA.., VA..)
+// instead of re-forming them.
+template <typename T>
+constexpr bool kHoldInv = sizeof(T) == 4;
+
+// One step on `rows` rows from row q on, each handed to `out` with its count.
+template <typename T, int EDGE, int C, typename XLds, typename XEdge, typename Div, typename Out>
+__device__ __forceinline__ void march_rows(const T *__restrict__ src, int ny, long pitch, long plane,
+                                           unsigned boff, int q, int rows, int t, const XEdge &ed,
+                                           const SweepCoef<T> &cx, const SweepCoef<T> &cy,
+                                           XLds &lds, Div &dv, Out out) {
+  // Slots A/B/D hold the x-swept rows q, q+1, q+2, F the face q-1 | q, wb the
+  // invariants of row q-1, N the raw row in flight.  Unrolled three times, so
+  // no slot is copied.
+  constexpr bool HOLD = kHoldInv<T>;
+#define ROW(p) load_nodes<T, C>(src + (long)ypos<EDGE>((p), ny) * pitch, plane, boff)
+  Nodes<T, C> A = {}, B = {}, D = {}, N;
+  Ws<T, C> F, wb = {}, WA, WB, WD;
+  int k = 0;
+  {
+    // x-sweep rows q-2 .. q+2, a loop so that no more rows are held than
+    // the march holds (unrolled, the compiler keeps all five until the end
+    // and spills)
+    Ws<T, C> w2 = {};
+    N = ROW(q - 2);
+#pragma unroll 1
+    for (int p = q - 1; p <= q + 3; ++p) {
+      Nodes<T, C> u = N;
+      N = ROW(p);
+      see_row(u, dv);
+      x_sweep(u, lds, t, ed, cx, dv);
+      w2 = wb;
+      wb = inv_y(A, cy);
+      A = B;
+      B = D;
+      D = u;
+    }
+    WA = inv_y(A, cy);
+    WB = inv_y(B, cy);
+    if constexpr (HOLD) WD = inv_y(D, cy);
+    F = faces(w2, wb, WA, WB, cy, dv);
+  }
+#define ADVANCE(P0, P1, P2, W0, W1, W2)                                              \
+  {                                                                                  \
+    const Ws<T, C> w0 = HOLD ? W0 : inv_y(P0, cy);                                   \
+    const Ws<T, C> fo =                                                              \
+        faces(wb, w0, HOLD ? W1 : inv_y(P1, cy), HOLD ? W2 : inv_y(P2, cy), cy, dv); \
+    apply_y(P0, w0, F, fo, cy);                                                      \
+    F = fo;                                                                          \
+    keep_ac(wb, w0);                                                                 \
+    out(k, P0);                                                                      \
+    if (++k >= rows) break;                                                          \
+    P0 = N;                                                                          \
+    N = ROW(q + 4);                                                                  \
+    see_row(P0, dv);                                                                 \
+    x_sweep(P0, lds, t, ed, cx, dv);                                                 \
+    if constexpr (HOLD) W0 = inv_y(P0, cy);                                          \
+    ++q;                                                                             \
+  }
+  for (;;) {
+    ADVANCE(A, B, D, WA, WB, WD)
+    ADVANCE(B, D, A, WB, WD, WA)
+    ADVANCE(D, A, B, WD, WA, WB)
+  }
+#undef ADVANCE
+#undef ROW
+}
+
 template <typename T, int C, typename Div>
 __device__ __forceinline__ void pair_march(const T *__restrict__ src, T *__restrict__ dst, int nx,
                                            int ny, long pitch, long plane, int strip, int j0, int j1,
                                            const SweepCoef<T> &cx, const SweepCoef<T> &cy,
                                            PairLds<T, C> &lds, Div &dv) {
-  // FP32, which has the registers, keeps each slot's y-invariants (WA.., VA..)
-  // instead of re-forming them.
-  constexpr bool HOLD = sizeof(T) == 4;
+  constexpr bool HOLD = kHoldInv<T>;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int t = (int)(threadIdx.x & 63);
   const int x0 = strip * (64 * C - 8);
@@ -410,64 +476,15 @@ __device__ __forceinline__ void pair_march(const T *__restrict__ src, T *__restr
   const int rows = j1 - j0 + 4;  // stage-1 rows j0-2 .. j1+1
 #define XS(u) x_sweep(u, lds.x[wave], t, ed, cx, dv)
   if (wave == 0) {
-    // Stage 1: slots A/B/D hold the x-swept time-n rows q, q+1, q+2, F the face
-    // q-1 | q, wb the invariants of row q-1, N the raw row in flight.  Unrolled
-    // three times, so no slot is copied.
     const unsigned boff = (unsigned)min(max(x, 0), (nx - 1) / C * C) * (unsigned)sizeof(T);
-#define ROW(p) load_nodes<T, C>(src + (long)ypos<EDGE_CLAMP>((p), ny) * pitch, plane, boff)
-    Nodes<T, C> A = {}, B = {}, D = {}, N;
-    Ws<T, C> F, wb = {}, WA, WB, WD;
-    int q = j0 - 2, k = 0;
-    {
-      // x-sweep rows q-2 .. q+2, a loop so that no more rows are held than
-      // the march holds (unrolled, the compiler keeps all five until the end
-      // and spills)
-      Ws<T, C> w2 = {};
-      N = ROW(q - 2);
-#pragma unroll 1
-      for (int p = q - 1; p <= q + 3; ++p) {
-        Nodes<T, C> u = N;
-        N = ROW(p);
-        see_row(u, dv);
-        XS(u);
-        w2 = wb;
-        wb = inv_y(A, cy);
-        A = B;
-        B = D;
-        D = u;
-      }
-      WA = inv_y(A, cy);
-      WB = inv_y(B, cy);
-      if constexpr (HOLD) WD = inv_y(D, cy);
-      F = faces(w2, wb, WA, WB, cy, dv);
-    }
-#define STAGE1(P0, P1, P2, W0, W1, W2)                                                   \
-  {                                                                                      \
-    const Ws<T, C> w0 = HOLD ? W0 : inv_y(P0, cy);                                       \
-    const Ws<T, C> fo =                                                                  \
-        faces(wb, w0, HOLD ? W1 : inv_y(P1, cy), HOLD ? W2 : inv_y(P2, cy), cy, dv);         \
-    apply_y(P0, w0, F, fo, cy);                                                          \
-    F = fo;                                                                              \
-    keep_ac(wb, w0);                                                                     \
-    Vec<T, C> out[5];                                                                    \
-    pack(P0, out);                                                                       \
-    _Pragma("unroll") for (int f = 0; f < 5; ++f) lds.ring[k & 1][f][t] = out[f];        \
-    split_sync();                                                                        \
-    if (++k >= rows) break;                                                              \
-    P0 = N;                                                                              \
-    N = ROW(q + 4);                                                                      \
-    see_row(P0, dv);                                                                     \
-    XS(P0);                                                                              \
-    if constexpr (HOLD) W0 = inv_y(P0, cy);                                              \
-    ++q;                                                                                 \
-  }
-    for (;;) {
-      STAGE1(A, B, D, WA, WB, WD)
-      STAGE1(B, D, A, WB, WD, WA)
-      STAGE1(D, A, B, WD, WA, WB)
-    }
-#undef STAGE1
-#undef ROW
+    march_rows<T, EDGE_CLAMP, C>(src, ny, pitch, plane, boff, j0 - 2, rows, t, ed, cx, cy,
+                                 lds.x[0], dv, [&](int k, const Nodes<T, C> &u) {
+                                   Vec<T, C> out[5];
+                                   pack(u, out);
+#pragma unroll
+                                   for (int f = 0; f < 5; ++f) lds.ring[k & 1][f][t] = out[f];
+                                   split_sync();
+                                 });
   } else {
     // Stage 2: slots A/B/D hold the x-swept time-(n+1) rows r, r+1, r+2, G the
     // face r-1 | r, vb the invariants of row r-1.  Positions above row 0 or
@@ -543,6 +560,44 @@ __device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restri
 #endif
   DivIeee<T> dv;
   pair_march<T, C>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds, dv);
+}
+
+// One step on the tile of strip `strip` (60 of 64 columns written) and rows
+// [j0, j1), by one wavefront.  Two columns per lane, which leave half as many wavefronts,
+// are slower on the grids that take this march (1500 x 1001 30.6 us against 26.0).
+template <typename T, int EDGE, typename Div>
+__device__ __forceinline__ void step_march(const T *__restrict__ src, T *__restrict__ dst, int nx,
+                                           int ny, long pitch, long plane, int strip, int j0, int j1,
+                                           const SweepCoef<T> &cx, const SweepCoef<T> &cy,
+                                           X1Lds<T> &lds, Div &dv) {
+  const int t = (int)threadIdx.x;
+  const int x0 = strip * 60, x = x0 - 2 + t;
+  const unsigned boff = (unsigned)min(max(x, 0), nx - 1) * (unsigned)sizeof(T);
+  const unsigned woff = (unsigned)max(x, 0) * (unsigned)sizeof(T);
+  const bool writer = t >= 2 && t < 62 && x < nx;
+  march_rows<T, EDGE, 1>(src, ny, pitch, plane, boff, j0, j1 - j0, t, x_edge<1, 2>(x0, nx, t), cx,
+                         cy, lds, dv, [&](int k, const Nodes<T, 1> &u) {
+                           if (writer)
+                             store_nodes<T, 1>(dst + (long)(j0 + k) * pitch, plane, woff, u);
+                         });
+}
+
+template <typename T, int EDGE>
+__device__ __forceinline__ void step_tile(const T *__restrict__ src, T *__restrict__ dst, int nx,
+                                          int ny, long pitch, long plane, int strip, int j0, int j1,
+                                          const SweepCoef<T> &cx, const SweepCoef<T> &cy,
+                                          X1Lds<T> &lds) {
+#if LE2D_LIMITER != 2
+  if constexpr (sizeof(T) == 8) {  // as pair_tile
+    if (coef_bounded(cx) && coef_bounded(cy)) {
+      DivBounded dv;
+      step_march<T, EDGE>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds, dv);
+      if (__syncthreads_and(dv.ok())) return;
+    }
+  }
+#endif
+  DivIeee<T> dv;
+  step_march<T, EDGE>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds, dv);
 }
 
 }  // namespace le2d

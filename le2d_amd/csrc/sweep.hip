@@ -102,18 +102,38 @@ __global__ __launch_bounds__(256) void k_sweep_y(const T *__restrict__ src, T *_
 }
 
 // ---------------------------------------------------------------------------
-// Fused step over one grid (layout and march: march_tile in sweep_dev.h).
+// One step over one grid, marched in windows of FB columns: 64 by one wavefront
+// that keeps its own state (step_tile in pair_dev.h; FP64 1500 x 1001 26.0 us against
+// 27.9 through march_tile, 2048^2 77 against 82), wider ones, which only a caller
+// asks for, through march_tile in sweep_dev.h.
 template <typename T, int EDGE, int FB>
 __global__ __launch_bounds__(FB, 3) void k_step_xy(const T *__restrict__ src, T *__restrict__ dst,
                                                 int nx, int ny, long pitch, long plane, int seg,
                                                 int nstrips, SweepCoef<T> cx, SweepCoef<T> cy) {
-  __shared__ W4<T> sw[FB];
-  __shared__ W4<T> sf[FB];
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int strip = tile % nstrips, segi = tile / nstrips;
   const int j0 = segi * seg;
   const int j1 = min(j0 + seg, ny);
-  march_tile_alt<T, EDGE, FB>(src, dst, nx, ny, pitch, plane, strip, j0, j1, segi, cx, cy, sw, sf);
+  if constexpr (FB == 64) {
+    __shared__ X1Lds<T> lds;
+    step_tile<T, EDGE>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds);
+  } else {
+    __shared__ W4<T> sw[FB];
+    __shared__ W4<T> sf[FB];
+    march_tile_alt<T, EDGE, FB>(src, dst, nx, ny, pitch, plane, strip, j0, j1, segi, cx, cy, sw,
+                                sf);
+  }
+}
+
+// One step over one grid in blocks of R rows on each of WV wavefronts (block_tile).
+template <typename T, int EDGE, int R, int WV>
+__global__ __launch_bounds__(64 * WV, (R > 6 ? 2 : 1)) void k_step_block(
+    const T *__restrict__ src, T *__restrict__ dst, int nx, int ny, long pitch, long plane,
+    int nstrips, SweepCoef<T> cx, SweepCoef<T> cy) {
+  __shared__ BlockLds<T> lds[WV];
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  block_tile<T, 1, EDGE, R, WV>(src, dst, nx, ny, pitch, plane, tile % nstrips,
+                                tile / nstrips * (R * WV - 4), cx, cy, lds);
 }
 
 // Two steps over one grid (pair_tile in pair_dev.h) in windows of FB columns,
@@ -152,7 +172,7 @@ __global__ __launch_bounds__(64 * WV) void k_step2_block(const T *__restrict__ s
                                                        SweepCoef<T> cx, SweepCoef<T> cy) {
   __shared__ BlockLds<T> lds[WV];
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  block_tile<T, R, WV>(src, dst, nx, ny, pitch, plane, tile % nstrips,
+  block_tile<T, 2, EDGE_CLAMP, R, WV>(src, dst, nx, ny, pitch, plane, tile % nstrips,
                        tile / nstrips * (R * WV - 8), cx, cy, lds);
 }
 
@@ -172,27 +192,6 @@ static void launch_step_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T
                        dst, g->nx, g->ny, g->pitch, g->plane, seg, nstrips, cx, cy);
 }
 
-template <typename T>
-int step_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy, int edge) {
-  if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "step_xy: element size mismatch");
-  const int fb = g->tiles.xy_block == 64 || g->tiles.xy_block == 256 ? g->tiles.xy_block : 128;
-  const int nstrips = (g->nx + fb - 5) / (fb - 4);
-  const int seg = max(1, g->tiles.xy_seg);
-  const long nsegs = (g->ny + seg - 1) / seg;
-  const long nblocks = nsegs * nstrips;
-  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "step_xy: grid too large");
-  if (fb == 64)
-    launch_step_xy<T, 64>(g, cx, cy, edge, seg, (unsigned)nblocks, nstrips);
-  else if (fb == 128)
-    launch_step_xy<T, 128>(g, cx, cy, edge, seg, (unsigned)nblocks, nstrips);
-  else
-    launch_step_xy<T, 256>(g, cx, cy, edge, seg, (unsigned)nblocks, nstrips);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return set_error(ERR_DEVICE, "step_xy launch: %s", hipGetErrorString(e));
-  g->cur ^= 1;
-  return OK;
-}
-
 // The two-step kernel of a window of `cols` columns (pair_cols).
 template <typename T>
 using PairKernel = void (*)(const T *, T *, int, int, long, long, int, int, SweepCoef<T>,
@@ -205,7 +204,7 @@ static PairKernel<T> pair_kernel(int cols) {
   return k_step2_xy<T, 128>;
 }
 
-// The block kernels by the rows they write, shortest first.
+// The block kernels by the rows they write, shortest first: two steps ...
 template <typename T>
 struct BlockKernel {
   int rows, wavefronts;
@@ -229,6 +228,26 @@ static const BlockKernel<T> *block_kernels() {
   else return kBlocks4;
 }
 
+// ... and one, with either edge.
+template <typename T, int R, int WV, int EDGE>
+constexpr BlockKernel<T> step_block_kernel() {
+  return {R * WV - 4, WV, k_step_block<T, EDGE, R, WV>};
+}
+template <typename T, int EDGE>
+static const BlockKernel<T> *step_block_kernels() {
+  constexpr int last_r = sizeof(T) == 8 ? 7 : 4, last_wv = sizeof(T) == 8 ? 4 : 12;
+  static const BlockKernel<T> kernels[] = {
+      step_block_kernel<T, 2, 4, EDGE>(), step_block_kernel<T, 2, 8, EDGE>(),
+      step_block_kernel<T, 3, 8, EDGE>(), step_block_kernel<T, last_r, last_wv, EDGE>()};
+  static_assert(sizeof kernels / sizeof *kernels == kStepBlockKinds);
+  return kernels;
+}
+
+int step_block_rows(int elem, int kind) {
+  return elem == 8 ? step_block_kernels<double, EDGE_CLAMP>()[kind].rows
+                   : step_block_kernels<float, EDGE_CLAMP>()[kind].rows;
+}
+
 int block_rows(int elem, int kind) {
   return elem == 8 ? kBlocks8[kind].rows : kBlocks4[kind].rows;
 }
@@ -241,19 +260,49 @@ int device_cus() {
   return cus;
 }
 
+// Launches the kernel of `kinds` that writes `rows` rows (the first if none does)
+// on the blocks of `width` columns that cover the grid.
 template <typename T>
-static int step2_block(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy) {
-  const int nstrips = (g->nx + 55) / 56;
-  const BlockKernel<T> *b = block_kernels<T>();
-  for (int k = 1; k < kBlockKinds; ++k)
-    if (block_kernels<T>()[k].rows == g->tiles.block_rows) b = block_kernels<T>() + k;
+static int launch_blocks(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy,
+                         const BlockKernel<T> *kinds, int count, int rows, int width,
+                         const char *what) {
+  const BlockKernel<T> *b = kinds;
+  for (int k = 1; k < count; ++k)
+    if (kinds[k].rows == rows) b = kinds + k;
+  const int nstrips = (g->nx + width - 1) / width;
   const long nblocks = (long)nstrips * ((g->ny + b->rows - 1) / b->rows);
-  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "step2_xy: grid too large");
+  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "%s: grid too large", what);
   hipLaunchKernelGGL(b->kernel, dim3((unsigned)nblocks), dim3(64 * b->wavefronts), 0, g->stream,
                      static_cast<const T *>(g->buf[g->cur]), static_cast<T *>(g->buf[g->cur ^ 1]),
                      g->nx, g->ny, g->pitch, g->plane, nstrips, cx, cy);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return set_error(ERR_DEVICE, "step2_xy launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return set_error(ERR_DEVICE, "%s launch: %s", what, hipGetErrorString(e));
+  g->cur ^= 1;
+  return OK;
+}
+
+template <typename T>
+int step_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy, int edge) {
+  if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "step_xy: element size mismatch");
+  if (g->tiles.step_rows)
+    return launch_blocks<T>(g, cx, cy,
+                            edge == EDGE_RING ? step_block_kernels<T, EDGE_RING>()
+                                              : step_block_kernels<T, EDGE_CLAMP>(),
+                            kStepBlockKinds, g->tiles.step_rows, 60, "step_xy");
+  const int fb = g->tiles.xy_block == 64 || g->tiles.xy_block == 256 ? g->tiles.xy_block : 128;
+  const int nstrips = (g->nx + fb - 5) / (fb - 4);
+  const int seg = max(1, g->tiles.xy_seg);
+  const long nsegs = (g->ny + seg - 1) / seg;
+  const long nblocks = nsegs * nstrips;
+  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "step_xy: grid too large");
+  if (fb == 64)
+    launch_step_xy<T, 64>(g, cx, cy, edge, seg, (unsigned)nblocks, nstrips);
+  else if (fb == 128)
+    launch_step_xy<T, 128>(g, cx, cy, edge, seg, (unsigned)nblocks, nstrips);
+  else
+    launch_step_xy<T, 256>(g, cx, cy, edge, seg, (unsigned)nblocks, nstrips);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_error(ERR_DEVICE, "step_xy launch: %s", hipGetErrorString(e));
   g->cur ^= 1;
   return OK;
 }
@@ -261,7 +310,8 @@ static int step2_block(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &c
 template <typename T>
 int step2_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy) {
   if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "step2_xy: element size mismatch");
-  if (g->tiles.block_rows) return step2_block<T>(g, cx, cy);
+  if (g->tiles.block_rows) return launch_blocks<T>(g, cx, cy, block_kernels<T>(), kBlockKinds, g->tiles.block_rows, 56,
+                            "step2_xy");
   const int seg = g->tiles.pair_seg;
   if (seg < 1) return set_error(ERR_ARG, "step2_xy: no pair segment height");
   const int cols = pair_cols(g->elem, g->tiles.pair_block);
@@ -284,35 +334,23 @@ static int occupancy_of(K kernel, int lanes) {
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, lanes, 0) == hipSuccess ? n : 0;
 }
 
-template <typename T>
-static int occupancy(bool pair, int cols) {
-  if (pair) return min(4, occupancy_of(pair_kernel<T>(cols), 128));
-  return cols == 64    ? occupancy_of(k_step_xy<T, EDGE_CLAMP, 64>, 64)
-         : cols == 128 ? occupancy_of(k_step_xy<T, EDGE_CLAMP, 128>, 128)
-                       : occupancy_of(k_step_xy<T, EDGE_CLAMP, 256>, 256);
-}
-
 // Workgroups per CU x CUs of the current device, cached per device.
-static long resident_of(bool pair, int elem, int cols) {
+long pair_resident(int elem, int window) {
   static std::mutex mu;
-  static std::map<std::tuple<int, bool, int, int>, long> cache;
+  static std::map<std::tuple<int, int, int>, long> cache;
   int dev = 0;
-  const int cus = device_cus();
+  const int cus = device_cus(), cols = pair_cols(elem, window);
   if (!cus || hipGetDevice(&dev) != hipSuccess) return 0;
   std::lock_guard<std::mutex> lk(mu);
-  const auto key = std::make_tuple(dev, pair, elem, cols);
+  const auto key = std::make_tuple(dev, elem, cols);
   auto it = cache.find(key);
   if (it != cache.end()) return it->second;
-  const int per = elem == 8 ? occupancy<double>(pair, cols) : occupancy<float>(pair, cols);
-  const long r = (long)per * cus;
+  const int per = elem == 8 ? occupancy_of(pair_kernel<double>(cols), 128)
+                            : occupancy_of(pair_kernel<float>(cols), 128);
+  const long r = (long)min(4, per) * cus;
   cache[key] = r;
   return r;
 }
-
-long pair_resident(int elem, int window) {
-  return resident_of(true, elem, pair_cols(elem, window));
-}
-long step_resident(int elem, int fb) { return resident_of(false, elem, fb); }
 
 template int step2_xy<double>(DevGrid *, const SweepCoef<double> &, const SweepCoef<double> &);
 template int step2_xy<float>(DevGrid *, const SweepCoef<float> &, const SweepCoef<float> &);
