@@ -41,13 +41,14 @@ struct SweepCoef {
 
 // Launch shape of the sweeps (chosen per grid by the autotuner).
 struct Tiles {
-  int x_rows;   // rows per x-sweep workgroup
-  int y_seg;    // rows per y-sweep segment (each segment re-reads 4 halo rows)
+  int x_rows;   // rows per x-sweep workgroup (used where x_fixed, and in FP32 on large grids)
+  int y_seg;    // rows per y-sweep segment (every kYRows of them re-read 4 halo rows)
   int y_block;  // columns per y-sweep workgroup (64, 128 or 256)
   int xy_seg;   // rows per segment of the fused x+y step
   int xy_block; // lanes per fused-step workgroup (64, 128, 256); writes xy_block-4 columns
   int pair_seg; // rows per segment of the two-step pass (0: one step per pass)
   int pair_block; // window of the two-step pass: 64, 128 or 256 columns (pair_cols)
+  bool x_fixed = false;  // x_rows is the caller's
   int step_rows = 0;  // fused step in blocks that write this many rows (0: the march of xy_seg)
   int block_rows = 0; // two-step pass in blocks that write this many rows (0: the march)
   int pair_split = 0; // a caller's setting that is kept and reported; every window runs its

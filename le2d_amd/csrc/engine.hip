@@ -276,7 +276,7 @@ static int step_segment(int nx, int ny);
 Tiles default_tiles(int elem, int nx, int ny) {
   Tiles t;
   // one row per x-sweep workgroup (the most workgroups in flight): 8192^2
-  // FP64 0.895 ms against 1.026 at 4 rows, FP32 0.426 against 0.457
+  // FP32 0.426 ms against 0.457 at 4 rows
   t.x_rows = 1;
   t.pair_split = 0;
   t.step_rows = step_blocks(elem, nx, ny);
@@ -296,15 +296,7 @@ Tiles default_tiles(int elem, int nx, int ny) {
       t.xy_seg = std::min(16, step_segment(nx, ny));
   }
   t.y_block = nx >= 8 * 256 ? 256 : (nx >= 8 * 128 ? 128 : 64);
-  // about 512 workgroups (two per CU), each marching at least 32 rows:
-  // longer marches re-read fewer halo rows (8192^2 FP64 1.019 ms at 512
-  // rows against 1.059 at 128, FP32 0.510 against 0.540; 2048^2 keeps 32)
-  const long cols = (nx + t.y_block - 1) / t.y_block;
-  long want = (512 + cols - 1) / cols;
-  long seg = (ny + want - 1) / want;
-  if (seg < 32) seg = 32;
-  if (seg > ny) seg = ny;
-  t.y_seg = (int)seg;
+  t.y_seg = std::min(4, ny);  // one group of rows (kYRows in sweep.hip)
   const GridSize size{nx, ny};
   const PairShape p = pick_pair_shape(elem, &size, 1, 0, 192);
   t.pair_block = p.window;

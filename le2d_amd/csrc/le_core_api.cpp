@@ -658,7 +658,10 @@ int le2d_set_tiles(le_task *task, int x_rows, int y_seg, int y_block, int xy_seg
   if (x_rows < 0 || y_seg < 0 || xy_seg < 0 || !width_ok(y_block) || !width_ok(xy_block))
     return le2d::set_error(LE2D_ERR_ARG, "tiles %d %d %d %d %d", x_rows, y_seg, y_block, xy_seg,
                            xy_block);
-  if (x_rows) s->g.tiles.x_rows = x_rows;
+  if (x_rows) {
+    s->g.tiles.x_rows = x_rows;
+    s->g.tiles.x_fixed = true;
+  }
   if (y_seg) s->g.tiles.y_seg = y_seg;
   if (y_block) s->g.tiles.y_block = y_block;
   if (xy_seg) s->g.tiles.xy_seg = xy_seg;

@@ -9,7 +9,8 @@
 namespace le2d {
 
 // ---------------------------------------------------------------------------
-// x-sweep.  A workgroup of BX lanes owns BX consecutive nodes of a row and
+// x-sweep of FP32 grids that leave the last-level cache, and of a caller who set
+// the rows of a workgroup.  A workgroup of BX lanes owns BX consecutive nodes of a row and
 // walks `rows` rows.  Per row: coalesced loads of the five planes, invariants
 // to LDS (with a 2-node clamped halo each side), one face per lane (lane 0
 // also the segment's left face) to LDS, then the node update and coalesced
@@ -54,51 +55,78 @@ __global__ __launch_bounds__(BX) void k_sweep_x(const T *__restrict__ src, T *__
   }
 }
 
+// The x-sweep by wavefronts on their own, one row of a 64-column window each (60
+// written, as the fused step's): no barrier, 2 KB of LDS per wavefront and the tiles of
+// one XCD side by side, so that a window's halo and the cache lines it shares with
+// its neighbour are in that XCD's L2.  What bounds it is memory: FP64 4096 x 2049 116 us
+// against 138 above, 1500 x 1001 18.2 against 25.0, 8192 x 4096 460 against 502 (copy
+// rate 107, 19 and 427); FP32 1500 x 1001 9.7 against 12.3.
+template <typename T>
+constexpr int kRowWaves = sizeof(T) == 8 ? 1 : 4;  // FP64 4096 x 2049 118 us with 4
+
+template <typename T>
+__global__ __launch_bounds__(64 * kRowWaves<T>) void k_sweep_x_row(
+    const T *__restrict__ src, T *__restrict__ dst, int nx, int ny, long pitch, long plane,
+    int nstrips, SweepCoef<T> c) {
+  __shared__ X1Lds<T> lds[kRowWaves<T>];
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int v = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int t = (int)(threadIdx.x & 63);
+  const int x0 = tile % nstrips * 60, x = x0 - 2 + t;
+  const int j = tile / nstrips * kRowWaves<T> + v;
+  if (j >= ny) return;  // no barriers below
+  const unsigned boff = (unsigned)min(max(x, 0), nx - 1) * (unsigned)sizeof(T);
+  Nodes<T, 1> u = load_nodes<T, 1>(src + (long)j * pitch, plane, boff);
+  DivIeee<T> dv;
+  x_sweep(u, lds[v], t, x_edge<1, 2>(x0, nx, t), c, dv);
+  if (t >= 2 && t < 62 && x < nx)
+    store_nodes<T, 1>(dst + (long)j * pitch, plane, (unsigned)x * (unsigned)sizeof(T), u);
+}
+
 // ---------------------------------------------------------------------------
-// y-sweep.  Each lane owns one column and marches down a segment of `seg`
-// rows with a register window of invariants (positions j-1 .. j+2) and the
-// raw nodes of rows j .. j+2; every step reads one new row and writes one
-// row, so a wavefront's accesses are contiguous row pieces (no strided
-// loads, no transpose).  The face flux at j+1/2 computed in step j is reused
-// as the inflow face in step j+1.  Segments re-read two rows above and below.
+// y-sweep.  Each lane owns one column and takes a segment of `seg` rows in
+// groups of kYRows: all the group's rows and the two above and below it are loaded
+// before any arithmetic, so a wavefront has 40 accesses in flight where a march that
+// reads one row ahead had 5, and no access is strided.  The re-read rows come from
+// the caches.  Measured at the default, one group a segment, against the march
+// (us): FP32 4096 x 2049 57.8 against 69.3, 512^2 4.1 against 11.1, 8192^2 441 against
+// 511; FP64 1500 x 1001 20.2 against 30.1, 8192 x 4096 488 against 511 (copy rate
+// 53.5, 1.7, 427, 19 and 427).
+//
+// by_xcd: the tiles of one XCD are consecutive (xcd_tile), which keeps the re-read rows in
+// its L2 and pays where both buffers stay in the last-level cache (FP64 1500 x 1001
+// 20.2 us against 25.2); larger grids are walked in order (FP32 8192^2 441 against 456).
+constexpr int kYRows = 4;
+
 template <typename T, int EDGE>
 __global__ __launch_bounds__(256) void k_sweep_y(const T *__restrict__ src, T *__restrict__ dst,
                                                  int nx, int ny, long pitch, long plane, int seg,
-                                                 SweepCoef<T> c) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
+                                                 int nstrips, bool by_xcd, SweepCoef<T> c) {
+  const int tile = by_xcd ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  const int x = tile % nstrips * (int)blockDim.x + (int)threadIdx.x;
   if (x >= nx) return;  // no barriers below
-  const int j0 = blockIdx.y * seg;
-  const int j1 = min(j0 + seg, ny);
+  const int j0 = tile / nstrips * seg, j1 = min(j0 + seg, ny);
   const unsigned boff = (unsigned)x * (unsigned)sizeof(T);
-#define YROW(p) load_row_node(src + (long)ypos<EDGE>((p), ny) * pitch, plane, boff)
-
-  // prologue: positions j0-2 .. j0+2
-  const W4<T> wm2 = inv_y(YROW(j0 - 2), c);
-  W4<T> wm1 = inv_y(YROW(j0 - 1), c);
-  Node<T> u0 = YROW(j0);
-  Node<T> u1 = YROW(j0 + 1);
-  Node<T> u2 = YROW(j0 + 2);
-  W4<T> w0 = inv_y(u0, c), w1 = inv_y(u1, c), w2 = inv_y(u2, c);
-  W4<T> fin = faces(wm2, wm1, w0, w1, c);  // face j0-1/2
-
-  for (int j = j0; j < j1; ++j) {
-    // issue the read of position j+3 before this row's arithmetic (reading
-    // a row further ahead measured no faster)
-    const Node<T> un = YROW(j + 3);
-    const W4<T> fout = faces(wm1, w0, w1, w2, c);  // face j+1/2
-    Node<T> u = u0;
-    apply(u.vy, u.vx, u.syy, u.sxx, u.sxy, w0, fin, fout, c);
-    store_row_node(dst + (long)j * pitch, plane, boff, u);
-    fin = fout;
-    wm1 = w0;
-    w0 = w1;
-    w1 = w2;
-    u0 = u1;
-    u1 = u2;
-    u2 = un;
-    w2 = inv_y(un, c);
+  for (int j = j0; j < j1; j += kYRows) {
+    Node<T> u[kYRows + 4];  // positions j-2 ..
+#pragma unroll
+    for (int r = 0; r < kYRows + 4; ++r)
+      u[r] = load_row_node(src + (long)min(ypos<EDGE>(j + r - 2, ny), ny - 1) * pitch, plane, boff);
+    W4<T> wm = inv_y(u[1], c), w0 = inv_y(u[2], c), w1 = inv_y(u[3], c);
+    W4<T> fin = faces(inv_y(u[0], c), wm, w0, w1, c);  // face j-1/2
+#pragma unroll
+    for (int r = 0; r < kYRows; ++r) {
+      const W4<T> w2 = inv_y(u[r + 4], c);
+      const W4<T> fout = faces(wm, w0, w1, w2, c);
+      Node<T> &n = u[r + 2];
+      apply(n.vy, n.vx, n.syy, n.sxx, n.sxy, w0, fin, fout, c);
+      if (j + r < j1) store_row_node(dst + (long)(j + r) * pitch, plane, boff, n);
+      fin = fout;
+      wm = w0;
+      w0 = w1;
+      w1 = w2;
+    }
   }
-#undef YROW
 }
 
 // ---------------------------------------------------------------------------
@@ -357,17 +385,35 @@ template int step2_xy<float>(DevGrid *, const SweepCoef<float> &, const SweepCoe
 template int step_xy<double>(DevGrid *, const SweepCoef<double> &, const SweepCoef<double> &, int);
 template int step_xy<float>(DevGrid *, const SweepCoef<float> &, const SweepCoef<float> &, int);
 
+// Both buffers of the grid stay in the 256 MB last-level cache from one sweep to
+// the next.
+static bool stays_cached(const DevGrid *g) {
+  return 2 * g->pitch * (long)g->ny * g->elem <= 256l << 20;
+}
+
 template <typename T>
 int sweep_x(DevGrid *g, const SweepCoef<T> &c) {
   if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "sweep_x: element size mismatch");
-  constexpr int BX = 256;
-  // gridDim.y is at most 65535
-  const int rows = max(max(1, g->tiles.x_rows), (g->ny + 65534) / 65535);
   const T *src = static_cast<const T *>(g->buf[g->cur]);
   T *dst = static_cast<T *>(g->buf[g->cur ^ 1]);
-  dim3 grid((g->nx + BX - 1) / BX, (g->ny + rows - 1) / rows);
-  hipLaunchKernelGGL((k_sweep_x<T, BX>), grid, dim3(BX), 0, g->stream, src, dst, g->nx, g->ny,
-                     g->pitch, g->plane, rows, c);
+  // the wavefront form unless the caller set the rows of a workgroup; FP32 grids that
+  // leave the cache stay with whole workgroups, whose 1 KB row pieces need fewer
+  // halo lines (4096 x 2049 59 us against 62)
+  if (!g->tiles.x_fixed && (sizeof(T) == 8 || stays_cached(g))) {
+    constexpr int waves = kRowWaves<T>;
+    const int nstrips = (g->nx + 59) / 60;
+    const long nblocks = (long)nstrips * ((g->ny + waves - 1) / waves);
+    if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "sweep_x: grid too large");
+    hipLaunchKernelGGL((k_sweep_x_row<T>), dim3((unsigned)nblocks), dim3(64 * waves), 0, g->stream,
+                       src, dst, g->nx, g->ny, g->pitch, g->plane, nstrips, c);
+  } else {
+    constexpr int BX = 256;
+    // gridDim.y is at most 65535
+    const int rows = max(max(1, g->tiles.x_rows), (g->ny + 65534) / 65535);
+    dim3 grid((g->nx + BX - 1) / BX, (g->ny + rows - 1) / rows);
+    hipLaunchKernelGGL((k_sweep_x<T, BX>), grid, dim3(BX), 0, g->stream, src, dst, g->nx, g->ny,
+                       g->pitch, g->plane, rows, c);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(ERR_DEVICE, "sweep_x launch: %s", hipGetErrorString(e));
   g->cur ^= 1;
@@ -378,16 +424,18 @@ template <typename T>
 int sweep_y(DevGrid *g, const SweepCoef<T> &c, int edge) {
   if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "sweep_y: element size mismatch");
   const int bx = g->tiles.y_block == 64 || g->tiles.y_block == 128 ? g->tiles.y_block : 256;
-  const int seg = max(max(1, g->tiles.y_seg), (g->ny + 65534) / 65535);
-  dim3 grid((g->nx + bx - 1) / bx, (g->ny + seg - 1) / seg);
+  const int seg = max(1, g->tiles.y_seg), nstrips = (g->nx + bx - 1) / bx;
+  const long nblocks = (long)nstrips * ((g->ny + seg - 1) / seg);
+  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "sweep_y: grid too large");
   const T *src = static_cast<const T *>(g->buf[g->cur]);
   T *dst = static_cast<T *>(g->buf[g->cur ^ 1]);
+  const bool by_xcd = stays_cached(g);
   if (edge == EDGE_RING)
-    hipLaunchKernelGGL((k_sweep_y<T, EDGE_RING>), grid, dim3(bx), 0, g->stream, src, dst, g->nx,
-                       g->ny, g->pitch, g->plane, seg, c);
+    hipLaunchKernelGGL((k_sweep_y<T, EDGE_RING>), dim3((unsigned)nblocks), dim3(bx), 0, g->stream,
+                       src, dst, g->nx, g->ny, g->pitch, g->plane, seg, nstrips, by_xcd, c);
   else
-    hipLaunchKernelGGL((k_sweep_y<T, EDGE_CLAMP>), grid, dim3(bx), 0, g->stream, src, dst, g->nx,
-                       g->ny, g->pitch, g->plane, seg, c);
+    hipLaunchKernelGGL((k_sweep_y<T, EDGE_CLAMP>), dim3((unsigned)nblocks), dim3(bx), 0, g->stream,
+                       src, dst, g->nx, g->ny, g->pitch, g->plane, seg, nstrips, by_xcd, c);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(ERR_DEVICE, "sweep_y launch: %s", hipGetErrorString(e));
   g->cur ^= 1;
