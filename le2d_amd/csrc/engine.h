@@ -103,6 +103,8 @@ void grid_free(DevGrid *g);
 // nx*ny nodes of five values; SOA host arrays hold five planes of nx*ny.
 int grid_upload(DevGrid *g, const void *host, int soa);
 int grid_download(DevGrid *g, void *host, int soa);
+// Starts on the grid's stream the AOS image of the state in the idle buffer.
+int grid_aos_image(DevGrid *g, void **image);
 
 // One sweep of the current state into the other buffer, then swap.
 template <typename T>

@@ -250,7 +250,19 @@ int grid_download(DevGrid *g, void *host, int soa) {
     }
     return check(hipStreamSynchronize(g->stream), "download sync");
   }
-  void *stage = g->buf[g->cur ^ 1];
+  void *stage = nullptr;
+  int rc = grid_aos_image(g, &stage);
+  if (rc) return rc;
+  rc = check(hipMemcpyAsync(host, stage, (size_t)g->nx * g->ny * 5 * es, hipMemcpyDeviceToHost,
+                            g->stream),
+             "download");
+  if (rc) return rc;
+  return check(hipStreamSynchronize(g->stream), "download sync");
+}
+
+int grid_aos_image(DevGrid *g, void **image) {
+  const void *cur = g->buf[g->cur];
+  void *stage = *image = g->buf[g->cur ^ 1];
   const long n = (long)g->nx * g->ny;
   const int bs = 256;
   const unsigned nb = (unsigned)((n + bs - 1) / bs);
@@ -262,12 +274,7 @@ int grid_download(DevGrid *g, void *host, int soa) {
     hipLaunchKernelGGL(k_planes_to_aos<float>, dim3(nb), dim3(bs), 0, g->stream,
                        static_cast<const float *>(cur), static_cast<float *>(stage), g->nx, g->ny,
                        g->pitch, g->plane);
-  int rc = check(hipGetLastError(), "planes_to_aos launch");
-  if (rc) return rc;
-  rc = check(hipMemcpyAsync(host, stage, (size_t)n * 5 * es, hipMemcpyDeviceToHost, g->stream),
-             "download");
-  if (rc) return rc;
-  return check(hipStreamSynchronize(g->stream), "download sync");
+  return check(hipGetLastError(), "planes_to_aos launch");
 }
 
 static int step_blocks(int elem, int nx, int ny);
