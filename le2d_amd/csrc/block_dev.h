@@ -1,22 +1,24 @@
 // block_dev.h -- one or two full steps per pass on blocks held in registers.
 //
-// Two steps, for grids that do not fill the device.
-// What bounds a pass of pair_dev.h's march on a small grid is one workgroup's
-// march: every row waits for the row before it, two exchanges and a barrier, and
-// short segments, which put more of the device to work, recompute more halo
-// rows.  Here a workgroup of WV wavefronts holds a block of 64 columns by R*WV
-// rows, R rows per wavefront and one column per lane, and takes each of the four
-// sweeps on all of it at once: all loads in flight together, the x-sweeps of a
-// wavefront's rows independent of each other, and two exchanges of boundary
-// rows between neighbouring wavefronts per y-sweep.  It writes the 56 columns
-// and R*WV-8 rows between the halos (one step: 60 and R*WV-4).  It does not overlap one block's loads with
-// another's arithmetic, so it is taken where every block has a compute unit to
-// itself and the march stays elsewhere.
+// Two steps, for grids that do not fill the device.  What bounds a pass of
+// pair_dev.h's march on a small grid is one workgroup's march: every row waits
+// for the row before it, two exchanges and a barrier, and short segments, which
+// put more of the device to work, recompute more halo rows.  Here a workgroup
+// of WV wavefronts holds a block of 64 columns by R*WV rows, R rows per
+// wavefront and one column per lane, and takes each of the four sweeps on all
+// of it at once: all loads in flight together, the x-sweeps of a wavefront's
+// rows independent of each other, and two exchanges of boundary rows between
+// neighbouring wavefronts per y-sweep.  It writes the 56 columns and R*WV-8
+// rows between the halos (one step: 60 and R*WV-4).  One block's loads do not
+// overlap its own arithmetic, so FP64, whose registers allow one block a
+// compute unit, takes it where every block has a unit to itself, FP32 up to a
+// few more.
 //
 // us a pass, block against march: FP64 96 x 80 7.6 against 9.1, 250 x 300 8.5 against
 // 12.4, 512^2 14.6 against 19.1, 724^2 23.0 against 25.3, but 900^2 (two rounds
 // of blocks) 37 against 34; FP32 250 x 300 4.5 against 6.5, 512^2 7.1 against 9.3, 1031
-// x 517 9.5 against 12.1, 900^2 13.4 against 16.1.
+// x 517 9.5 against 12.1, 900^2 13.4 against 16.1, and past one block a unit 1500 x
+// 1001 21.4 against 23.3, but 3000^2 95 against 94.
 //
 // One step.  With half the halo the blocks pay on larger grids too: in FP32,
 // where two or more of them share a compute unit and one loads while another computes,
