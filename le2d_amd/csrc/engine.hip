@@ -310,13 +310,15 @@ Tiles default_tiles(int elem, int nx, int ny) {
   t.pair_seg = p.seg;
   // blocks where each has a compute unit to itself, of the fewest rows that give
   // that (block_dev.h has both sides' times); in FP32, where several share one, also
-  // blocks of 40 rows on grids of up to five for each (1200^2 21.0 us against 23.2
-  // marched, 2048 x 1024 28.2 against 29.6, 2048^2, 7.5 for each, 43.5 against 43.0)
+  // blocks of 40 rows on grids of up to 16 for each (us a pass, blocks against the
+  // march at its default shape: 2500 x 1500 41.2 and 45.1, 2961 x 2216 64.9 and 70.2,
+  // 3500 x 2500, 15.5 for each, 89.8 and 95.5; against the march's fastest shape 1200^2
+  // 21.0 and 23.2, 2048^2 43.5 and 43.0)
   auto blocks = [&](int rows) { return (long)((nx + 55) / 56) * ((ny + rows - 1) / rows); };
   t.block_rows = 0;
   for (int k = 0; k < kBlockKinds && !t.block_rows; ++k)
     if (blocks(block_rows(elem, k)) <= device_cus()) t.block_rows = block_rows(elem, k);
-  if (elem == 4 && !t.block_rows && blocks(40) <= 5 * device_cus()) t.block_rows = 40;
+  if (elem == 4 && !t.block_rows && blocks(40) <= 16 * device_cus()) t.block_rows = 40;
   return t;
 }
 

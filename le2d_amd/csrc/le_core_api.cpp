@@ -248,12 +248,12 @@ int tune_pairs(le_task *t, TaskState *s) {
       if (ms < best.ms) best = {ms, c.block, c.seg};
     }
   }
-  // blocks, up to two for each compute unit (FP32 eight), against the fastest march
+  // blocks, up to two for each compute unit (FP32 16), against the fastest march
   int rows = 0;
   for (int k = 0; k < le2d::kBlockKinds && !rc && best.ms < 1e30f; ++k) {
     const int r = le2d::block_rows((int)sizeof(real), k);
     const long n = (long)((s->g.nx + 55) / 56) * ((s->g.ny + r - 1) / r);
-    if (n > (sizeof(real) == 4 ? 8 : 2) * le2d::device_cus()) continue;
+    if (n > (sizeof(real) == 4 ? 16 : 2) * le2d::device_cus()) continue;
     const float ms = time_one(best.block, best.seg, r, 12);
     if (ms < 0) break;
     if (ms < best.ms) {

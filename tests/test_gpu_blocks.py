@@ -55,7 +55,7 @@ def test_values_outside_the_bounds(value):
     assert gd.same_bits(got[~nan], ref[~nan])
 
 
-@pytest.mark.parametrize("nx,ny", [(1201, 1161), (1960, 1400), (1961, 1441)])
+@pytest.mark.parametrize("nx,ny", [(1201, 1161), (1960, 1400), (1961, 1441), (3501, 2521)])
 def test_fp32_blocks_that_share_units(nx, ny):
     g0 = np.random.default_rng(nx * ny).standard_normal((ny, nx, 5)).astype(np.float32)
     assert gd.same_bits(_run(g0, np.float32, 2), _run(g0, np.float32, 2, pairs=0))
