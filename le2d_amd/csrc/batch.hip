@@ -49,6 +49,7 @@ struct Shape {
              // workgroups walk the table; FORM_PAIRS: one workgroup per tile of
              // the two-step table, two steps per launch, in windows of 64, 128
              // or 256 columns; FORM_PAIRS_SPLIT: the same in windows of 64
+  int rows = 0;  // FORM_PAIRS: blocks of this many rows (fb 64, seg rows), 0: the march
 };
 
 std::mutex g_tune_mu;
@@ -206,10 +207,10 @@ struct BatchImpl {
     if (shape.form == FORM_PERSISTENT)
       hipLaunchKernelGGL((k_step_batch<T, FB>), dim3(blocks), dim3(FB), 0, stream, d, d_tiles,
                          ntiles, par);
-    else if (two_step(shape.form))
-      hipLaunchKernelGGL(batch_pair_kernel<T>(pair_cols(elem, FB)), dim3(ntiles), dim3(128), 0,
-                         stream, d, d_tiles, par);
-    else
+    else if (two_step(shape.form)) {
+      const BatchPairKernel<T> k = batch_pair_kernel<T>(pair_cols(elem, FB), shape.rows);
+      hipLaunchKernelGGL(k.kernel, dim3(ntiles), dim3(k.lanes), 0, stream, d, d_tiles, par);
+    } else
       hipLaunchKernelGGL((k_step_batch_tiles<T, FB>), dim3(ntiles), dim3(FB), 0, stream, d,
                          d_tiles, par);
   }
@@ -369,6 +370,8 @@ int le2d_batch_commit(le2d_batch *b) {
   for (const auto &in : B.inst) sizes.push_back({in.nx, in.ny});
   const le2d::PairShape p = le2d::pick_pair_shape(B.elem, sizes.data(), sizes.size(), 0, 160);
   le2d::Shape s{p.window, p.seg, le2d::FORM_PAIRS};
+  if (const int rows = le2d::batch_block_rows(B.elem, sizes.data(), sizes.size(), 160))
+    s = {64, rows, le2d::FORM_PAIRS, rows};
   {
     std::lock_guard<std::mutex> lk(le2d::g_tune_mu);
     auto it = le2d::g_tune.find({B.elem, (int)B.inst.size(), B.total_nodes() >> 20});
@@ -506,7 +509,7 @@ int le2d_batch_time(le2d_batch *b, int steps, int plain, double *ms) {
 
 // Times every candidate shape and keeps the fastest (per step): the
 // single-step forms at every window width and segment height, and the
-// two-step form at every segment height.  Stepping the batch is part of
+// two-step form at every segment height, and the default if that is in blocks.  Stepping the batch is part of
 // tuning: the instances advance by an even number of steps per candidate,
 // so callers tune before loading their initial state or account for it.
 int le2d_batch_autotune(le2d_batch *b, int trials, int *best_fb, int *best_seg, double *best_ms) {
@@ -515,6 +518,7 @@ int le2d_batch_autotune(le2d_batch *b, int trials, int *best_fb, int *best_seg, 
   const int fbs[3] = {64, 128, 256};
   const int segs[4] = {16, 32, 64, 128};
   std::vector<le2d::Shape> cand;
+  if (B.shape.rows) cand.push_back(B.shape);
   for (int form : {le2d::FORM_TILES, le2d::FORM_PERSISTENT})
     for (int fb : fbs)
       for (int seg : segs) cand.push_back({fb, seg, form});

@@ -5,7 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
-#include "pair_dev.h"
+#include "block_dev.h"
 
 namespace le2d {
 
@@ -89,15 +89,55 @@ __global__ __launch_bounds__(128, (pair_waves<T, 1>())) void k_step_batch_pairs_
                   d.cx, d.cy, lds);
 }
 
-// The batched two-step kernel of a window of `cols` columns (pair_cols).
+// The two-step pass in blocks of R rows on each of WV wavefronts (block_tile): a
+// table of 56-column strips in segments of a block's R*WV-8 rows.
+template <typename T, int R, int WV>
+__global__ __launch_bounds__(64 * WV) void k_step_batch_blocks(
+    const InstDesc<T> *__restrict__ inst, const TileJob *__restrict__ tiles, int step_parity) {
+  __shared__ BlockLds<T> lds[WV];
+  const TileJob tj = tiles[xcd_tile(blockIdx.x, gridDim.x)];
+  const InstDesc<T> &d = inst[tj.inst];
+  const int p = d.par ^ step_parity;
+  block_tile<T, 2, EDGE_CLAMP, R, WV>(d.buf[p], d.buf[p ^ 1], d.nx, d.ny, d.pitch, d.plane,
+                                      tj.strip, tj.j0, d.cx, d.cy, lds);
+}
+
+// The batched two-step kernel of a shape and its lanes: blocks of `rows` rows, or
+// (rows = 0) the march in windows of `cols` columns (pair_cols).
 template <typename T>
-using BatchPairKernel = void (*)(const InstDesc<T> *, const TileJob *, int);
+struct BatchPairKernel {
+  void (*kernel)(const InstDesc<T> *, const TileJob *, int);
+  int lanes;
+};
 template <typename T>
-inline BatchPairKernel<T> batch_pair_kernel(int cols) {
-  if (cols == 64) return k_step_batch_pairs_split<T>;
-  if constexpr (sizeof(T) == 4)
-    if (cols == 256) return k_step_batch_pairs<T, 256>;
-  return k_step_batch_pairs<T, 128>;
+inline BatchPairKernel<T> batch_pair_kernel(int cols, int rows) {
+  if (rows == 8) return {k_step_batch_blocks<T, 2, 8>, 512};
+  if (rows == 16) return {k_step_batch_blocks<T, 3, 8>, 512};
+  if (rows == 24) return {k_step_batch_blocks<T, 4, 8>, 512};
+  if constexpr (sizeof(T) == 4) {
+    if (rows == 40) return {k_step_batch_blocks<T, 4, 12>, 768};
+    if (cols == 256) return {k_step_batch_pairs<T, 256>, 128};
+  } else {
+    if (rows == 32) return {k_step_batch_blocks<T, 5, 8>, 512};
+  }
+  if (cols == 64) return {k_step_batch_pairs_split<T>, 128};
+  return {k_step_batch_pairs<T, 128>, 128};
+}
+
+// Rows of the blocks that a two-step launch over n grids runs in (at most `cap`), 0
+// for the march: the lowest blocks of which each has a compute unit to itself, as
+// on a single grid (us for 20 steps of 6 instances of 48 to 200, march against
+// blocks: FP32 110 and 96, FP64 183 and 152).  More blocks than that are no faster
+// than the march, FP32 either (48 of 128 to 1024 997 and 999, 12 of 128 to 300 178
+// and 175): on many grids their last strips and rows are a larger share.
+inline int batch_block_rows(int elem, const GridSize *g, size_t n, int cap) {
+  for (int rows : {8, 16, 24, elem == 8 ? 32 : 40}) {
+    long blocks = 0;
+    for (size_t i = 0; i < n; ++i)
+      blocks += (long)((g[i].nx + 55) / 56) * ((g[i].ny + rows - 1) / rows);
+    if (rows <= cap && blocks <= device_cus()) return rows;
+  }
+  return 0;
 }
 
 // Disk initial condition with the host le_set_ball's arithmetic: the node

@@ -231,6 +231,7 @@ struct Server {
     int fb = 256, seg = 16, pair_seg = 64, pair_fb = 0;
   } act;
   int pair_window[2] = {64, 64};  // columns of the current tables' two-step windows
+  int pair_rows[2] = {0, 0};      // rows of their blocks (0: the march)
   char *arena_dev = nullptr;
   Arena arena;
   std::mutex mu;
@@ -372,14 +373,16 @@ struct Server {
     return OK;
   }
 
-  // Window and segment height (at most pair_seg rows) of the two-step launches
-  // for the live set of one precision, from the model of the single-grid
+  // Window and segment height (at most pair_seg rows), or block height, of the two-step
+  // launches for the live set of one precision, from the model of the single-grid
   // pass over all live requests.  Many live requests keep wide windows and
   // tall segments; the few of a light load or of the tail of a burst take
   // narrow and short ones, as a small grid does.
-  PairShape live_pair_shape(int si, const std::vector<Req *> &set) const {
+  PairShape live_pair_shape(int si, const std::vector<Req *> &set, int *rows) const {
     std::vector<GridSize> g;
     for (const Req *r : set) g.push_back({r->spec.nx, r->spec.ny});
+    *rows = act.pair_fb ? 0 : batch_block_rows(si == 1 ? 8 : 4, g.data(), g.size(), act.pair_seg);
+    if (*rows) return {64, *rows};
     return pick_pair_shape(si == 1 ? 8 : 4, g.data(), g.size(), act.pair_fb, act.pair_seg);
   }
 
@@ -389,7 +392,7 @@ struct Server {
     std::vector<TileJob> tiles, tiles2;
     int seg2 = 0;
     if (act.pair_seg > 0) {
-      const PairShape p = live_pair_shape(si, set);
+      const PairShape p = live_pair_shape(si, set, &pair_rows[si]);
       seg2 = p.seg;
       pair_window[si] = pair_cols((int)sizeof(T), p.window);
     }
@@ -470,8 +473,8 @@ struct Server {
     if (count <= 0) return;
     const dim3 grid((unsigned)count);
     const InstDesc<T> *d = static_cast<const InstDesc<T> *>(d_inst[si]);
-    hipLaunchKernelGGL(batch_pair_kernel<T>(pair_window[si]), grid, dim3(128), 0, stream[si], d,
-                       d_tiles2[si], step_parity);
+    const BatchPairKernel<T> k = batch_pair_kernel<T>(pair_window[si], pair_rows[si]);
+    hipLaunchKernelGGL(k.kernel, grid, dim3(k.lanes), 0, stream[si], d, d_tiles2[si], step_parity);
   }
 
   // Requests of the current tables of precision si with at least k steps
