@@ -821,7 +821,8 @@ int le2d_set_material_plane(le_task *task, int count, const double *c1_c2_rho,
     // 147 against 168 at 256).
     const le2d::GridSize g{s->g.nx, s->g.ny};
     const int only = count > 0 && (long)g.nx * g.ny < (1L << 26) ? 64 : 0;
-    const le2d::PairShape p = le2d::pick_pair_shape((int)sizeof(real), &g, 1, only, only ? 64 : 192);
+    const int cap = only || (count > 0 && sizeof(real) == 4) ? 64 : 192;
+    const le2d::PairShape p = le2d::pick_pair_shape((int)sizeof(real), &g, 1, only, cap);
     s->g.tiles.pair_block = p.window;
     s->g.tiles.pair_seg = p.seg;
   }

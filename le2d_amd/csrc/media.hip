@@ -532,18 +532,25 @@ static int join_aux(DevGrid *g, MatPlane *m) {
 }
 
 // Whether the interface tiles run as `blocks` blocks rather than as `mixed`
-// marched tiles of `lanes` lanes and `rows` rows.  Measured (FP64 / FP32): a
-// round of blocks, one / two per CU, takes 11 / 7 us; a marched row 5 / 3 us while
-// its wavefronts fit in a round of three per SIMD, and the second stream that
-// hides the march behind the single-material tiles 15 us.  Two layers and an inclusion
-// on 4100 x 3000: 382 us a pass with blocks against 478 (FP64), 186 against 194
-// (FP32), on 1500 x 1000 76 against 114 and 31 against 65; a checkerboard of
-// interface tiles only, 3000 x 2000: 439 us marched against 546 in blocks.
-static bool blocks_pay(int elem, size_t mixed, int lanes, int rows, size_t blocks) {
+// marched tiles of `lanes` lanes and `rows` rows beside `nodes` nodes of single-material
+// tiles.  Measured (FP64 / FP32): a round of blocks, one / two per CU, takes 11 / 7 us; a
+// marched row 5 / 3 us while its wavefronts fit in a round of three per SIMD; the
+// second stream that hides the march behind the single-material tiles 15 us.
+// What that does not hide, or else the march's share of the device (both faces of
+// every node, so about twice a single-material node's), adds to the pass.  Two
+// layers and an inclusion on 4100 x 3000: 382 us a pass with blocks against 478 (FP64),
+// 186 against 194 (FP32), on 1500 x 1000 76 against 114 and 31 against 65.
+// Two layers on 16384^2, where the march is hidden: FP64 5.04 ms with blocks, FP32 2.52
+// against 2.27.  A checkerboard of interface tiles only, 3000 x 2000: 439 us marched against
+// 546 in blocks.
+static bool blocks_pay(int elem, size_t mixed, int lanes, int rows, size_t blocks, double nodes) {
   const size_t waves = mixed * (lanes / 64), round = elem == 8 ? 256 : 512;
   const double block_us = elem == 8 ? 11 : 7, row_us = elem == 8 ? 5 : 3;
+  const double nodes_per_us = elem == 8 ? 40e3 : 100e3;  // of a two-step pass
+  const double march = (double)((waves + 3071) / 3072) * (rows + 8) * row_us;
+  const double share = 2 * (double)mixed * lanes * rows / nodes_per_us;
   return (double)((blocks + round - 1) / round) * block_us <
-         (double)((waves + 3071) / 3072) * (rows + 8) * row_us + 15;
+         (elem == 8 ? std::max(march - nodes / nodes_per_us, share) : march) + 15;
 }
 
 // Tables of the two-step pass: strips of (window - 8) columns read 4 halo
@@ -557,7 +564,9 @@ static int mat_tiles2(DevGrid *g, MatPlane *m) {
   std::vector<MatTile> homogb = homog;
   std::vector<MixBlock> blocks;
   split_bands(m, g->nx, g->ny, fb - 8, mixed, &homogb, &blocks);
-  if (blocks_pay(g->elem, mixed.size(), fb, std::min(seg, g->ny), blocks.size())) {
+  double nodes = 0;
+  for (const MatTile &t : homog) nodes += (double)(t.j1 - t.j0) * (fb - 8);
+  if (blocks_pay(g->elem, mixed.size(), fb, std::min(seg, g->ny), blocks.size(), nodes)) {
     homog.swap(homogb);
     mixed.clear();
   } else {
