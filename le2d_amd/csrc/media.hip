@@ -506,11 +506,11 @@ static int mat_tiles(DevGrid *g, MatPlane *m, int edge) {
   return OK;
 }
 
-// Marched interface tiles are slow (both faces of every node), so run after the single-material tiles they would leave the device mostly
-// idle: 0.44 ms of a 6.5 ms two-step pass on 16384^2.  They are launched
-// first, on a second stream forked from the grid's stream, and joined back
-// before the next launch on it.  Both launches read the same input and write
-// disjoint tiles.
+// Marched interface tiles are slow (both faces of every node), so run after the
+// single-material tiles they would leave the device mostly idle: 0.44 ms of a 6.5 ms
+// two-step pass on 16384^2.  They are launched first, on a second stream forked from
+// the grid's stream, and joined back before the next launch on it.  Both launches
+// read the same input and write disjoint tiles.
 static int fork_aux(DevGrid *g, MatPlane *m) {
   if (!m->aux) {
     if (hipStreamCreateWithFlags(&m->aux, hipStreamNonBlocking) != hipSuccess ||
@@ -536,13 +536,15 @@ static int join_aux(DevGrid *g, MatPlane *m) {
 // tiles.  Measured (FP64 / FP32): a round of blocks, one / two per CU, takes 11 / 7 us; a
 // marched row 5 / 3 us while its wavefronts fit in a round of three per SIMD; the
 // second stream that hides the march behind the single-material tiles 15 us.
-// What that does not hide, or else the march's share of the device (both faces of
-// every node, so about twice a single-material node's), adds to the pass.  Two
-// layers and an inclusion on 4100 x 3000: 382 us a pass with blocks against 478 (FP64),
-// 186 against 194 (FP32), on 1500 x 1000 76 against 114 and 31 against 65.
-// Two layers on 16384^2, where the march is hidden: FP64 5.04 ms with blocks, FP32 2.52
-// against 2.27.  A checkerboard of interface tiles only, 3000 x 2000: 439 us marched against
-// 546 in blocks.
+// Two layers and an inclusion on 4100 x 3000: 382 us a pass with blocks against 478
+// (FP64), 186 against 194 (FP32), on 1500 x 1000 76 against 114 and 31 against 65.  A
+// checkerboard of interface tiles only, 3000 x 2000: 439 us marched against 546
+// in blocks.
+// In FP64 only what the single-material tiles do not hide of the march, or else its
+// share of the device (both faces of every node, about twice a single-material
+// node's work), adds to the pass: two layers on 16384^2 4.9 ms marched against 5.04.  In
+// FP32 two wavefronts of 223 registers a SIMD leave it no room beside them (2.95 ms
+// marched against 2.52).
 static bool blocks_pay(int elem, size_t mixed, int lanes, int rows, size_t blocks, double nodes) {
   const size_t waves = mixed * (lanes / 64), round = elem == 8 ? 256 : 512;
   const double block_us = elem == 8 ? 11 : 7, row_us = elem == 8 ? 5 : 3;

@@ -167,9 +167,9 @@ __global__ __launch_bounds__(64 * WV, (R > 6 ? 2 : 1)) void k_step_block(
 // Two steps over one grid (pair_tile in pair_dev.h) in windows of FB columns,
 // FB/64 per lane ...
 template <typename T, int FB>
-__global__ __launch_bounds__(128, (pair_waves<T, FB / 64>())) void k_step2_xy(const T *__restrict__ src, T *__restrict__ dst,
-                                                  int nx, int ny, long pitch, long plane, int seg,
-                                                  int nstrips, SweepCoef<T> cx, SweepCoef<T> cy) {
+__global__ __launch_bounds__(128, (pair_waves<T, FB / 64>())) void k_step2_xy(
+    const T *__restrict__ src, T *__restrict__ dst, int nx, int ny, long pitch, long plane,
+    int seg, int nstrips, SweepCoef<T> cx, SweepCoef<T> cy) {
   __shared__ PairLds<T, FB / 64> lds;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int strip = tile % nstrips, segi = tile / nstrips;
@@ -338,7 +338,8 @@ int step_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy, int edge
 template <typename T>
 int step2_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy) {
   if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "step2_xy: element size mismatch");
-  if (g->tiles.block_rows) return launch_blocks<T>(g, cx, cy, block_kernels<T>(), kBlockKinds, g->tiles.block_rows, 56,
+  if (g->tiles.block_rows)
+    return launch_blocks<T>(g, cx, cy, block_kernels<T>(), kBlockKinds, g->tiles.block_rows, 56,
                             "step2_xy");
   const int seg = g->tiles.pair_seg;
   if (seg < 1) return set_error(ERR_ARG, "step2_xy: no pair segment height");
