@@ -433,6 +433,28 @@ PairShape pick_pair_shape(int elem, const GridSize *g, size_t n, int only, int c
       if (s >= tall) break;
     }
   }
+  // Several FP32 grids that this puts into one round of 64-column workgroups: with
+  // 75 registers three rounds are resident at once, and r of them last (1 + r) / 2 of
+  // one (25 instances of 128 to 384, 37 steps: 517 us at 32 rows, one round, 455 at
+  // 14, two; 16 of 96 to 500, 36 steps: 400 at 20, one, 370 at 10, two).
+  if (n > 1 && elem == 4 && best.window == 64) {
+    const long slots = pair_slots(elem, 64);
+    double cost = 0;
+    for (int k = (int)(sizeof few / sizeof *few) - 1; k >= 0; --k) {
+      if (few[k] > best.seg || few[k] > cap) continue;
+      long blocks = 0;
+      for (size_t i = 0; i < n; ++i)
+        blocks += (long)((g[i].nx + 55) / 56) * ((g[i].ny + few[k] - 1) / few[k]);
+      const long rounds = (blocks + slots - 1) / slots;
+      if (!cost && rounds != 1) break;
+      if (rounds > 3) break;
+      const double c = (few[k] + 8) * (1.0 + rounds) / 2;
+      if (!cost || c < cost) {
+        cost = c;
+        best.seg = few[k];
+      }
+    }
+  }
   best.seg = std::max(1, std::min(best.seg, cap));
   return best;
 }
