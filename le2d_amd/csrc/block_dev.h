@@ -75,7 +75,7 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
   for (int r = 0; r < R; ++r)
     u[r] = load_nodes<T, 1>(src + (long)min(ypos<EDGE>(jw + r, ny), ny - 1) * pitch, plane, boff);
 #pragma unroll
-  for (int r = 0; r < R; ++r) see_row(u[r], dv);
+  for (int r = 0; r < R; ++r) see_row(u[r], ed, t, dv);
 #pragma unroll 1
   for (int s = 0;; ++s) {
 #pragma unroll

@@ -114,7 +114,7 @@ __device__ __forceinline__ Nodes<T, C> load_nodes(const T *__restrict__ row, lon
 }
 
 // Columns past nx-1 of a lane's access fall in the row's padding to 256 bytes,
-// which nothing reads as a node.
+// which no output depends on and which may hold anything (see_row).
 template <typename T, int C>
 __device__ __forceinline__ void store_nodes(T *__restrict__ row, long plane, unsigned boff,
                                             const Nodes<T, C> &u) {
@@ -140,8 +140,19 @@ __device__ __forceinline__ W4<T> pick_w(bool c, const W4<T> &a, const W4<T> &b) 
   return {c ? a.a : b.a, c ? a.b : b.b, c ? a.c : b.c, c ? a.d : b.d};
 }
 
-template <typename T, int C, typename Div>
-__device__ __forceinline__ void see_row(const Nodes<T, C> &u, Div &dv) {
+// Shows the row's values to `dv`.  With several columns per lane the lanes from
+// the grid's last column on also hold columns of the padding, which is never
+// initialised: they take the last column's values, so that what the memory held
+// before cannot send a tile to the IEEE divisions (FP64 2047 x 2048 with NaN in the
+// padding 167 us a pass, 121 with zeros or this).
+template <typename T, int C, typename Edge, typename Div>
+__device__ __forceinline__ void see_row(Nodes<T, C> &u, const Edge &d, int t, Div &dv) {
+  if constexpr (C > 1 && Div::kSees) {
+    if (d.any) {  // wavefront-uniform
+#pragma unroll
+      for (int k = 1; k < C; ++k) u.n[k] = pick_node(t >= d.th && k > d.e, u.n[k - 1], u.n[k]);
+    }
+  }
 #pragma unroll
   for (int k = 0; k < C; ++k) {
     const T f[5] = {u.n[k].vx, u.n[k].vy, u.n[k].sxx, u.n[k].sxy, u.n[k].syy};
@@ -423,7 +434,7 @@ __device__ __forceinline__ void march_rows(const T *__restrict__ src, int ny, lo
     for (int p = q - 1; p <= q + 3; ++p) {
       Nodes<T, C> u = N;
       N = ROW(p);
-      see_row(u, dv);
+      see_row(u, ed, t, dv);
       x_sweep(u, lds, t, ed, cx, dv);
       w2 = wb;
       wb = inv_y(A, cy);
@@ -448,7 +459,7 @@ __device__ __forceinline__ void march_rows(const T *__restrict__ src, int ny, lo
     if (++k >= rows) break;                                                          \
     P0 = N;                                                                          \
     N = ROW(q + 4);                                                                  \
-    see_row(P0, dv);                                                                 \
+    see_row(P0, ed, t, dv);                                                          \
     x_sweep(P0, lds, t, ed, cx, dv);                                                 \
     if constexpr (HOLD) W0 = inv_y(P0, cy);                                          \
     ++q;                                                                             \

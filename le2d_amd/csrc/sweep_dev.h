@@ -115,6 +115,7 @@ __device__ __forceinline__ float slope_ratio(float n, float d) {
 // How a march divides.  DivIeee: slope_ratio whatever the operands.
 template <typename T>
 struct DivIeee {
+  static constexpr bool kSees = false;  // whether see and row do anything
   __device__ __forceinline__ T ratio(T n, T d) { return slope_ratio(n, d); }
   __device__ __forceinline__ void see(T, T) {}
   __device__ __forceinline__ void row(const T (&)[5]) {}
@@ -145,6 +146,7 @@ struct DivIeee {
 // 2^39 divisors below a power of two (1.4e12 quotients), and on 2e10 random
 // ones: all equal to n / d.
 struct DivBounded {
+  static constexpr bool kSees = true;
   float big = 0.0f, small = 1.0f;
   static __device__ __forceinline__ float hi(double x) {
     return __builtin_bit_cast(float, (int)(__builtin_bit_cast(unsigned long long, x) >> 32));
