@@ -76,12 +76,24 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
     u[r] = load_nodes<T, 1>(src + (long)min(ypos<EDGE>(jw + r, ny), ny - 1) * pitch, plane, boff);
 #pragma unroll
   for (int r = 0; r < R; ++r) see_row(u[r], ed, t, dv);
+  // A wavefront whose rows are out of the divisions' range only passes the barriers
+  // from here on, as block_tile takes the block again (FP64 512^2 with NaN everywhere 20.9
+  // us a pass, 27.9 with both marches in full; finite 16.7 either way).  It is asked
+  // behind x-sweeps, which need not wait for every row's load then (asked before
+  // them 512^2 is 17.2); the tall block, short of registers, before its last ones.
+  auto stand_by = [&] {
+    if (!Div::kSees || __all(dv.in_range())) return false;
+#pragma unroll 1
+    for (int k = 0; k < 4 * STEPS - 1; ++k) __syncthreads();
+    return true;
+  };
 #pragma unroll 1
   for (int s = 0;; ++s) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       x_sweep(u[r], lds[v].x, t, ed, cx, dv);
       pin(u[r].n[0]);
+      if (R > 6 && r == R - 3 && stand_by()) return;
     }
     // after a step rows outside the grid take the edge row's value (one step's are
     // loaded so)
@@ -98,6 +110,7 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
     lds[v].y.first[t] = w.w[0];
     lds[v].y.second[t] = {w.w[1].b, w.w[1].d};
     lds[v].y.last[t] = {w.w[R - 1].a, w.w[R - 1].c};
+    if (R <= 6 && s == 0 && stand_by()) return;
     __syncthreads();
     // the row above (a and c) and two rows below; rows past the block's own
     // edge stand for nothing that an output reads, rows past the grid's take its

@@ -403,6 +403,7 @@ template <typename T, int C>
 struct PairLds {
   typename XLdsOf<T, C>::type x[2];  // one per stage
   Vec<T, C> ring[2][5][64];
+  int go;  // the values of stage 1's first rows are in the divisions' range
 };
 
 // FP32, which has the registers, keeps each slot's y-invariants (WA.., VA..)
@@ -410,12 +411,15 @@ struct PairLds {
 template <typename T>
 constexpr bool kHoldInv = sizeof(T) == 4;
 
-// One step on `rows` rows from row q on, each handed to `out` with its count.
-template <typename T, int EDGE, int C, typename XLds, typename XEdge, typename Div, typename Out>
+// One step on `rows` rows from row q on, each handed to `out` with its count; one
+// row only if a value of the first five raw rows is out of the divisions' range,
+// which `start` is told.
+template <typename T, int EDGE, int C, typename XLds, typename XEdge, typename Div,
+          typename Start, typename Out>
 __device__ __forceinline__ void march_rows(const T *__restrict__ src, int ny, long pitch, long plane,
                                            unsigned boff, int q, int rows, int t, const XEdge &ed,
                                            const SweepCoef<T> &cx, const SweepCoef<T> &cy,
-                                           XLds &lds, Div &dv, Out out) {
+                                           XLds &lds, Div &dv, Start start, Out out) {
   // Slots A/B/D hold the x-swept rows q, q+1, q+2, F the face q-1 | q, wb the
   // invariants of row q-1, N the raw row in flight.  Unrolled three times, so
   // no slot is copied.
@@ -441,6 +445,11 @@ __device__ __forceinline__ void march_rows(const T *__restrict__ src, int ny, lo
       A = B;
       B = D;
       D = u;
+    }
+    if constexpr (Div::kSees) {
+      const bool go = __all(dv.in_range());
+      start(go);
+      if (!go) rows = 1;
     }
     WA = inv_y(A, cy);
     WB = inv_y(B, cy);
@@ -488,14 +497,16 @@ __device__ __forceinline__ void pair_march(const T *__restrict__ src, T *__restr
 #define XS(u) x_sweep(u, lds.x[wave], t, ed, cx, dv)
   if (wave == 0) {
     const unsigned boff = (unsigned)min(max(x, 0), (nx - 1) / C * C) * (unsigned)sizeof(T);
-    march_rows<T, EDGE_CLAMP, C>(src, ny, pitch, plane, boff, j0 - 2, rows, t, ed, cx, cy,
-                                 lds.x[0], dv, [&](int k, const Nodes<T, C> &u) {
-                                   Vec<T, C> out[5];
-                                   pack(u, out);
+    auto start = [&](bool go) { lds.go = go; };  // read behind the first barrier
+    auto put = [&](int k, const Nodes<T, C> &u) {
+      Vec<T, C> out[5];
+      pack(u, out);
 #pragma unroll
-                                   for (int f = 0; f < 5; ++f) lds.ring[k & 1][f][t] = out[f];
-                                   split_sync();
-                                 });
+      for (int f = 0; f < 5; ++f) lds.ring[k & 1][f][t] = out[f];
+      split_sync();
+    };
+    march_rows<T, EDGE_CLAMP, C>(src, ny, pitch, plane, boff, j0 - 2, rows, t, ed, cx, cy,
+                                 lds.x[0], dv, start, put);
   } else {
     // Stage 2: slots A/B/D hold the x-swept time-(n+1) rows r, r+1, r+2, G the
     // face r-1 | r, vb the invariants of row r-1.  Positions above row 0 or
@@ -506,8 +517,7 @@ __device__ __forceinline__ void pair_march(const T *__restrict__ src, T *__restr
     Nodes<T, C> A, B, D, M1, M2;
     Ws<T, C> G, vb, VA, VB, VD;
     int k = 0;
-    auto get = [&](Nodes<T, C> &u) {
-      split_sync();
+    auto take = [&](Nodes<T, C> &u) {
       Vec<T, C> in[5];
 #pragma unroll
       for (int f = 0; f < 5; ++f) in[f] = lds.ring[k & 1][f][t];
@@ -515,7 +525,14 @@ __device__ __forceinline__ void pair_march(const T *__restrict__ src, T *__restr
       u = unpack(in);
       XS(u);
     };
-    get(M2);  // row j0-2
+    auto get = [&](Nodes<T, C> &u) {
+      split_sync();
+      take(u);
+    };
+    split_sync();
+    if constexpr (Div::kSees)
+      if (!__builtin_amdgcn_readfirstlane(lds.go)) return;  // stage 1 ends here too
+    take(M2);  // row j0-2
     get(M1);  // row j0-1
     get(A);   // row j0
     get(B);   // row j0+1
@@ -555,6 +572,12 @@ __device__ __forceinline__ void pair_march(const T *__restrict__ src, T *__restr
 // divisions if it does not meet their conditions (the output of the first
 // march is overwritten; the input is another buffer).  FP64 8192^2 random field 1.55 ms a
 // pass against 1.65, disk 1.24 against 1.34; 2048^2 111 us against 122.
+//
+// The first march ends after its first rows if a value of them is out of range,
+// so a field that is so everywhere costs little more than the IEEE march alone
+// (2048^2 with NaN everywhere 118 us a pass against 214 in two full marches); a
+// tile whose first such value, or whose only zero divisor, is further down
+// costs both.
 template <typename T, int C>
 __device__ __forceinline__ void pair_tile(const T *__restrict__ src, T *__restrict__ dst, int nx,
                                           int ny, long pitch, long plane, int strip, int j0, int j1,
@@ -586,11 +609,11 @@ __device__ __forceinline__ void step_march(const T *__restrict__ src, T *__restr
   const unsigned boff = (unsigned)min(max(x, 0), nx - 1) * (unsigned)sizeof(T);
   const unsigned woff = (unsigned)max(x, 0) * (unsigned)sizeof(T);
   const bool writer = t >= 2 && t < 62 && x < nx;
+  auto put = [&](int k, const Nodes<T, 1> &u) {
+    if (writer) store_nodes<T, 1>(dst + (long)(j0 + k) * pitch, plane, woff, u);
+  };
   march_rows<T, EDGE, 1>(src, ny, pitch, plane, boff, j0, j1 - j0, t, x_edge<1, 2>(x0, nx, t), cx,
-                         cy, lds, dv, [&](int k, const Nodes<T, 1> &u) {
-                           if (writer)
-                             store_nodes<T, 1>(dst + (long)(j0 + k) * pitch, plane, woff, u);
-                         });
+                         cy, lds, dv, [](bool) {}, put);
 }
 
 template <typename T, int EDGE>

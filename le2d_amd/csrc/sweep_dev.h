@@ -119,6 +119,7 @@ struct DivIeee {
   __device__ __forceinline__ T ratio(T n, T d) { return slope_ratio(n, d); }
   __device__ __forceinline__ void see(T, T) {}
   __device__ __forceinline__ void row(const T (&)[5]) {}
+  __device__ __forceinline__ bool in_range() const { return true; }
 };
 
 // FP64 quotients of a tile whose values stay below 2^764: the compiler's IEEE
@@ -174,10 +175,12 @@ struct DivBounded {
     big = mx(hi(u[2]), hi(u[3]), big);
     big = __builtin_elementwise_maximum(__builtin_fabsf(hi(u[4])), big);
   }
+  // high words of 2^300 and 2^-80
+  __device__ __forceinline__ bool in_range() const {
+    return big < __builtin_bit_cast(float, (1023 + 300) << 20);
+  }
   __device__ __forceinline__ bool ok() const {
-    // high words of 2^300 and 2^-80
-    return big < __builtin_bit_cast(float, (1023 + 300) << 20) &&
-           small > __builtin_bit_cast(float, (1023 - 80) << 20);
+    return in_range() && small > __builtin_bit_cast(float, (1023 - 80) << 20);
   }
 };
 
