@@ -91,7 +91,13 @@ int le2d_get_tiles(le_task *task, int *x_rows, int *y_seg, int *y_block, int *xy
  * tasks (with or without a material plane) two steps per kernel pass while
  * at least two remain, `seg` rows per segment; each pass reads and writes
  * every node once for two steps.  Bit-identical to single steps.  seg = 0:
- * one step per pass.  le_step always takes one step. */
+ * one step per pass.  le_step always takes one step.
+ * Grids that do not fill the device run in blocks held in registers: heights of
+ * 4, 8, 16, 24, 32 or 40 rows (FP32 4, 8, 16, 24, 40 or 64) in the 64-column window
+ * name them where at most two such blocks (FP32 four, of 40 rows sixteen) fall to a
+ * compute unit.
+ * Height and window name the whole shape, the default's and the tuner's too, so
+ * setting what was read changes nothing. */
 int le2d_set_step_pairs(le_task *task, int seg);
 int le2d_get_step_pairs(le_task *task, int *seg);
 /* Window of the two-step pass: 64, 128 or 256 columns, of which a workgroup
@@ -105,8 +111,8 @@ int le2d_set_step_pair_split(le_task *task, int on);
 int le2d_get_step_pair_split(le_task *task, int *on);
 /* Time the two-step pass at segment heights 16 .. 160 and those that fill
  * whole rounds of workgroups (4 .. 160 on grids too small to fill the device
- * with 16-row segments) and windows of 64, 128 and (FP32) 256 columns on the
- * task's grid and keep the fastest.  The state does not
+ * with 16-row segments) and windows of 64, 128 and (FP32) 256 columns, and in
+ * blocks of every height, on the task's grid and keep the fastest.  The state does not
  * advance: each candidate reads the current state and writes the idle
  * buffer.  le_step_n does this once per
  * grid shape and process on its first call of 8 or more steps, unless the
@@ -114,6 +120,9 @@ int le2d_get_step_pair_split(le_task *task, int *on);
  * the environment has LE2D_TUNE=0.  A task with a material plane keeps the
  * default window and height. */
 int le2d_tune_step_pairs(le_task *task, int *seg);
+/* Rows that a register block writes in single steps and in two-step passes as
+ * the task is set now; 0: a march. */
+int le2d_get_step_blocks(le_task *task, int *step_rows, int *pair_rows);
 /* Run `passes` two-step passes, timing each launch with HIP events; mean ms
  * of one pass (two steps).  Needs seg > 0 and an ST_AOS task. */
 int le2d_time_pairs(le_task *task, int passes, double *ms_pass);

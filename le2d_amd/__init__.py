@@ -37,6 +37,7 @@ _EXT = {
                           ctypes.POINTER(ctypes.c_double)], ctypes.c_int),
     "le2d_time_steps": (["T", ctypes.c_int, ctypes.POINTER(ctypes.c_double)], ctypes.c_int),
     "le2d_set_step_pairs": (["T", ctypes.c_int], ctypes.c_int),
+    "le2d_get_step_blocks": (["T"] + [ctypes.POINTER(ctypes.c_int)] * 2, ctypes.c_int),
     "le2d_get_step_pairs": (["T", ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
     "le2d_set_step_pair_window": (["T", ctypes.c_int], ctypes.c_int),
     "le2d_get_step_pair_window": (["T", ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
@@ -313,7 +314,7 @@ class Task:
         return a.value
 
     def set_step_pairs(self, seg):
-        """Rows per segment of the two-step pass used by step_n (0: off)."""
+        """Rows per segment, or of a block, of the two-step pass used by step_n (0: off)."""
         self._check(self.lib.le2d_set_step_pairs(self.ref, seg), "set_step_pairs")
 
     def set_step_pair_window(self, lanes):
@@ -348,6 +349,13 @@ class Task:
         v = ctypes.c_int()
         self._check(self.lib.le2d_get_step_pairs(self.ref, ctypes.byref(v)), "get_step_pairs")
         return v.value
+
+    def get_step_blocks(self):
+        """Rows of the register blocks of single steps and of two-step passes (0: a march)."""
+        v = [ctypes.c_int() for _ in range(2)]
+        self._check(self.lib.le2d_get_step_blocks(self.ref, *[ctypes.byref(x) for x in v]),
+                    "get_step_blocks")
+        return tuple(x.value for x in v)
 
     def time_pairs(self, passes):
         """Mean ms of one two-step pass (HIP events)."""

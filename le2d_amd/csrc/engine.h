@@ -46,11 +46,14 @@ struct Tiles {
   int y_block;  // columns per y-sweep workgroup (64, 128 or 256)
   int xy_seg;   // rows per segment of the fused x+y step
   int xy_block; // lanes per fused-step workgroup (64, 128, 256); writes xy_block-4 columns
-  int pair_seg; // rows per segment of the two-step pass (0: one step per pass)
-  int pair_block; // window of the two-step pass: 64, 128 or 256 columns (pair_cols)
+  // two-step pass (set_pair_shape): rows per segment (0: one step per pass), window of
+  // 64, 128 or 256 columns (pair_cols), and the rows of the blocks that this
+  // shape runs in (pair_block_rows; 0: the march)
+  int pair_seg;
+  int pair_block;
+  int block_rows = 0;
   bool x_fixed = false;  // x_rows is the caller's
   int step_rows = 0;  // fused step in blocks that write this many rows (0: the march of xy_seg)
-  int block_rows = 0; // two-step pass in blocks that write this many rows (0: the march)
   int pair_split = 0; // a caller's setting that is kept and reported; every window runs its
                       // two stages on two wavefronts
 };
@@ -125,6 +128,12 @@ int step2_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy);
 int copy_probe(size_t bytes, int iters, double *ms);
 
 Tiles default_tiles(int elem, int nx, int ny);
+// Rows of the register blocks (block_dev.h) that a two-step pass over an nx x ny
+// grid runs in with this window and segment height, 0 for the march.  A height and
+// a window name one form on every task of a grid, so a shape that was read can be
+// set again, also by another process.
+int pair_block_rows(int elem, int nx, int ny, int window, int seg);
+void set_pair_shape(DevGrid *g, int window, int seg);
 // Columns that a two-step window setting of 64, 128 or 256 runs in (of which
 // 8 are halo): FP64 at most 128, as two columns per lane fill the registers.
 inline int pair_cols(int elem, int window) {

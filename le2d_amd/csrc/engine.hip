@@ -279,6 +279,7 @@ int grid_aos_image(DevGrid *g, void **image) {
 
 static int step_blocks(int elem, int nx, int ny);
 static int step_segment(int nx, int ny);
+static long pair_blocks(int nx, int ny, int rows);
 
 Tiles default_tiles(int elem, int nx, int ny) {
   Tiles t;
@@ -312,20 +313,51 @@ Tiles default_tiles(int elem, int nx, int ny) {
   t.y_seg = std::min(4, ny);  // one group of rows (kYRows in sweep.hip)
   const GridSize size{nx, ny};
   const PairShape p = pick_pair_shape(elem, &size, 1, 0, 192);
-  t.pair_block = p.window;
-  t.pair_seg = p.seg;
+  int window = p.window, seg = p.seg;
   // blocks where each has a compute unit to itself, of the fewest rows that give
   // that (block_dev.h has both sides' times); in FP32, where several share one, also
   // blocks of 40 rows on grids of up to 16 for each (us a pass, blocks against the
   // march at its default shape: 2500 x 1500 41.2 and 45.1, 2961 x 2216 64.9 and 70.2,
   // 3500 x 2500, 15.5 for each, 89.8 and 95.5; against the march's fastest shape 1200^2
   // 21.0 and 23.2, 2048^2 43.5 and 43.0)
-  auto blocks = [&](int rows) { return (long)((nx + 55) / 56) * ((ny + rows - 1) / rows); };
-  t.block_rows = 0;
-  for (int k = 0; k < kBlockKinds && !t.block_rows; ++k)
-    if (blocks(block_rows(elem, k)) <= device_cus()) t.block_rows = block_rows(elem, k);
-  if (elem == 4 && !t.block_rows && blocks(40) <= 16 * device_cus()) t.block_rows = 40;
+  int rows = 0;
+  for (int k = 0; k < kBlockKinds && !rows; ++k)
+    if (pair_blocks(nx, ny, block_rows(elem, k)) <= device_cus()) rows = block_rows(elem, k);
+  if (elem == 4 && !rows && pair_blocks(nx, ny, 40) <= 16 * device_cus()) rows = 40;
+  if (rows) {
+    window = 64;
+    seg = rows;
+  }
+  t.pair_block = window;
+  t.pair_seg = seg;
+  t.block_rows = pair_block_rows(elem, nx, ny, window, seg);
   return t;
+}
+
+static long pair_blocks(int nx, int ny, int rows) {
+  return (long)((nx + 55) / 56) * ((ny + rows - 1) / rows);
+}
+
+// A block height in the 64-column window, on grids of up to two such blocks for each
+// compute unit, in FP32 up to four, of 40 rows up to sixteen: there blocks are no
+// slower than a march of that height (us a pass, blocks of so many rows and so
+// many for each unit against marches one row lower and higher: FP64 900^2 32, 1.9:
+// 37 and 47, 49; FP32 1500 x 1001 24, 4.4: 23.0 and 26.0, 27.1, but 2500 x 1500 24, 11:
+// 50 and 45, 44 and 64, 4.2: 55 and 52, 53; 40, 6.7: 43.0 and 43.9, 45.2).
+int pair_block_rows(int elem, int nx, int ny, int window, int seg) {
+  if (window != 64) return 0;
+  for (int k = 0; k < kBlockKinds; ++k)
+    if (block_rows(elem, k) == seg) {
+      const int each = elem == 8 ? 2 : seg == 40 ? 16 : 4;
+      return pair_blocks(nx, ny, seg) <= each * device_cus() ? seg : 0;
+    }
+  return 0;
+}
+
+void set_pair_shape(DevGrid *g, int window, int seg) {
+  g->tiles.pair_block = window;
+  g->tiles.pair_seg = seg;
+  g->tiles.block_rows = pair_block_rows(g->elem, g->nx, g->ny, window, seg);
 }
 
 // Rows of the single step's blocks, 0 for the march.  The lowest blocks of which every

@@ -55,7 +55,7 @@ std::unordered_map<const real *, TaskState *> g_tasks;
 // tuned two-step segment heights and windows per (element size, nx, ny), for
 // the process
 std::mutex g_pair_mu;
-std::map<std::tuple<int, int, int>, std::tuple<int, int, int>> g_pair_seg;  // rows, window, block
+std::map<std::tuple<int, int, int>, le2d::PairShape> g_pair_seg;
 
 int env_mode() {
   const char *s = getenv("LE2D_SYNC");
@@ -167,9 +167,7 @@ int tune_pairs(le_task *t, TaskState *s) {
     std::lock_guard<std::mutex> lk(g_pair_mu);
     auto it = g_pair_seg.find(key);
     if (it != g_pair_seg.end()) {
-      s->g.tiles.pair_seg = std::get<0>(it->second);
-      s->g.tiles.pair_block = std::get<1>(it->second);
-      s->g.tiles.block_rows = std::get<2>(it->second);
+      le2d::set_pair_shape(&s->g, it->second.window, it->second.seg);
       s->pairs_fixed = true;
       return LE2D_OK;
     }
@@ -179,12 +177,9 @@ int tune_pairs(le_task *t, TaskState *s) {
   hipEvent_t ev[2];
   for (auto &e : ev) (void)hipEventCreate(&e);
   int rc = LE2D_OK;
-  // mean ms of one pass at (block, seg), or in blocks of `rows` rows, after one
-  // untimed pass; < 0 on error
-  auto time_one = [&](int block, int seg, int rows, int reps) -> float {
-    s->g.tiles.pair_seg = seg;
-    s->g.tiles.pair_block = block;
-    s->g.tiles.block_rows = rows;
+  // mean ms of one pass at (block, seg) after one untimed pass; < 0 on error
+  auto time_one = [&](int block, int seg, int reps) -> float {
+    le2d::set_pair_shape(&s->g, block, seg);
     for (int k = 0; k <= reps && !rc; ++k) {
       if (k == 1) (void)hipEventRecord(ev[0], s->stream);
       rc = le2d::step2_xy<real>(&s->g, cx, cy);
@@ -206,11 +201,11 @@ int tune_pairs(le_task *t, TaskState *s) {
   // warm-up at the default shape, about 25 ms: after host-side work the
   // device clocks are still low and would make the first candidates look slow
   {
-    const int b0 = s->g.tiles.pair_block, s0 = s->g.tiles.pair_seg, r0 = s->g.tiles.block_rows;
-    const float est = time_one(b0, s0, r0, 1);
+    const int b0 = s->g.tiles.pair_block, s0 = s->g.tiles.pair_seg;
+    const float est = time_one(b0, s0, 1);
     if (est > 0) {
       const int reps = std::max(1, std::min(64, (int)(25.0f / est)));
-      (void)time_one(b0, s0, r0, reps);
+      (void)time_one(b0, s0, reps);
     }
   }
   std::vector<Cand> res;
@@ -233,7 +228,7 @@ int tune_pairs(le_task *t, TaskState *s) {
         if (seg >= 16 && seg <= s->g.ny && !std::count(segs.begin(), segs.end(), seg))
           segs.push_back(seg);
     for (int seg : segs) {
-      const float ms = time_one(block, seg, 0, 4);
+      const float ms = time_one(block, seg, 4);
       if (ms < 0) break;
       res.push_back({ms, block, seg});
     }
@@ -243,33 +238,27 @@ int tune_pairs(le_task *t, TaskState *s) {
     std::sort(res.begin(), res.end(), [](const Cand &a, const Cand &b) { return a.ms < b.ms; });
     if (res.size() > 3) res.resize(3);
     for (const Cand &c : res) {
-      const float ms = time_one(c.block, c.seg, 0, 12);
+      const float ms = time_one(c.block, c.seg, 12);
       if (ms < 0) break;
       if (ms < best.ms) best = {ms, c.block, c.seg};
     }
   }
-  // blocks, up to two for each compute unit (FP32 16), against the fastest march
-  int rows = 0;
+  // every block height that the grid runs in, against the fastest of those
   for (int k = 0; k < le2d::kBlockKinds && !rc && best.ms < 1e30f; ++k) {
     const int r = le2d::block_rows((int)sizeof(real), k);
-    const long n = (long)((s->g.nx + 55) / 56) * ((s->g.ny + r - 1) / r);
-    if (n > (sizeof(real) == 4 ? 16 : 2) * le2d::device_cus()) continue;
-    const float ms = time_one(best.block, best.seg, r, 12);
+    if (!le2d::pair_block_rows((int)sizeof(real), s->g.nx, s->g.ny, 64, r)) continue;
+    const float ms = time_one(64, r, 12);
     if (ms < 0) break;
-    if (ms < best.ms) {
-      best.ms = ms;
-      rows = r;
-    }
+    if (ms < best.ms) best = {ms, 64, r};
+    const long n = (long)((s->g.nx + 55) / 56) * ((s->g.ny + r - 1) / r);
     if (2 * n < le2d::device_cus()) break;  // taller ones leave more of the device idle
   }
   for (auto &e : ev) (void)hipEventDestroy(e);
-  s->g.tiles.pair_seg = best.seg;
-  s->g.tiles.pair_block = best.block;
-  s->g.tiles.block_rows = rows;
+  le2d::set_pair_shape(&s->g, best.block, best.seg);
   s->pairs_fixed = true;
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(g_pair_mu);
-  g_pair_seg[key] = {best.seg, best.block, rows};
+  g_pair_seg[key] = {best.block, best.seg};
   return LE2D_OK;
 }
 
@@ -714,8 +703,7 @@ int le2d_set_step_pairs(le_task *task, int seg) {
   int rc = ensure_device(task, s);
   if (rc) return rc;
   if (seg < 0) return le2d::set_error(LE2D_ERR_ARG, "step pairs: segment %d", seg);
-  s->g.tiles.pair_seg = seg;
-  s->g.tiles.block_rows = 0;  // a height is the march's
+  le2d::set_pair_shape(&s->g, s->g.tiles.pair_block, seg);
   s->pairs_fixed = true;
   return LE2D_OK;
 }
@@ -724,7 +712,7 @@ int le2d_tune_step_pairs(le_task *task, int *seg) {
   TaskState *s = find(task);
   int rc = ensure_device(task, s);
   if (rc) return rc;
-  if (s->g.tiles.pair_seg < 1) s->g.tiles.pair_seg = 64;
+  if (s->g.tiles.pair_seg < 1) le2d::set_pair_shape(&s->g, s->g.tiles.pair_block, 64);
   s->pairs_fixed = false;
   {
     std::lock_guard<std::mutex> lk(g_pair_mu);
@@ -742,8 +730,7 @@ int le2d_set_step_pair_window(le_task *task, int lanes) {
   if (rc) return rc;
   if (lanes != 64 && lanes != 128 && lanes != 256)
     return le2d::set_error(LE2D_ERR_ARG, "step pairs: window %d", lanes);
-  s->g.tiles.pair_block = lanes;
-  s->g.tiles.block_rows = 0;  // a window is the march's
+  le2d::set_pair_shape(&s->g, lanes, s->g.tiles.pair_seg);
   s->pairs_fixed = true;
   return LE2D_OK;
 }
@@ -779,6 +766,15 @@ int le2d_get_step_pairs(le_task *task, int *seg) {
   int rc = ensure_device(task, s);
   if (rc) return rc;
   *seg = s->g.tiles.pair_seg;
+  return LE2D_OK;
+}
+
+int le2d_get_step_blocks(le_task *task, int *step_rows, int *pair_rows) {
+  TaskState *s = find(task);
+  int rc = ensure_device(task, s);
+  if (rc) return rc;
+  *step_rows = s->g.tiles.step_rows;
+  *pair_rows = s->g.tiles.block_rows;
   return LE2D_OK;
 }
 
@@ -820,11 +816,15 @@ int le2d_set_material_plane(le_task *task, int count, const double *c1_c2_rho,
     // halo columns (4100 x 3000 FP64 402 us a pass against 425 at 128, FP32
     // 147 against 168 at 256).
     const le2d::GridSize g{s->g.nx, s->g.ny};
-    const int only = count > 0 && (long)g.nx * g.ny < (1L << 26) ? 64 : 0;
-    const int cap = only || (count > 0 && sizeof(real) == 4) ? 64 : 192;
-    const le2d::PairShape p = le2d::pick_pair_shape((int)sizeof(real), &g, 1, only, cap);
-    s->g.tiles.pair_block = p.window;
-    s->g.tiles.pair_seg = p.seg;
+    if (count > 0) {
+      const int only = (long)g.nx * g.ny < (1L << 26) ? 64 : 0;
+      const int cap = only || sizeof(real) == 4 ? 64 : 192;
+      const le2d::PairShape p = le2d::pick_pair_shape((int)sizeof(real), &g, 1, only, cap);
+      le2d::set_pair_shape(&s->g, p.window, p.seg);
+    } else {
+      const le2d::Tiles d = le2d::default_tiles((int)sizeof(real), g.nx, g.ny);
+      le2d::set_pair_shape(&s->g, d.pair_block, d.pair_seg);
+    }
   }
   if (count == 0) {
     le2d::mat_release(&s->mat);

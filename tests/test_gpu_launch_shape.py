@@ -1,0 +1,64 @@
+"""A launch shape that was read and is set again, on the same task or on another of
+that grid, runs in the form it ran in: register blocks or a march, as the default
+or the tuner chose.  The forms expected of each grid assume 256 compute units."""
+import numpy as np
+import pytest
+
+import golden_data as gd
+import le2d_amd
+
+pytestmark = pytest.mark.gpu
+ARGS = (0.2, (1.0, 0.9), (2.0, 1.0, 1.5))
+F8, F4 = np.float64, np.float32
+# grid -> rows of the default two-step blocks (0: a march)
+PAIRS = {(F8, 96, 80): 4, (F8, 250, 300): 8, (F8, 400, 500): 16, (F8, 512, 512): 24,
+         (F8, 620, 640): 32, (F8, 724, 724): 40, (F8, 900, 900): 0, (F8, 2048, 1000): 0,
+         (F4, 96, 80): 4, (F4, 250, 300): 8, (F4, 400, 500): 16, (F4, 512, 512): 24,
+         (F4, 1031, 517): 40, (F4, 900, 900): 64, (F4, 1500, 1001): 40, (F4, 4200, 3000): 0}
+
+
+def _task(dtype, nx, ny):
+    return le2d_amd.Task(nx, ny, *ARGS, dtype=dtype)
+
+
+def _pairs(t):
+    return t.get_step_pairs(), t.get_step_pair_window(), t.get_step_blocks()[1]
+
+
+@pytest.mark.parametrize("dtype,nx,ny", PAIRS)
+def test_default_pair_shape(dtype, nx, ny):
+    rows = PAIRS[dtype, nx, ny]
+    with _task(dtype, nx, ny) as t:
+        shape = _pairs(t)
+        assert shape[2] == rows
+        assert not rows or shape[:2] == (rows, 64)
+        t.set_step_pairs(shape[0])
+        t.set_step_pair_window(shape[1])
+        assert _pairs(t) == shape
+
+
+@pytest.mark.parametrize("dtype,nx,ny", [(F8, 512, 512), (F8, 900, 900), (F4, 1031, 517)])
+def test_tuned_pair_shape(dtype, nx, ny):
+    with _task(dtype, nx, ny) as t:
+        assert t.tune_step_pairs() == t.get_step_pairs()
+        shape = _pairs(t)
+    with _task(dtype, nx, ny) as t:
+        t.set_step_pair_window(shape[1])
+        t.set_step_pairs(shape[0])
+        assert _pairs(t) == shape
+
+
+@pytest.mark.parametrize("dtype,heights", [(F8, (4, 8, 16, 24, 32, 40)), (F4, (4, 8, 16, 24, 40, 64))])
+def test_heights_name_blocks(dtype, heights):
+    """Every block height set by hand, a march one row higher and one in another window."""
+    g0 = np.random.default_rng(4).standard_normal((150, 313, 5)).astype(dtype)
+    out = []
+    for seg, window, rows in [(h, 64, h) for h in heights] + [(17, 64, 0), (16, 128, 0)]:
+        with _task(dtype, 313, 150) as t:
+            t.load(g0)
+            t.set_step_pairs(seg)
+            t.set_step_pair_window(window)
+            assert _pairs(t) == (seg, window, rows)
+            t.step_n(4)
+            out.append(t.grid().copy())
+    assert all(gd.same_bits(g, out[0]) for g in out[1:])
