@@ -80,9 +80,11 @@ int le_step_n(le_task *task, int steps);
 /* Launch shape: rows per x-sweep workgroup, rows per y-sweep segment,
  * columns per y-sweep workgroup (64, 128, 256), rows per segment of the fused
  * step, lanes per fused-step workgroup (64, 128, 256; it writes that many
- * columns less four).  Zero keeps the current value.  Setting the rows of the
- * x-sweep, or either of the last two, also selects the kernel form that has them
- * (the default may be another).  Results do not depend on the shape. */
+ * columns less four).  Zero keeps the current value.  The values that a new task
+ * of the grid reports select the default kernel forms (which may be others, see
+ * le2d_get_step_blocks); rows of the x-sweep, or either of the last two, that
+ * differ from them select the form that has them.  Results do not depend on the
+ * shape. */
 int le2d_set_tiles(le_task *task, int x_rows, int y_seg, int y_block, int xy_seg, int xy_block);
 int le2d_get_tiles(le_task *task, int *x_rows, int *y_seg, int *y_block, int *xy_seg,
                    int *xy_block);

@@ -41,7 +41,7 @@ struct SweepCoef {
 
 // Launch shape of the sweeps (chosen per grid by the autotuner).
 struct Tiles {
-  int x_rows;   // rows per x-sweep workgroup (used where x_fixed, and in FP32 on large grids)
+  int x_rows;   // rows per workgroup of k_sweep_x (sweep_x has where it runs)
   int y_seg;    // rows per y-sweep segment (every kYRows of them re-read 4 halo rows)
   int y_block;  // columns per y-sweep workgroup (64, 128 or 256)
   int xy_seg;   // rows per segment of the fused x+y step
@@ -52,7 +52,7 @@ struct Tiles {
   int pair_seg;
   int pair_block;
   int block_rows = 0;
-  bool x_fixed = false;  // x_rows is the caller's
+  bool x_fixed = false;  // x_rows is a caller's, not the default
   int step_rows = 0;  // fused step in blocks that write this many rows (0: the march of xy_seg)
   int pair_split = 0; // a caller's setting that is kept and reported; every window runs its
                       // two stages on two wavefronts

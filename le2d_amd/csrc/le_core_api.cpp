@@ -647,15 +647,16 @@ int le2d_set_tiles(le_task *task, int x_rows, int y_seg, int y_block, int xy_seg
   if (x_rows < 0 || y_seg < 0 || xy_seg < 0 || !width_ok(y_block) || !width_ok(xy_block))
     return le2d::set_error(LE2D_ERR_ARG, "tiles %d %d %d %d %d", x_rows, y_seg, y_block, xy_seg,
                            xy_block);
-  if (x_rows) {
-    s->g.tiles.x_rows = x_rows;
-    s->g.tiles.x_fixed = true;
-  }
-  if (y_seg) s->g.tiles.y_seg = y_seg;
-  if (y_block) s->g.tiles.y_block = y_block;
-  if (xy_seg) s->g.tiles.xy_seg = xy_seg;
-  if (xy_block) s->g.tiles.xy_block = xy_block;
-  if (xy_seg || xy_block) s->g.tiles.step_rows = 0;  // the march of that shape
+  le2d::Tiles &t = s->g.tiles;
+  if (x_rows) t.x_rows = x_rows;
+  if (y_seg) t.y_seg = y_seg;
+  if (y_block) t.y_block = y_block;
+  if (xy_seg) t.xy_seg = xy_seg;
+  if (xy_block) t.xy_block = xy_block;
+  // the default's values name the default's forms, others the form that has them
+  const le2d::Tiles d = le2d::default_tiles((int)sizeof(real), s->g.nx, s->g.ny);
+  t.x_fixed = t.x_rows != d.x_rows;
+  t.step_rows = t.xy_seg == d.xy_seg && t.xy_block == d.xy_block ? d.step_rows : 0;
   return LE2D_OK;
 }
 

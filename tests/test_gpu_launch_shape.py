@@ -1,5 +1,5 @@
 """A launch shape that was read and is set again, on the same task or on another of
-that grid, runs in the form it ran in: register blocks or a march, as the default
+its grid, runs in the form it ran in: register blocks or a march, as the default
 or the tuner chose.  The forms expected of each grid assume 256 compute units."""
 import numpy as np
 import pytest
@@ -62,3 +62,27 @@ def test_heights_name_blocks(dtype, heights):
             t.step_n(4)
             out.append(t.grid().copy())
     assert all(gd.same_bits(g, out[0]) for g in out[1:])
+
+
+@pytest.mark.parametrize("dtype,nx,ny,rows", [
+    (F8, 96, 80, 4), (F8, 300, 250, 12), (F8, 512, 512, 20), (F8, 900, 900, 0), (F8, 2400, 1930, 24),
+    (F4, 512, 512, 20), (F4, 1500, 1001, 20), (F4, 8192, 2049, 44)])
+def test_tiles(dtype, nx, ny, rows):
+    with _task(dtype, nx, ny) as t:
+        tiles = t.get_tiles()
+        assert t.get_step_blocks()[0] == rows
+        t.set_tiles(xy_seg=tiles[3] + 1)
+        assert t.get_step_blocks()[0] == 0
+        t.set_tiles(*tiles)
+        assert t.get_tiles() == tiles and t.get_step_blocks()[0] == rows
+
+
+def test_x_sweep_form():
+    """The default rows keep the wavefront form (FP64 512^2: 8.3 us a sweep, 12.6 in
+    whole workgroups; 1.25 is midway)."""
+    with _task(F8, 512, 512) as t:
+        t.time_sweeps(50)
+        before = min(t.time_sweeps(20)[0] for _ in range(9))
+        t.set_tiles(*t.get_tiles())
+        after = min(t.time_sweeps(20)[0] for _ in range(9))
+    assert after < 1.25 * before
