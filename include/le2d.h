@@ -233,7 +233,10 @@ int le2d_batch_wait(le2d_batch *b);
  * LE2D_BATCH_TILES, one workgroup per tile; LE2D_BATCH_PERSISTENT, resident
  * workgroups walk the tile table; LE2D_BATCH_PAIRS, one workgroup per tile
  * and two steps per launch (an odd step count ends with one single-step
- * launch); LE2D_BATCH_PAIRS_SPLIT, the same with windows of 64 columns.  All forms
+ * launch); LE2D_BATCH_PAIRS_SPLIT, the same with windows of 64 columns.  In
+ * LE2D_BATCH_PAIRS heights of 8, 16, 24 or 32 rows (FP32 8, 16, 24 or 40) in 64-column
+ * windows name register blocks where every block of the batch has a compute unit
+ * to itself; le2d_batch_get_blocks: their rows as set now, 0 for a march.  All forms
  * give the same results. */
 #define LE2D_BATCH_TILES 0
 #define LE2D_BATCH_PERSISTENT 1
@@ -242,6 +245,7 @@ int le2d_batch_wait(le2d_batch *b);
 int le2d_batch_set_shape(le2d_batch *b, int fb, int seg);
 int le2d_batch_set_launch(le2d_batch *b, int fb, int seg, int form);
 int le2d_batch_get_launch(le2d_batch *b, int *form);
+int le2d_batch_get_blocks(le2d_batch *b, int *rows);
 int le2d_batch_get_shape(le2d_batch *b, int *fb, int *seg, int *ntiles, int *blocks);
 /* Mean ms per step of `steps` batched (plain = 0) or per-instance (plain = 1)
  * steps, HIP events on the batch's stream. */

@@ -102,6 +102,7 @@ _BATCH = {
     "le2d_batch_wait": ([_VP], ctypes.c_int),
     "le2d_batch_set_shape": ([_VP, ctypes.c_int, ctypes.c_int], ctypes.c_int),
     "le2d_batch_set_launch": ([_VP, ctypes.c_int, ctypes.c_int, ctypes.c_int], ctypes.c_int),
+    "le2d_batch_get_blocks": ([_VP, _IP], ctypes.c_int),
     "le2d_batch_get_launch": ([_VP, _IP], ctypes.c_int),
     "le2d_batch_get_shape": ([_VP, _IP, _IP, _IP, _IP], ctypes.c_int),
     "le2d_batch_time": ([_VP, ctypes.c_int, ctypes.c_int, _DP], ctypes.c_int),
@@ -482,6 +483,12 @@ class Batch:
         v = ctypes.c_int()
         self._check(self.lib.le2d_batch_get_launch(self.h, ctypes.byref(v)), "get_launch")
         return {n: k for k, n in self.FORMS.items()}[v.value]
+
+    def get_blocks(self):
+        """Rows of the two-step launches' register blocks (0: a march)."""
+        v = ctypes.c_int()
+        self._check(self.lib.le2d_batch_get_blocks(self.h, ctypes.byref(v)), "get_blocks")
+        return v.value
 
     def get_shape(self):
         v = [ctypes.c_int() for _ in range(4)]

@@ -49,7 +49,8 @@ struct Shape {
              // workgroups walk the table; FORM_PAIRS: one workgroup per tile of
              // the two-step table, two steps per launch, in windows of 64, 128
              // or 256 columns; FORM_PAIRS_SPLIT: the same in windows of 64
-  int rows = 0;  // FORM_PAIRS: blocks of this many rows (fb 64, seg rows), 0: the march
+  int rows = 0;  // FORM_PAIRS: blocks of this many rows (build_tiles: batch_block_rows_at
+                 // of fb 64 and seg), 0: the march
 };
 
 std::mutex g_tune_mu;
@@ -110,6 +111,22 @@ struct BatchImpl {
     long n = 0;
     for (const Inst &in : inst) n += (long)in.nx * in.ny;
     return n;
+  }
+
+  std::vector<GridSize> sizes() const {
+    std::vector<GridSize> g;
+    for (const Inst &in : inst) g.push_back({in.nx, in.ny});
+    return g;
+  }
+
+  // The two-step form in blocks, or in the window and segment height that the model
+  // of the single-grid pass gives for all instances together.
+  Shape default_shape() const {
+    const std::vector<GridSize> g = sizes();
+    if (const int rows = batch_block_rows(elem, g.data(), g.size(), 160))
+      return {64, rows, FORM_PAIRS};
+    const PairShape p = pick_pair_shape(elem, g.data(), g.size(), 0, 160);
+    return {p.window, p.seg, FORM_PAIRS};
   }
 
   DevGrid view(int i) {
@@ -176,6 +193,10 @@ struct BatchImpl {
   int build_tiles(Shape s) {
     if (s.form == FORM_PAIRS && s.fb != 64 && s.fb != 128) s.fb = 256;
     if (s.form == FORM_PAIRS_SPLIT) s.fb = 64;
+    const std::vector<GridSize> g = sizes();
+    s.rows = s.form == FORM_PAIRS && s.fb == 64
+                 ? batch_block_rows_at(elem, g.data(), g.size(), s.seg)
+                 : 0;
     int rc = upload_table(two_step(s.form) ? pair_cols(elem, s.fb) - 8 : s.fb - 4, s.seg, &d_tiles,
                           &ntiles);
     if (rc) return rc;
@@ -363,15 +384,8 @@ int le2d_batch_commit(le2d_batch *b) {
   if (rc) return rc;
   rc = B.elem == 8 ? B.upload_desc<double>() : B.upload_desc<float>();
   if (rc) return rc;
-  // default shape until autotuned: the cached winner for this batch, else
-  // the two-step form in the window and segment height that the model of the
-  // single-grid pass gives for all instances together
-  std::vector<le2d::GridSize> sizes;
-  for (const auto &in : B.inst) sizes.push_back({in.nx, in.ny});
-  const le2d::PairShape p = le2d::pick_pair_shape(B.elem, sizes.data(), sizes.size(), 0, 160);
-  le2d::Shape s{p.window, p.seg, le2d::FORM_PAIRS};
-  if (const int rows = le2d::batch_block_rows(B.elem, sizes.data(), sizes.size(), 160))
-    s = {64, rows, le2d::FORM_PAIRS, rows};
+  // default shape until autotuned, or the cached winner for such a batch
+  le2d::Shape s = B.default_shape();
   {
     std::lock_guard<std::mutex> lk(le2d::g_tune_mu);
     auto it = le2d::g_tune.find({B.elem, (int)B.inst.size(), B.total_nodes() >> 20});
@@ -471,6 +485,12 @@ int le2d_batch_get_launch(le2d_batch *b, int *form) {
   return le2d::OK;
 }
 
+int le2d_batch_get_blocks(le2d_batch *b, int *rows) {
+  if (!b || !rows) return le2d::ERR_ARG;
+  *rows = b->impl.shape.rows;
+  return le2d::OK;
+}
+
 int le2d_batch_set_shape(le2d_batch *b, int fb, int seg) {
   if (!b) return le2d::ERR_ARG;
   return le2d_batch_set_launch(b, fb, seg, b->impl.shape.form);
@@ -509,9 +529,9 @@ int le2d_batch_time(le2d_batch *b, int steps, int plain, double *ms) {
 
 // Times every candidate shape and keeps the fastest (per step): the
 // single-step forms at every window width and segment height, and the
-// two-step form at every segment height, and the default if that is in blocks.  Stepping the batch is part of
-// tuning: the instances advance by an even number of steps per candidate,
-// so callers tune before loading their initial state or account for it.
+// two-step form at every segment height, and the default if that is in blocks.  Stepping the batch is part of tuning: the instances advance
+// by an even number of steps per candidate, so callers tune before loading their
+// initial state or account for it.
 int le2d_batch_autotune(le2d_batch *b, int trials, int *best_fb, int *best_seg, double *best_ms) {
   if (!b || !b->impl.committed || trials < 1) return le2d::ERR_ARG;
   BatchImpl &B = b->impl;

@@ -130,13 +130,23 @@ inline BatchPairKernel<T> batch_pair_kernel(int cols, int rows) {
 // blocks: FP32 110 and 96, FP64 183 and 152).  More blocks than that are no faster
 // than the march, FP32 either (48 of 128 to 1024 997 and 999, 12 of 128 to 300 178
 // and 175): on many grids their last strips and rows are a larger share.
+inline bool batch_blocks_fit(const GridSize *g, size_t n, int rows) {
+  long blocks = 0;
+  for (size_t i = 0; i < n; ++i)
+    blocks += (long)((g[i].nx + 55) / 56) * ((g[i].ny + rows - 1) / rows);
+  return blocks <= device_cus();
+}
 inline int batch_block_rows(int elem, const GridSize *g, size_t n, int cap) {
-  for (int rows : {8, 16, 24, elem == 8 ? 32 : 40}) {
-    long blocks = 0;
-    for (size_t i = 0; i < n; ++i)
-      blocks += (long)((g[i].nx + 55) / 56) * ((g[i].ny + rows - 1) / rows);
-    if (rows <= cap && blocks <= device_cus()) return rows;
-  }
+  for (int rows : {8, 16, 24, elem == 8 ? 32 : 40})
+    if (rows <= cap && batch_blocks_fit(g, n, rows)) return rows;
+  return 0;
+}
+// Rows of the blocks that a launch in 64-column windows and segments of `seg` rows
+// runs in, 0 for the march: height and window name the form (as pair_block_rows
+// does for one grid), so that a shape that was read can be set again.
+inline int batch_block_rows_at(int elem, const GridSize *g, size_t n, int seg) {
+  for (int rows : {8, 16, 24, elem == 8 ? 32 : 40})
+    if (rows == seg && batch_blocks_fit(g, n, rows)) return rows;
   return 0;
 }
 

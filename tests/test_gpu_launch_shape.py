@@ -86,3 +86,26 @@ def test_x_sweep_form():
         t.set_tiles(*t.get_tiles())
         after = min(t.time_sweeps(20)[0] for _ in range(9))
     assert after < 1.25 * before
+
+
+def _batch(dtype, sizes):
+    b = le2d_amd.Batch(dtype)
+    for nx, ny in sizes:
+        b.add(nx, ny, *ARGS)
+    b.commit()
+    return b
+
+
+@pytest.mark.parametrize("dtype,rows,sizes", [
+    (F8, 8, [(200, 170), (113, 121), (57, 9)]), (F8, 24, [(500, 400), (301, 241)]),
+    (F4, 40, [(640, 512), (57, 41)]), (F8, 0, [(900, 700), (57, 41)])])
+def test_batch_shape(dtype, rows, sizes):
+    with _batch(dtype, sizes) as b:
+        shape, form = b.get_shape(), b.form()
+        assert b.get_blocks() == rows
+        b.set_shape(128, 16, "tiles")
+        assert b.get_blocks() == 0
+        b.set_shape(shape[0], shape[1], form)
+        assert b.get_shape() == shape and b.get_blocks() == rows
+        b.set_shape(shape[0], shape[1])
+        assert b.get_shape() == shape and b.get_blocks() == rows
