@@ -250,8 +250,10 @@ int le2d_batch_get_shape(le2d_batch *b, int *fb, int *seg, int *ntiles, int *blo
 /* Mean ms per step of `steps` batched (plain = 0) or per-instance (plain = 1)
  * steps, HIP events on the batch's stream. */
 int le2d_batch_time(le2d_batch *b, int steps, int plain, double *ms);
-/* Times each window width x segment height on the batch and keeps the
- * fastest (remembered per element size, instance count and node total).
+/* Times each window width x segment height on the batch and the default shape, and
+ * keeps the fastest (remembered per element size, instance count and class of
+ * the node total; a height that named blocks is taken by another batch only
+ * where it names them there too).
  * Advances the instances by an even number of steps. */
 int le2d_batch_autotune(le2d_batch *b, int trials, int *best_fb, int *best_seg, double *best_ms);
 /* View of instance `inst`'s current state (see le2d_view). */

@@ -13,7 +13,7 @@
 // The launch shape -- window width (64, 128 or 256 lanes), rows per segment,
 // and the launch form -- is chosen by le2d_batch_autotune, which times candidate shapes
 // on the batch itself and keeps the fastest (per element size, instance
-// count and node total, for the life of the process).
+// count and class of the node total, for the life of the process).
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -54,7 +54,8 @@ struct Shape {
 };
 
 std::mutex g_tune_mu;
-std::map<std::tuple<int, int, long>, Shape> g_tune;  // (elem, instances, Mnodes) -> shape
+// tuned shapes by element size, instances and size class (tune_key)
+std::map<std::tuple<int, int, long>, Shape> g_tune;
 
 template <typename T>
 void inst_coef(const Inst &in, SweepCoef<T> *cx, SweepCoef<T> *cy) {
@@ -127,6 +128,13 @@ struct BatchImpl {
       return {64, rows, FORM_PAIRS};
     const PairShape p = pick_pair_shape(elem, g.data(), g.size(), 0, 160);
     return {p.window, p.seg, FORM_PAIRS};
+  }
+
+  // Batches of a key share a tuned shape.  Size class: the total in units of 2^20
+  // nodes, below that quarter octaves (as negative numbers).
+  std::tuple<int, int, long> tune_key() const {
+    const long n = total_nodes();
+    return {elem, (int)inst.size(), n >> 20 ? n >> 20 : (long)(4 * std::log2((double)n)) - 100};
   }
 
   DevGrid view(int i) {
@@ -386,10 +394,15 @@ int le2d_batch_commit(le2d_batch *b) {
   if (rc) return rc;
   // default shape until autotuned, or the cached winner for such a batch
   le2d::Shape s = B.default_shape();
+  const std::vector<le2d::GridSize> sizes = B.sizes();
   {
+    // a block height counts only for a batch that runs in blocks of it
     std::lock_guard<std::mutex> lk(le2d::g_tune_mu);
-    auto it = le2d::g_tune.find({B.elem, (int)B.inst.size(), B.total_nodes() >> 20});
-    if (it != le2d::g_tune.end()) s = it->second;
+    auto it = le2d::g_tune.find(B.tune_key());
+    if (it != le2d::g_tune.end() &&
+        (!it->second.rows ||
+         le2d::batch_block_rows_at(B.elem, sizes.data(), sizes.size(), it->second.rows)))
+      s = it->second;
   }
   rc = B.build_tiles(s);
   if (rc) return rc;
@@ -529,7 +542,8 @@ int le2d_batch_time(le2d_batch *b, int steps, int plain, double *ms) {
 
 // Times every candidate shape and keeps the fastest (per step): the
 // single-step forms at every window width and segment height, and the
-// two-step form at every segment height, and the default if that is in blocks.  Stepping the batch is part of tuning: the instances advance
+// two-step form at every segment height, and the default shape, whose height the
+// model chooses.  Stepping the batch is part of tuning: the instances advance
 // by an even number of steps per candidate, so callers tune before loading their
 // initial state or account for it.
 int le2d_batch_autotune(le2d_batch *b, int trials, int *best_fb, int *best_seg, double *best_ms) {
@@ -538,7 +552,7 @@ int le2d_batch_autotune(le2d_batch *b, int trials, int *best_fb, int *best_seg, 
   const int fbs[3] = {64, 128, 256};
   const int segs[4] = {16, 32, 64, 128};
   std::vector<le2d::Shape> cand;
-  if (B.shape.rows) cand.push_back(B.shape);
+  cand.push_back(B.default_shape());
   for (int form : {le2d::FORM_TILES, le2d::FORM_PERSISTENT})
     for (int fb : fbs)
       for (int seg : segs) cand.push_back({fb, seg, form});
@@ -565,7 +579,7 @@ int le2d_batch_autotune(le2d_batch *b, int trials, int *best_fb, int *best_seg, 
   if (rc) return rc;
   {
     std::lock_guard<std::mutex> lk(le2d::g_tune_mu);
-    le2d::g_tune[{B.elem, (int)B.inst.size(), B.total_nodes() >> 20}] = best;
+    le2d::g_tune[B.tune_key()] = B.shape;
   }
   if (best_fb) *best_fb = best.fb;
   if (best_seg) *best_seg = best.seg;

@@ -109,3 +109,21 @@ def test_batch_shape(dtype, rows, sizes):
         assert b.get_shape() == shape and b.get_blocks() == rows
         b.set_shape(shape[0], shape[1])
         assert b.get_shape() == shape and b.get_blocks() == rows
+
+
+@pytest.mark.parametrize("dtype", [F8, F4])
+def test_tuned_blocks_stay_with_such_batches(dtype):
+    """Three small grids tuned to blocks leave the default of three larger
+    ones of the same count alone, with a total in the same class too."""
+    small, large = [(200, 170), (113, 121), (57, 9)], [(500, 500), (500, 490), (490, 500)]
+    thin = [(3, 5000), (3, 5000), (3, 5900)]  # as many nodes, three times the blocks
+    want = []
+    for sizes in (large, thin):
+        with _batch(dtype, sizes) as b:
+            want.append((b.get_shape(), b.get_blocks()))
+    with _batch(dtype, small) as b:
+        b.autotune(1)
+        assert b.get_blocks() > 0
+    for sizes, shape in zip((large, thin), want):
+        with _batch(dtype, sizes) as b:
+            assert (b.get_shape(), b.get_blocks()) == shape
