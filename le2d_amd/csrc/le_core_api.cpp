@@ -811,29 +811,33 @@ int le2d_set_material_plane(le_task *task, int count, const double *c1_c2_rho,
   TaskState *s = find(task);
   int rc = ensure_device(task, s);
   if (rc) return rc;
-  if (!s->pairs_fixed) {
-    // With a plane the default two-step window is 64 columns below 2^26 nodes:
-    // wider ones put more nodes into tiles that hold an interface than they save in
-    // halo columns (4100 x 3000 FP64 402 us a pass against 425 at 128, FP32
-    // 147 against 168 at 256).
-    const le2d::GridSize g{s->g.nx, s->g.ny};
-    if (count > 0) {
-      const int only = (long)g.nx * g.ny < (1L << 26) ? 64 : 0;
-      const int cap = only || sizeof(real) == 4 ? 64 : 192;
-      const le2d::PairShape p = le2d::pick_pair_shape((int)sizeof(real), &g, 1, only, cap);
-      le2d::set_pair_shape(&s->g, p.window, p.seg);
-    } else {
-      const le2d::Tiles d = le2d::default_tiles((int)sizeof(real), g.nx, g.ny);
-      le2d::set_pair_shape(&s->g, d.pair_block, d.pair_seg);
-    }
-  }
   if (count == 0) {
     le2d::mat_release(&s->mat);
     s->mat.active = false;
-    return LE2D_OK;
-  }
-  return le2d::mat_set(&s->g, &s->mat, count, c1_c2_rho, ids, (double)task->dt,
+  } else {
+    rc = le2d::mat_set(&s->g, &s->mat, count, c1_c2_rho, ids, (double)task->dt,
                        (double)task->h.x, (double)task->h.y);
+    if (rc) return rc;
+  }
+  if (s->pairs_fixed) return LE2D_OK;
+  const le2d::GridSize g{s->g.nx, s->g.ny};
+  if (count > 0) {
+    // With a plane the default two-step window is 64 columns below 2^26 nodes, in
+    // segments of at most 64 rows: tall or wide tiles put more nodes into those
+    // that hold an interface.  Us a pass, two layers and an inclusion, in this shape
+    // and in the one that the tuner finds without a plane, which a task that was
+    // tuned before keeps: FP64 2050 x 1500 93 and 93, 3000 x 2000 183 and 188,
+    // 6000 x 4000 632 and 615; FP32 2050 x 1500 43.3 and 43.6, 3000 x 2000 68 and 69,
+    // 6000 x 4000 289 and 258.
+    const int only = (long)g.nx * g.ny < (1L << 26) ? 64 : 0;
+    const int cap = only || sizeof(real) == 4 ? 64 : 192;
+    const le2d::PairShape p = le2d::pick_pair_shape((int)sizeof(real), &g, 1, only, cap);
+    le2d::set_pair_shape(&s->g, p.window, p.seg);
+  } else {
+    const le2d::Tiles d = le2d::default_tiles((int)sizeof(real), g.nx, g.ny);
+    le2d::set_pair_shape(&s->g, d.pair_block, d.pair_seg);
+  }
+  return LE2D_OK;
 }
 
 int le2d_energy(le_task *task, double *e) {

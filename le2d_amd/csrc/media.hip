@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "pair_dev.h"
@@ -392,21 +393,28 @@ int mat_set(DevGrid *g, MatPlane *m, int count, const double *c1c2rho, const uns
   if (ids)
     for (long k = 0; k < n; ++k)
       if (ids[k] >= count) return set_error(ERR_ARG, "materials: id %d >= count %d", ids[k], count);
+  // built aside, so that a refused plane leaves the one in force as it is
+  MatPlane next;
+  next.count = count;
+  next.c1c2rho.assign(c1c2rho, c1c2rho + 3 * count);
+  next.ids.assign(n, 0);
+  if (ids) next.ids.assign(ids, ids + n);
+  next.idp = (g->nx + 255) / 256 * 256;
+  int rc = dev_alloc((void **)&next.d_ids, (size_t)next.idp * g->ny, "materials: id plane");
+  if (!rc)
+    rc = mcheck(hipMemcpy2D(next.d_ids, next.idp, next.ids.data(), g->nx, g->nx, g->ny,
+                            hipMemcpyHostToDevice),
+                "materials: ids");
+  if (!rc)
+    rc = g->elem == 8 ? upload_coefs<double>(&next, dt, hx, hy)
+                      : upload_coefs<float>(&next, dt, hx, hy);
+  if (rc) {
+    mat_release(&next);
+    return rc;
+  }
+  next.active = true;
   mat_release(m);
-  m->count = count;
-  m->c1c2rho.assign(c1c2rho, c1c2rho + 3 * count);
-  m->ids.assign(n, 0);
-  if (ids) m->ids.assign(ids, ids + n);
-  m->idp = (g->nx + 255) / 256 * 256;
-  int rc = dev_alloc((void **)&m->d_ids, (size_t)m->idp * g->ny, "materials: id plane");
-  if (rc) return rc;
-  rc = mcheck(hipMemcpy2D(m->d_ids, m->idp, m->ids.data(), g->nx, g->nx, g->ny,
-                              hipMemcpyHostToDevice),
-                  "materials: ids");
-  if (rc) return rc;
-  rc = g->elem == 8 ? upload_coefs<double>(m, dt, hx, hy) : upload_coefs<float>(m, dt, hx, hy);
-  if (rc) return rc;
-  m->active = true;
+  *m = std::move(next);
   return OK;
 }
 
