@@ -28,11 +28,11 @@
 #include <cstdio>
 #include <cstring>
 #include <deque>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -164,7 +164,7 @@ class HostStage {
     if (e == hipSuccess && bytes > 2 * kGrain) {
       try {
         for (auto &h : helper) h = std::thread(move);
-      } catch (const std::system_error &) {  // fewer helpers
+      } catch (const std::exception &) {  // no thread or no memory for one: fewer helpers
       }
     }
     for (size_t p = 0, off = 0; off < sent && e == hipSuccess; ++p) {
