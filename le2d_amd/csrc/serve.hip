@@ -188,6 +188,24 @@ class HostStage {
   hipEvent_t ev_[kPieces] = {};
 };
 
+// Makes `device` the calling thread's current one for a scope.
+class DeviceScope {
+ public:
+  explicit DeviceScope(int device) {
+    if (hipGetDevice(&before_) != hipSuccess) before_ = device;
+    if (before_ != device) (void)hipSetDevice(device);
+    device_ = device;
+  }
+  ~DeviceScope() {
+    if (before_ != device_) (void)hipSetDevice(before_);
+  }
+  DeviceScope(const DeviceScope &) = delete;
+  DeviceScope &operator=(const DeviceScope &) = delete;
+
+ private:
+  int before_ = 0, device_ = 0;
+};
+
 // States in order: a request is finished from DONE on.  RELEASING: a
 // result download holds the request (a second le2d_server_result or a
 // cancel finds it busy).  CANCELLED: removed before or while it ran, or its
@@ -212,6 +230,7 @@ struct Server {
   size_t budget;
   int max_live;
   int plain;
+  int device = 0;  // of the arena, the streams and the stages: the creating thread's
   int max_chunk = 16;
   // queue limit (0: none; submit returns -LE2D_ERR_BUSY at the limit), the
   // queued requests admission looks at, and how often one that does not
@@ -536,7 +555,7 @@ struct Server {
   }
 
   void run() {
-    if (hipSetDevice(0) != hipSuccess) {
+    if (hipSetDevice(device) != hipSuccess) {
       fail("server: device");
       return;
     }
@@ -667,6 +686,7 @@ le2d_server *le2d_server_create(size_t hbm_budget, int max_live, int plain) {
     return nullptr;
   }
   Server *s = new Server(hbm_budget, plain ? 1 : max_live, plain);
+  (void)hipGetDevice(&s->device);
   if (le2d::dev_alloc((void **)&s->arena_dev, hbm_budget, "server: arena")) {
     delete s;
     return nullptr;
@@ -816,6 +836,7 @@ int le2d_server_result(le2d_server *h, long long id, void *aos) {
   g.buf[0] = s->buf(r, 0);
   g.buf[1] = s->buf(r, 1);
   g.cur = r.cur;
+  const le2d::DeviceScope scope(s->device);  // a stage outlives this call
   int rc = le2d::OK;
   hipStream_t st;
   if (auto stage = s->take_stage()) {

@@ -1,5 +1,7 @@
 """Host side of the serving loop's results, run against a HIP runtime in host
-memory (fake_hip.cpp): a thread that cannot be started costs speed only."""
+memory (fake_hip.cpp): a thread that cannot be started costs speed only, and the
+library's streams and events stay on the server's device whatever device a
+caller has current."""
 import os
 import shutil
 import subprocess
@@ -59,3 +61,37 @@ with le2d_amd.Server(1 << 28, 4) as s:
 print("done")
 """ % k)
 
+
+def test_callers_with_another_device(fake):
+    _run(fake, """
+with le2d_amd.Server(1 << 28, 4) as s:
+    ids = requests(s, 3)
+
+    def caller():
+        fake.hipSetDevice(1)
+        result(s, ids[0])
+        d = ctypes.c_int()
+        fake.hipGetDevice(ctypes.byref(d))
+        assert d.value == 1
+        left.append(True)
+
+    left = []
+    t = threading.Thread(target=caller)
+    t.start()
+    t.join()
+    assert left
+    result(s, ids[1])
+    assert fake.fake_foreign() == 0 and fake.fake_cross() == 0, (fake.fake_foreign(), fake.fake_cross())
+print("done")
+""")
+
+
+def test_server_on_the_creating_thread_s_device(fake):
+    _run(fake, """
+fake.hipSetDevice(1)
+with le2d_amd.Server(1 << 28, 4) as s:
+    for i in requests(s, 2):
+        result(s, i)
+assert fake.fake_cross() == 0, fake.fake_cross()
+print("done")
+""")
