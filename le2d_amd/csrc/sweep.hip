@@ -288,6 +288,14 @@ int device_cus() {
   return cus;
 }
 
+// Rows per segment for a launch of `lanes` lanes per segment and strip: `seg`, or
+// the lowest height above it at which the launch stays under 2^32 work-items,
+// the runtime's limit (one row each on 2^32 nodes of 40 bytes is past it).
+static int launch_rows(int seg, int ny, int nstrips, int lanes) {
+  while ((long)nstrips * (((long)ny + seg - 1) / seg) * lanes > 0xffffffffL) ++seg;
+  return seg;
+}
+
 // Launches the kernel of `kinds` that writes `rows` rows (the first if none does)
 // on the blocks of `width` columns that cover the grid.
 template <typename T>
@@ -341,13 +349,11 @@ int step2_xy(DevGrid *g, const SweepCoef<T> &cx, const SweepCoef<T> &cy) {
   if (g->tiles.block_rows)
     return launch_blocks<T>(g, cx, cy, block_kernels<T>(), kBlockKinds, g->tiles.block_rows, 56,
                             "step2_xy");
-  const int seg = g->tiles.pair_seg;
-  if (seg < 1) return set_error(ERR_ARG, "step2_xy: no pair segment height");
+  if (g->tiles.pair_seg < 1) return set_error(ERR_ARG, "step2_xy: no pair segment height");
   const int cols = pair_cols(g->elem, g->tiles.pair_block);
   const int nstrips = (g->nx + cols - 9) / (cols - 8);
-  const long nsegs = (g->ny + seg - 1) / seg;
-  const long nblocks = nsegs * nstrips;
-  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "step2_xy: grid too large");
+  const int seg = launch_rows(g->tiles.pair_seg, g->ny, nstrips, 128);
+  const long nblocks = ((long)g->ny + seg - 1) / seg * nstrips;
   hipLaunchKernelGGL(pair_kernel<T>(cols), dim3((unsigned)nblocks), dim3(128), 0, g->stream,
                      static_cast<const T *>(g->buf[g->cur]), static_cast<T *>(g->buf[g->cur ^ 1]),
                      g->nx, g->ny, g->pitch, g->plane, seg, nstrips, cx, cy);
@@ -427,9 +433,9 @@ template <typename T>
 int sweep_y(DevGrid *g, const SweepCoef<T> &c, int edge) {
   if (g->elem != (int)sizeof(T)) return set_error(ERR_ARG, "sweep_y: element size mismatch");
   const int bx = g->tiles.y_block == 64 || g->tiles.y_block == 128 ? g->tiles.y_block : 256;
-  const int seg = max(1, g->tiles.y_seg), nstrips = (g->nx + bx - 1) / bx;
-  const long nblocks = (long)nstrips * ((g->ny + seg - 1) / seg);
-  if (nblocks > 0x7fffffffL) return set_error(ERR_ARG, "sweep_y: grid too large");
+  const int nstrips = (g->nx + bx - 1) / bx;
+  const int seg = launch_rows(max(1, g->tiles.y_seg), g->ny, nstrips, bx);
+  const long nblocks = ((long)g->ny + seg - 1) / seg * nstrips;
   const T *src = static_cast<const T *>(g->buf[g->cur]);
   T *dst = static_cast<T *>(g->buf[g->cur ^ 1]);
   const bool by_xcd = stays_cached(g);

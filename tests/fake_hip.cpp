@@ -1,7 +1,11 @@
 // A HIP runtime of two devices in host memory, preloaded to run the library's
 // host code where no GPU is: copies are done at once, launches do nothing.  It
 // counts uses of a stream or event by a thread whose current device is another,
-// and fails operator new on request.
+// and fails operator new on request.  Memory is taken only where it is touched,
+// copies of 1 GB and more are left out, and launches of 2^32 work-items and more in
+// a dimension are refused, as the real runtime does.
+#include <sys/mman.h>
+
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -15,7 +19,7 @@ struct Handle {
 struct Dim {
   uint32_t x, y, z;
 };
-thread_local int g_device = 0, g_fail_new = 0;
+thread_local int g_device = 0, g_fail_new = 0, g_error = 0;
 thread_local Dim g_grid, g_block;
 thread_local size_t g_shared;
 thread_local void *g_stream;
@@ -36,8 +40,20 @@ int drop(void *h) {
   return 0;
 }
 int get(void **p, size_t n) {
-  *p = calloc(1, n);
-  return *p ? 0 : 2;
+  *p = mmap(nullptr, n + 4096, PROT_READ | PROT_WRITE,
+            MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  if (*p == MAP_FAILED) return 2;
+  *static_cast<size_t *>(*p) = n + 4096;  // the mapping's length, a page below
+  *p = static_cast<char *>(*p) + 4096;
+  return 0;
+}
+int put(void *p) {
+  if (!p) return 0;
+  void *base = static_cast<char *>(p) - 4096;
+  return munmap(base, *static_cast<size_t *>(base));
+}
+void copy(void *d, const void *s, size_t n) {
+  if (n < size_t(1) << 30) memcpy(d, s, n);
 }
 }  // namespace
 
@@ -62,12 +78,16 @@ int hipDeviceSynchronize() { return 0; }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) {
   return *n = 4, 0;
 }
-int hipGetLastError() { return 0; }
+int hipGetLastError() {
+  const int e = g_error;
+  g_error = 0;
+  return e;
+}
 const char *hipGetErrorString(int) { return "fake"; }
 int hipMalloc(void **p, size_t n) { return get(p, n); }
-int hipFree(void *p) { return free(p), 0; }
+int hipFree(void *p) { return put(p); }
 int hipHostMalloc(void **p, size_t n, unsigned) { return get(p, n); }
-int hipHostFree(void *p) { return free(p), 0; }
+int hipHostFree(void *p) { return put(p); }
 int hipStreamCreateWithFlags(void **s, unsigned) { return make(s); }
 int hipStreamDestroy(void *s) { return drop(s); }
 int hipStreamSynchronize(void *) { return 0; }
@@ -78,9 +98,9 @@ int hipEventDestroy(void *e) { return drop(e); }
 int hipEventRecord(void *e, void *s) { return use(e), use(s); }
 int hipEventSynchronize(void *) { return 0; }
 int hipEventElapsedTime(float *ms, void *, void *) { return *ms = 1.0f, 0; }
-int hipMemcpy(void *d, const void *s, size_t n, int) { return memcpy(d, s, n), 0; }
+int hipMemcpy(void *d, const void *s, size_t n, int) { return copy(d, s, n), 0; }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int, void *stream) {
-  memcpy(d, s, n);
+  copy(d, s, n);
   return use(stream);
 }
 int hipMemset(void *d, int v, size_t n) { return memset(d, v, n), 0; }
@@ -88,7 +108,14 @@ int hipMemsetAsync(void *d, int v, size_t n, void *stream) {
   memset(d, v, n);
   return use(stream);
 }
-int hipLaunchKernel(const void *, Dim, Dim, void **, size_t, void *stream) { return use(stream); }
+int hipLaunchKernel(const void *, Dim grid, Dim block, void **, size_t, void *stream) {
+  g_error = 0;
+  const uint64_t limit = uint64_t(1) << 32;
+  if (uint64_t(grid.x) * block.x >= limit || uint64_t(grid.y) * block.y >= limit ||
+      uint64_t(grid.z) * block.z >= limit)
+    return g_error = 9;  // hipErrorInvalidConfiguration
+  return use(stream);
+}
 int __hipPushCallConfiguration(Dim grid, Dim block, size_t shared, void *stream) {
   g_grid = grid;
   g_block = block;
