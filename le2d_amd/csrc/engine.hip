@@ -288,11 +288,7 @@ Tiles default_tiles(int elem, int nx, int ny) {
   t.x_rows = 1;
   t.pair_split = 0;
   t.step_rows = step_blocks(elem, nx, ny);
-  // FP64 grids of 2^26 nodes and more march 256-lane windows (8192^2 disk 1.06 ms
-  // against 1.08 in blocks)
-  const bool vast = elem == 8 && (long)nx * ny >= 1l << 26 && nx >= 4096;
-  if (vast) t.step_rows = 0;
-  if (t.step_rows == 0 && !vast) {
+  if (t.step_rows == 0) {
     t.xy_block = 64;
     t.xy_seg = step_segment(nx, ny);
   } else {
@@ -369,7 +365,9 @@ void set_pair_shape(DevGrid *g, int window, int seg) {
 // blocks hold the registers of two wavefronts per SIMD and last long, so the march
 // comes first (900^2 18.4 against 20.4, 1500 x 1001 26.0 against 30.9) until blocks of 24
 // rows make several rounds (2048^2 77 both, 3000^2 170 against 153, 8192 x 4096
-// 577 against 565).
+// 577 against 565; from 2^26 nodes on, against 256-lane windows, the fastest march
+// there: 4096 x 17000 1057 against 988, 10000^2 1617 against 1559, 14000^2 3206
+// against 3114, but 8192^2 1061 to 1081 against 1080).
 static int step_blocks(int elem, int nx, int ny) {
   const long strips = (nx + 59) / 60, cus = device_cus();
   auto blocks = [&](int kind) {
