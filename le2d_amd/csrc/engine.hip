@@ -465,8 +465,10 @@ PairShape pick_pair_shape(int elem, const GridSize *g, size_t n, int only, int c
   }
   // Several FP32 grids that this puts into one round of 64-column workgroups: with
   // 75 registers three rounds are resident at once, and r of them last (1 + r) / 2 of
-  // one (25 instances of 128 to 384, 37 steps: 517 us at 32 rows, one round, 455 at
-  // 14, two; 16 of 96 to 500, 36 steps: 400 at 20, one, 370 at 10, two).
+  // one (us a step at the rows of one round and at the rows taken here: 12 instances of
+  // 300 to 600 17.8 at 48, 16.0 at 24; 16 of 96 to 500 10.4 at 20, 10.3 at 10; 25 of 128 to
+  // 384 12.5 at 28, 12.0 at 14; 40 of 128 to 384 19.6 at 56, 16.0 at 24; 100 of 64 to
+  // 200 14.9 at 37, about 13.4 at 16).
   if (n > 1 && elem == 4 && best.window == 64) {
     const long slots = pair_slots(elem, 64);
     double cost = 0;

@@ -127,3 +127,28 @@ def test_tuned_blocks_stay_with_such_batches(dtype):
     for sizes, shape in zip((large, thin), want):
         with _batch(dtype, sizes) as b:
             assert (b.get_shape(), b.get_blocks()) == shape
+
+
+def test_short_segments_of_fp32_sets():
+    """FP32 sets that one round of 64-column workgroups would hold take two or three
+    of shorter segments, with the results of another shape."""
+    rng = np.random.default_rng(16)
+    sizes = [tuple(int(v) for v in np.exp(rng.uniform(np.log(96), np.log(500), 2)))
+             for _ in range(16)]
+    states = [np.random.default_rng(k).standard_normal((ny, nx, 5)).astype(F4)
+              for k, (nx, ny) in enumerate(sizes)]
+    out = []
+    for march in (False, True):
+        with _batch(F4, sizes) as b:
+            if march:
+                b.set_shape(128, 37)
+            else:
+                width, seg = b.get_shape()[:2]
+                strips = sum(-(-nx // 56) * -(-ny // seg) for nx, ny in sizes)
+                assert width == 64 and b.get_blocks() == 0 and 1024 < strips <= 3 * 1024
+            for k, g in enumerate(states):
+                b.load(k, g)
+            b.step(9)
+            b.wait()
+            out.append([b.read(k) for k in range(len(sizes))])
+    assert all(gd.same_bits(x, y) for x, y in zip(*out))
