@@ -202,14 +202,20 @@ def measured_counters(n, dtype, kernel):
     return json.load(open(p))
 
 
-def roofline(n, es, ms_pair, ms_step, ms_x, ms_y, dtype_name, split=0):
+def step_kernels(t):
+    """The kernels of the task's two-step pass and single step, as it is set."""
+    step_rows, pair_rows = t.get_step_blocks()
+    pair = ("k_step2_block" if pair_rows else
+            "k_step2_split" if t.get_step_pair_window() == 64 else "k_step2_xy")
+    return pair, "k_step_block" if step_rows else "k_step_xy"
+
+
+def roofline(n, es, ms_pair, ms_step, ms_x, ms_y, dtype_name, kernels):
     """Roofline of the launch that carries le_step_n: the two-step kernel
-    (two node-updates per node per launch; k_step2_split when the tuner
-    chose 64-column windows) when it is on, else the
-    single-step kernel."""
+    (two node-updates per node per launch) when it is on, else the
+    single-step kernel (kernels: step_kernels)."""
     nodes = n * n
-    pair_kernel = "k_step2_split" if split else "k_step2_xy"
-    kernel, ms, steps = (pair_kernel, ms_pair, 2) if ms_pair else ("k_step_xy", ms_step, 1)
+    kernel, ms, steps = (kernels[0], ms_pair, 2) if ms_pair else (kernels[1], ms_step, 1)
     # Algorithmic bytes per node-update: 2 sweeps x (5 reads + 5 writes) x
     # sizeof(real), times the node-updates per node one launch performs.
     alg = nodes * 20 * es * steps
@@ -238,8 +244,8 @@ def roofline(n, es, ms_pair, ms_step, ms_x, ms_y, dtype_name, split=0):
                           "valu_issue_frac are at most 1",
             "compulsory_bytes_per_launch": compulsory,
             "algorithmic_bytes_per_launch": alg, "steps_per_launch": steps,
-            "ms_per_launch": {pair_kernel: round(ms_pair, 4) if ms_pair else None,
-                              "k_step_xy": round(ms_step, 4), "k_sweep_x": round(ms_x, 4),
+            "ms_per_launch": {kernels[0]: round(ms_pair, 4) if ms_pair else None,
+                              kernels[1]: round(ms_step, 4), "k_sweep_x": round(ms_x, 4),
                               "k_sweep_y": round(ms_y, 4)},
             "two_kernel_GBps": {"k_sweep_x": round(nodes * 10 * es / ms_x / 1e6, 1),
                                 "k_sweep_y": round(nodes * 10 * es / ms_y / 1e6, 1)}}
@@ -776,8 +782,7 @@ def main():
                                                      args.warmup, args.profile_steps)
     el = els[0]
     value = n * n * args.steps / el / 1e9
-    roof = roofline(n, es, ms_pair, ms_step, ms_x, ms_y, args.dtype,
-                    t.get_step_pair_window() == 64)
+    roof = roofline(n, es, ms_pair, ms_step, ms_x, ms_y, args.dtype, step_kernels(t))
     tiles = t.get_tiles() + (t.get_step_pairs(), t.get_step_pair_window(),
                              t.get_step_pair_split())
     other = None
@@ -793,7 +798,7 @@ def main():
         other = {"dtype": o_name, "value": round(n * n * args.steps / el2 / 1e9, 3),
                  "ms_per_step": round(el2 / args.steps * 1e3, 4),
                  "roofline": roofline(n, np.dtype(o_dt).itemsize, mp2, ms2, mx2, my2, o_name,
-                                      t2.get_step_pair_window() == 64),
+                                      step_kernels(t2)),
                  "tiles": {"pair_seg": t2.get_step_pairs(),
                            "pair_lanes": t2.get_step_pair_window(),
                            "pair_split": t2.get_step_pair_split()},

@@ -152,3 +152,12 @@ def test_short_segments_of_fp32_sets():
             b.wait()
             out.append([b.read(k) for k in range(len(sizes))])
     assert all(gd.same_bits(x, y) for x, y in zip(*out))
+
+
+@pytest.mark.parametrize("dtype,nx,ny,kernels", [
+    (F8, 96, 80, ("k_step2_block", "k_step_block")), (F8, 900, 900, ("k_step2_split", "k_step_xy")),
+    (F8, 2048, 2048, ("k_step2_xy", "k_step_xy")), (F4, 1500, 1001, ("k_step2_block", "k_step_block"))])
+def test_bench_names_the_kernels_that_run(dtype, nx, ny, kernels):
+    import bench
+    with _task(dtype, nx, ny) as t:
+        assert bench.step_kernels(t) == kernels
