@@ -145,7 +145,8 @@ struct DivIeee {
 // compiled.  Checked on the GPU where rounding is closest, on every quotient
 // within 5 units of the product's last place of a rounding boundary for the
 // 2^39 divisors below a power of two (1.4e12 quotients), and on 2e10 random
-// ones: all equal to n / d.
+// ones: all equal to n / d; the test of the quotients repeats that for 2^30 divisors
+// of each kind.
 struct DivBounded {
   static constexpr bool kSees = true;
   float big = 0.0f, small = 1.0f;
