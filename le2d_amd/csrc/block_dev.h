@@ -10,15 +10,16 @@
 // rows independent of each other, and two exchanges of boundary rows between
 // neighbouring wavefronts per y-sweep.  It writes the 56 columns and R*WV-8
 // rows between the halos (one step: 60 and R*WV-4).  One block's loads do not
-// overlap its own arithmetic, so FP64, whose registers allow one block a
-// compute unit, takes it where every block has a unit to itself, FP32 up to a
-// few more.
+// overlap its own arithmetic, so FP64, whose registers allow one block a compute
+// unit (two of the lowest), takes it where every block has a unit to itself, FP32
+// up to sixteen for each.
 //
 // us a pass, block against march: FP64 96 x 80 7.6 against 9.1, 250 x 300 8.5 against
-// 12.4, 512^2 14.6 against 19.1, 724^2 23.0 against 25.3, but 900^2 (two rounds
+// 12.4, 512^2 14.6 against 19.1, 724^2 21.4 against 25.3, but 900^2 (two rounds
 // of blocks) 37 against 34; FP32 250 x 300 4.5 against 6.5, 512^2 7.1 against 9.3, 1031
 // x 517 9.5 against 12.1, 900^2 13.4 against 16.1, and past one block a unit 1500 x
-// 1001 21.4 against 23.3, but 3000^2 95 against 94.
+// 1001 21.4 against 23.3, 3000^2 95 against 94 to 100 (the march at its default and
+// near heights is slower, at the tuner's best the same).
 //
 // One step.  With half the halo the blocks pay on larger grids too: in FP32,
 // where two or more of them share a compute unit and one loads while another computes,
@@ -76,15 +77,20 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
     u[r] = load_nodes<T, 1>(src + (long)min(ypos<EDGE>(jw + r, ny), ny - 1) * pitch, plane, boff);
 #pragma unroll
   for (int r = 0; r < R; ++r) see_row(u[r], ed, t, dv);
-  // A wavefront whose rows are out of the divisions' range only passes the barriers
-  // from here on, as block_tile takes the block again (FP64 512^2 with NaN everywhere 20.9
-  // us a pass, 27.9 with both marches in full; finite 16.7 either way).  It is asked
-  // behind x-sweeps, which need not wait for every row's load then (asked before
-  // them 512^2 is 17.2); the tall block, short of registers, before its last ones.
-  auto stand_by = [&] {
+  // A wavefront whose rows are out of the divisions' range only passes the remaining
+  // barriers, as block_tile takes the block again.  Where it is asked costs finite
+  // fields the least: tall blocks before the first barrier (before the x-sweeps it would
+  // wait for every row's load), or before the last x-sweeps where registers are short,
+  // low ones between the two steps, the lowest not at all in one step.  FP64 us a pass
+  // with NaN everywhere, finite in brackets: 96 x 80 13.7 (10.5), 512^2 23.1 (16.8); with both
+  // marches in full 15.8 and 27.9.
+  enum { NEVER, IN_X, BEFORE_Y, BETWEEN };
+  constexpr int ask = STEPS > 1 ? (R > 4 ? BEFORE_Y : BETWEEN)
+                                : (R > 6 ? IN_X : R > 2 ? BEFORE_Y : NEVER);
+  auto stand_by = [&](int passed) {
     if (!Div::kSees || __all(dv.in_range())) return false;
 #pragma unroll 1
-    for (int k = 0; k < 4 * STEPS - 1; ++k) __syncthreads();
+    for (int k = passed; k < 4 * STEPS - 1; ++k) __syncthreads();
     return true;
   };
 #pragma unroll 1
@@ -93,7 +99,7 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
     for (int r = 0; r < R; ++r) {
       x_sweep(u[r], lds[v].x, t, ed, cx, dv);
       pin(u[r].n[0]);
-      if (R > 6 && r == R - 3 && stand_by()) return;
+      if (ask == IN_X && r == R - 3 && stand_by(0)) return;
     }
     // after a step rows outside the grid take the edge row's value (one step's are
     // loaded so)
@@ -110,7 +116,7 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
     lds[v].y.first[t] = w.w[0];
     lds[v].y.second[t] = {w.w[1].b, w.w[1].d};
     lds[v].y.last[t] = {w.w[R - 1].a, w.w[R - 1].c};
-    if (R <= 6 && s == 0 && stand_by()) return;
+    if (ask == BEFORE_Y && s == 0 && stand_by(0)) return;
     __syncthreads();
     // the row above (a and c) and two rows below; rows past the block's own
     // edge stand for nothing that an output reads, rows past the grid's take its
@@ -144,6 +150,7 @@ __device__ __forceinline__ void block_march(const T *__restrict__ src, T *__rest
       fi = fo;
     }
     if (s + 1 >= STEPS) break;
+    if (ask == BETWEEN && stand_by(4)) return;
   }
   const unsigned woff = (unsigned)max(x, 0) * (unsigned)sizeof(T);
   const bool writer = t >= H && t < 64 - H && x < nx;
