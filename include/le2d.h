@@ -119,8 +119,9 @@ int le2d_get_step_pair_split(le_task *task, int *on);
  * buffer.  le_step_n does this once per
  * grid shape and process on its first call of 8 or more steps, unless the
  * caller has set a height (le2d_set_step_pairs), a material plane is set or
- * the environment has LE2D_TUNE=0.  A task with a material plane keeps the
- * default window and height. */
+ * the environment has LE2D_TUNE=0.  A task with a material plane is not tuned: it
+ * has the default shape of grids with a plane, or keeps the one that it was
+ * tuned to or given before the plane was set. */
 int le2d_tune_step_pairs(le_task *task, int *seg);
 /* Rows that a register block writes in single steps and in two-step passes as
  * the task is set now; 0: a march. */
@@ -328,7 +329,15 @@ int le2d_server_wait(le2d_server *srv, long long id, double timeout_s);
 int le2d_server_drain(le2d_server *srv, double timeout_s);
 /* Copy a kept result into an AOS host array (nx*ny nodes of five reals of
  * the request's type) and release its device memory.  Only one call per
- * result succeeds; a concurrent second call returns LE2D_ERR_STATE. */
+ * result succeeds; a concurrent second call returns LE2D_ERR_STATE.
+ * Host resources: the result passes through pinned host memory, up to four
+ * stages of 8 MB for each server, made by the first calls that need them (as many
+ * as run at once) and kept until the server is destroyed; further concurrent
+ * calls, and those that cannot have a stage, copy without one.  A call on more than
+ * 512 KB runs up to three threads of its own until it returns.  Pinned memory is not
+ * device memory and does not come from le2d_set_device_allocator's functions.
+ * The server works on the device that was current when it was created, whatever
+ * device the caller has current. */
 int le2d_server_result(le2d_server *srv, long long id, void *aos);
 /* Submission, admission and completion times (seconds, steady clock). */
 int le2d_server_times(le2d_server *srv, long long id, double *t_submit, double *t_admit,

@@ -314,8 +314,9 @@ Tiles default_tiles(int elem, int nx, int ny) {
   // that (block_dev.h has both sides' times); in FP32, where several share one, also
   // blocks of 40 rows on grids of up to 16 for each (us a pass, blocks against the
   // march at its default shape: 2500 x 1500 41.2 and 45.1, 2961 x 2216 64.9 and 70.2,
-  // 3500 x 2500, 15.5 for each, 89.8 and 95.5; against the march's fastest shape 1200^2
-  // 21.0 and 23.2, 2048^2 43.5 and 43.0)
+  // 3500 x 2500, 15.5 for each, 89.8 and 95.5; against the march's fastest shape, which
+  // only the tuner finds, 1200^2 21.0 and 23.2, 2048^2 43.5 and 43.0, 3000^2 and 3500
+  // x 2500 the same or better: the tuner keeps the blocks)
   int rows = 0;
   for (int k = 0; k < kBlockKinds && !rows; ++k)
     if (pair_blocks(nx, ny, block_rows(elem, k)) <= device_cus()) rows = block_rows(elem, k);

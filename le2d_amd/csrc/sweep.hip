@@ -9,9 +9,10 @@
 namespace le2d {
 
 // ---------------------------------------------------------------------------
-// x-sweep of FP32 grids that leave the last-level cache, and of a caller who set
-// the rows of a workgroup.  A workgroup of BX lanes owns BX consecutive nodes of a row and
-// walks `rows` rows.  Per row: coalesced loads of the five planes, invariants
+// x-sweep of grids that leave the last-level cache (FP32; FP64 from 2^24 nodes on, see
+// sweep_x), and of a caller who set the rows of a workgroup to other than the
+// default.  A workgroup of BX lanes owns BX consecutive nodes of a row and walks
+// `rows` rows.  Per row: coalesced loads of the five planes, invariants
 // to LDS (with a 2-node clamped halo each side), one face per lane (lane 0
 // also the segment's left face) to LDS, then the node update and coalesced
 // stores.  LDS is double-buffered by row parity, so a row costs two barriers.
@@ -178,7 +179,9 @@ __global__ __launch_bounds__(128, (pair_waves<T, FB / 64>())) void k_step2_xy(
   pair_tile<T, FB / 64>(src, dst, nx, ny, pitch, plane, strip, j0, j1, cx, cy, lds);
 }
 
-// ... and in windows of 64 columns, one per lane.
+// ... and in windows of 64 columns, one per lane: the same kernel at FB = 64 under the
+// name that profiles and the resource report know.  HOLD is part of that name
+// (the march goes by kHoldInv).
 template <typename T, bool HOLD>
 __global__ __launch_bounds__(128, (pair_waves<T, 1>())) void k_step2_split(
     const T *__restrict__ src, T *__restrict__ dst, int nx, int ny, long pitch, long plane,
