@@ -120,8 +120,8 @@ int le2d_get_step_pair_split(le_task *task, int *on);
  * grid shape and process on its first call of 8 or more steps, unless the
  * caller has set a height (le2d_set_step_pairs), a material plane is set or
  * the environment has LE2D_TUNE=0.  A task with a material plane is not tuned: it
- * has the default shape of grids with a plane, or keeps the one that it was
- * tuned to or given before the plane was set. */
+ * has the default shape of grids with a plane, whatever it ran before, or the one
+ * that the caller gave it. */
 int le2d_tune_step_pairs(le_task *task, int *seg);
 /* Rows that a register block writes in single steps and in two-step passes as
  * the task is set now; 0: a march. */

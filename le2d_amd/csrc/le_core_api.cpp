@@ -42,7 +42,8 @@ struct TaskState {
   bool owned = true;        // mirror allocated by le_init_task
   int mode = LE2D_SYNC_WAIT;
   hipStream_t stream = nullptr;
-  bool pairs_fixed = false;  // segment height set by the caller or tuned
+  bool pairs_fixed = false;  // two-step shape set by the caller or tuned
+  bool pairs_tuned = false;  // ... by the tuner
   // A step accepted by le_step but not yet run, so that it and the next
   // le_step share one two-step pass; run before anything else touches the
   // device state (flush_pending), with the coefficients it was called with.
@@ -154,6 +155,16 @@ SweepCoef<real> coef(const le_task *t, real h) {
 
 enum { DO_X = 1, DO_Y = 2 };
 
+// Takes the shape that the tuner found for this grid earlier in the process.
+bool recall_pairs(TaskState *s) {
+  std::lock_guard<std::mutex> lk(g_pair_mu);
+  auto it = g_pair_seg.find(std::make_tuple((int)sizeof(real), s->g.nx, s->g.ny));
+  if (it == g_pair_seg.end()) return false;
+  le2d::set_pair_shape(&s->g, it->second.window, it->second.seg);
+  s->pairs_fixed = s->pairs_tuned = true;
+  return true;
+}
+
 // Two-step segment height and window width for this grid: each candidate is
 // timed out of place -- the pass reads the current state and writes the idle
 // buffer (scratch between steps), and the buffer swap is undone -- so the
@@ -162,16 +173,8 @@ enum { DO_X = 1, DO_Y = 2 };
 // candidates differ by less than their noise); the fastest is kept, and
 // remembered for the grid shape.
 int tune_pairs(le_task *t, TaskState *s) {
+  if (recall_pairs(s)) return LE2D_OK;
   const auto key = std::make_tuple((int)sizeof(real), s->g.nx, s->g.ny);
-  {
-    std::lock_guard<std::mutex> lk(g_pair_mu);
-    auto it = g_pair_seg.find(key);
-    if (it != g_pair_seg.end()) {
-      le2d::set_pair_shape(&s->g, it->second.window, it->second.seg);
-      s->pairs_fixed = true;
-      return LE2D_OK;
-    }
-  }
   const SweepCoef<real> cx = coef(t, t->h.x), cy = coef(t, t->h.y);
   const int cand[] = {4, 8, 12, 16, 24, 32, 48, 64, 80, 96, 128, 160};
   hipEvent_t ev[2];
@@ -255,7 +258,7 @@ int tune_pairs(le_task *t, TaskState *s) {
   }
   for (auto &e : ev) (void)hipEventDestroy(e);
   le2d::set_pair_shape(&s->g, best.block, best.seg);
-  s->pairs_fixed = true;
+  s->pairs_fixed = s->pairs_tuned = true;
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(g_pair_mu);
   g_pair_seg[key] = {best.block, best.seg};
@@ -706,6 +709,7 @@ int le2d_set_step_pairs(le_task *task, int seg) {
   if (seg < 0) return le2d::set_error(LE2D_ERR_ARG, "step pairs: segment %d", seg);
   le2d::set_pair_shape(&s->g, s->g.tiles.pair_block, seg);
   s->pairs_fixed = true;
+  s->pairs_tuned = false;
   return LE2D_OK;
 }
 
@@ -733,6 +737,7 @@ int le2d_set_step_pair_window(le_task *task, int lanes) {
     return le2d::set_error(LE2D_ERR_ARG, "step pairs: window %d", lanes);
   le2d::set_pair_shape(&s->g, lanes, s->g.tiles.pair_seg);
   s->pairs_fixed = true;
+  s->pairs_tuned = false;
   return LE2D_OK;
 }
 
@@ -743,6 +748,7 @@ int le2d_set_step_pair_split(le_task *task, int on) {
   if (on != 0 && on != 1) return le2d::set_error(LE2D_ERR_ARG, "step pairs: split %d", on);
   s->g.tiles.pair_split = on;
   s->pairs_fixed = true;
+  s->pairs_tuned = false;
   return LE2D_OK;
 }
 
@@ -819,21 +825,21 @@ int le2d_set_material_plane(le_task *task, int count, const double *c1_c2_rho,
                        (double)task->h.x, (double)task->h.y);
     if (rc) return rc;
   }
-  if (s->pairs_fixed) return LE2D_OK;
   const le2d::GridSize g{s->g.nx, s->g.ny};
   if (count > 0) {
+    if (s->pairs_fixed && !s->pairs_tuned) return LE2D_OK;  // a caller's shape stays
     // With a plane the default two-step window is 64 columns below 2^26 nodes, in
     // segments of at most 64 rows: tall or wide tiles put more nodes into those
     // that hold an interface.  Us a pass, two layers and an inclusion, in this shape
-    // and in the one that the tuner finds without a plane, which a task that was
-    // tuned before keeps: FP64 2050 x 1500 93 and 93, 3000 x 2000 183 and 188,
-    // 6000 x 4000 632 and 615; FP32 2050 x 1500 43.3 and 43.6, 3000 x 2000 68 and 69,
-    // 6000 x 4000 289 and 258.
+    // and at 64 rows in the widest window: FP64 3000 x 2000 186 and 194, 4100 x 3000 346
+    // and 386, 8000 x 6000 1186 and 1212; FP32 70 and 142, 150 and 174, 520 and 559, but
+    // 6000 x 4000 295 and, in 128 columns, 277.  What the tuner finds without a plane is
+    // not the plane's: 4100 x 3000 FP64 324 in this shape, 333 to 400 in tuned ones.
     const int only = (long)g.nx * g.ny < (1L << 26) ? 64 : 0;
     const int cap = only || sizeof(real) == 4 ? 64 : 192;
     const le2d::PairShape p = le2d::pick_pair_shape((int)sizeof(real), &g, 1, only, cap);
     le2d::set_pair_shape(&s->g, p.window, p.seg);
-  } else {
+  } else if (!s->pairs_fixed || (s->pairs_tuned && !recall_pairs(s))) {
     const le2d::Tiles d = le2d::default_tiles((int)sizeof(real), g.nx, g.ny);
     le2d::set_pair_shape(&s->g, d.pair_block, d.pair_seg);
   }

@@ -77,17 +77,23 @@ def test_no_memory_for_a_second_plane(granted):
 
 @pytest.mark.parametrize("count", [8, 9])
 def test_plane_set_after_the_tuner_ran_and_taken_away(count):
-    """The tuned shape stays in force with the plane and after it."""
+    """What the tuner found without a plane is not the plane's shape: it has the
+    default of grids with one, and the tuned shape is back when the plane goes."""
     ref = _state()
     o = Oracle(np.float64)
     o.run(ref, *ARGS, count)
     o.run_mat(ref, ARGS[0], ARGS[1], MATS, _ids(60), count)
     o.run(ref, *ARGS, count)
     with le2d_amd.Task(NX, NY, *ARGS) as t:
+        t.set_materials(MATS, _ids(60))
+        default = t.get_step_pairs(), t.get_step_pair_window()
+    with le2d_amd.Task(NX, NY, *ARGS) as t:
         t.load(_state())
         t.step_n(count)
         shape = t.get_step_pairs(), t.get_step_pair_window(), t.get_step_blocks()
+        assert shape[2][1] > 0  # blocks
         t.set_materials(MATS, _ids(60))
+        assert (t.get_step_pairs(), t.get_step_pair_window()) == default
         t.step_n(count)
         t._check(t.lib.le2d_set_material_plane(t.ref, 0, None, None), "remove the plane")
         assert (t.get_step_pairs(), t.get_step_pair_window(), t.get_step_blocks()) == shape
